@@ -16,6 +16,7 @@
 #include "lbm_device.hpp"
 #include "lbm_internal.h"
 #include "lbm_mi355x.h"
+#include "lbm_tile2d.hpp"
 
 using namespace lbm;
 
@@ -84,6 +85,7 @@ struct lbm_handle {
   int bmap8 = 0;        // its length / 8
   int bmap_bs = 0;      // the node block it was built for
   int lds_cu = 0;       // LDS per CU of the device (bytes)
+  int cus = 256;        // compute units of the device
   int *amap = nullptr;  // row-band block map of the adjoint step (kAdjBlock threads)
   size_t st_bytes = 8;
   void *F = nullptr;
@@ -105,6 +107,18 @@ struct lbm_handle {
   int n_lo = 0, n_hi = 0, n_flux = 0;
   int zb_ok = 0;  // the z faces are the compact ranges [0, n_lo) and [nf - n_hi, nf)
   double *ns = nullptr;  // [nf] Walsh partial bounce-back fraction, or null
+  // 2-D runs of several steps per launch (k_tile2d): the plan, its tables and
+  // the population array its launches write (swapped with F after each)
+  struct {
+    int state = 0;  // 0 not planned, 1 ready, -1 not for this lattice
+    TileGeo T{};
+    int steps = 0, shrink = 0, threads = 0;
+    int lds_set = 0;  // kernels whose LDS limit has been raised
+    size_t lds = 0;
+    int *gidx = nullptr, *cnt = nullptr;
+    uint32_t *list = nullptr;
+    void *F2 = nullptr;
+  } tile;
   bool off64 = false;    // 64-bit element offsets at every size (LBM_OFFSET64=1)
   int *plane_lo = nullptr, *plane_hi = nullptr, *tgt_lo = nullptr, *tgt_hi = nullptr;
   void *halo_pos = nullptr, *halo_neg = nullptr;
@@ -341,9 +355,17 @@ void drop_chunks(lbm_handle *h) {
   h->gen++;
 }
 
+void free_tiles(lbm_handle *h) {
+  void *ptrs[] = {h->tile.gidx, h->tile.cnt, h->tile.list, h->tile.F2};
+  for (void *q : ptrs)
+    if (q) (void)hipFree(q);
+  h->tile = {};
+}
+
 void free_lattice(lbm_handle *h) {
   drop_chunks(h);
   free_objective(h);
+  free_tiles(h);
   void *ptrs[] = {h->F, h->rw, h->mv, h->node, h->face_lo, h->face_hi, h->face_flux, h->plane_lo,
                   h->plane_hi, h->tgt_lo, h->tgt_hi, h->halo_pos, h->halo_neg, h->ns, h->bmap, h->amap};
   for (void *q : ptrs)
@@ -785,6 +807,7 @@ extern "C" int lbm_create(const lbm_params *p, lbm_handle **out) {
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) == hipSuccess)
       h->lds_cu = v;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) h->cus = v;
   }
   if (p->c_bot_map && p->dims == 3) {
     size_t E = (size_t)h->E;
@@ -1121,11 +1144,210 @@ hipGraphExec_t chunk_for(lbm_handle *h) {
   return x;
 }
 
+// ---- several 2-D steps per launch -----------------------------------------
+
+// the one flow condition of a 2-D row (0 north, 1 south): its kind (0 none,
+// 1 density, 2 y momentum) and which of the n_in / n_out / s_in / s_out
+// values it takes; false when the row carries more than one
+bool row_condition(const lbm_params &p, int side, int &kind, int &which) {
+  const int pin = side == 0 ? p.pressure_n_in[0] : p.pressure_s_in[0];
+  const int pout = side == 0 ? p.pressure_n_out[0] : p.pressure_s_out[0];
+  const int vin = side == 0 ? p.velocity_n_in : p.velocity_s_in;
+  const int vout = side == 0 ? p.velocity_n_out : p.velocity_s_out;
+  kind = pin || pout ? 1 : (vin || vout ? 2 : 0);
+  which = 2 * side + ((pin || vin) ? 0 : 1);
+  return (pin != 0) + (pout != 0) + (vin != 0) + (vout != 0) <= 1;
+}
+
+template <int NS, bool SOL, bool WALSH>
+int tile_launch(lbm_handle *h, const TileArgs &B) {
+  const dim3 grid(8 * B.T.tiles8);
+  auto go = [&](auto *fn, int nt) -> int {
+    // every handle asks for the same limit, the CU's whole LDS
+    constexpr int bit = 1 << ((NS - 1) * 4 + SOL * 2 + WALSH);
+    if (!(h->tile.lds_set & bit)) {
+      HIP_OK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, h->lds_cu));
+      h->tile.lds_set |= bit;
+    }
+    hipLaunchKernelGGL(fn, grid, dim3(nt), h->tile.lds, h->stream, B);
+    HIP_OK(hipGetLastError());
+    return 0;
+  };
+  if (h->tile.threads == 512) return go(k_tile2d<NS, SOL, WALSH, 512>, 512);
+  return go(k_tile2d<NS, SOL, WALSH, 1024>, 1024);
+}
+
+// Steps per launch, core and threads of k_tile2d for the handle's lattice.
+// A lattice that one tile per CU covers takes the smallest square core that
+// does: its time is launch (2 us) and per-step latency (1 us), so it takes
+// as many steps a launch as the halo's work allows, 8 (two components with
+// cores above 12: 6; cores above 20: 4).  Measured, us per step, flow | flow +
+// solute with row conditions: 128^2 8 x 8 cores 1.54 | 1.94 (4 steps 1.74 |
+// 2.06), 200 x 170 12 x 12 cores 1.64 | 2.07 (4 steps 1.9 | 2.19), 300 x 310
+// 20 x 20 cores 1.97 with 8 steps | 2.71 with 6 (4 steps: 2.3 | 2.86).
+// Larger lattices run several tiles per CU and are bound by the loads of the
+// halo and the FP64 units together: 4 steps, flow in 32 x 16 cores of which a
+// CU holds two (1000^2 10.8, 2100 x 1900 44.9 us; 30 x 30 cores with 8 steps
+// 11.3, 43.7), flow + solute in the largest square core that LDS holds, 25 x
+// 25 (19.7, 85.3 us; 32 x 16 20.4, 91.4; 20 x 20 with 6 steps 22.2, 94.9).
+void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy, int &threads) {
+  const int ns = h->p.nsubs;
+  const double per_cu = (double)h->N / h->cus;
+  int s = 8;
+  while ((double)s * s < per_cu && s < 64) s++;
+  steps = s <= 12 ? 8 : (s <= 20 ? (ns == 1 ? 8 : 6) : 4);
+  auto most = [&](int k) {  // largest square core of k steps
+    int c = 0;
+    const int halo = shrink * k / 2;
+    while (c + 1 + 2 * halo <= 64 && (size_t)(c + 1 + 2 * halo) * (c + 1 + 2 * halo) * (72 * ns + 4) <= (size_t)h->lds_cu)
+      c++;
+    return c;
+  };
+  if (most(steps) < s) steps = 4;
+  cx = cy = std::min(s, most(steps));
+  if (s > 20 && ns == 1) {
+    cx = 32;
+    cy = 16;
+  }
+  const int halo = shrink * steps / 2;
+  threads = (cx + 2 * halo) * (cy + 2 * halo) > 800 && !(s > 20 && ns == 1) ? 1024 : 512;
+}
+
+// Plans the tiles of the handle's lattice on first use; h->tile.state tells
+// whether lbm_run may use them.
+int plan_tiles(lbm_handle *h) {
+  auto &t = h->tile;
+  if (t.state) return 0;
+  t.state = -1;
+  const lbm_params &p = h->p;
+  if (h->D != 2 || p.storage != LBM_STORE_F64 || p.compute != LBM_COMPUTE_F64 || p.halo_mode || h->off64) return 0;
+  int kind[2], which;
+  if (!row_condition(p, 0, kind[0], which) || !row_condition(p, 1, kind[1], which)) return 0;
+  const bool two = p.nsubs == 2;
+  if (two && (p.pressure_n_in[1] || p.pressure_n_out[1] || p.pressure_s_in[1] || p.pressure_s_out[1])) return 0;
+  const int grad[2] = {two && p.zeroconcgrad_n, two && p.zeroconcgrad_s};
+  const bool rows = kind[0] || kind[1] || grad[0] || grad[1];
+  const int ni = p.ni, nj = p.nj;
+  if (rows && nj < 3) return 0;
+  // whether a density or zero-gradient row hands a value to a neighbour: a
+  // row node whose source across the wrapped edge is solid
+  bool handed = false;
+  for (int side = 0; side < 2 && !handed; side++) {
+    if (kind[side] != 1 && !grad[side]) continue;
+    const long row = side == 0 ? nj - 1 : 0, src = side == 0 ? 0 : nj - 1;
+    for (int i = 0; i < ni && !handed; i++) {
+      if (h->fid[row * ni + i] < 0) continue;
+      for (int d = -1; d <= 1; d++) handed |= h->fid[src * ni + (i + d + ni) % ni] < 0;
+    }
+  }
+  t.shrink = handed ? 3 : 2;
+  tile_shape(h, t.shrink, t.steps, t.T.cx, t.T.cy, t.threads);
+  const int cx = t.T.cx, cy = t.T.cy;
+  TileGeo &T = t.T;
+  T.ni = ni;
+  T.nj = nj;
+  T.halo = t.shrink * t.steps / 2;
+  T.tx = (ni + cx - 1) / cx;
+  T.ty = (nj + cy - 1) / cy;
+  T.cx = (ni + T.tx - 1) / T.tx;
+  T.cy = (nj + T.ty - 1) / T.ty;
+  T.tx = (ni + T.cx - 1) / T.cx;
+  T.ty = (nj + T.cy - 1) / T.cy;
+  T.rx = T.cx + 2 * T.halo;
+  T.rn = T.rx * (T.cy + 2 * T.halo);
+  T.tiles8 = (T.tx * T.ty + 7) / 8;
+  t.lds = (size_t)T.rn * (72 * p.nsubs + 4);
+  if (T.rn > kTileRegion || t.lds > (size_t)h->lds_cu) return 0;
+  const long n = (long)T.tx * T.ty;
+  const size_t sb = (size_t)h->tiles * p.nsubs * h->Q * kTile * h->st_bytes;
+  if (hipMalloc(&t.gidx, (size_t)n * T.rn * sizeof(int)) != hipSuccess ||
+      hipMalloc(&t.list, (size_t)n * T.rn * sizeof(uint32_t)) != hipSuccess ||
+      hipMalloc(&t.cnt, (size_t)n * (kTileHalo + 1) * sizeof(int)) != hipSuccess ||
+      hipMalloc(&t.F2, sb) != hipSuccess) {
+    (void)hipGetLastError();
+    free_tiles(h);
+    h->tile.state = -1;
+    return 0;
+  }
+  const StepArgs<double, double> A = make_args<double, double>(h);
+  hipLaunchKernelGGL(k_tile_build, dim3((unsigned)n), dim3(256), 0, h->stream, A.G, T, t.gidx, t.list, t.cnt);
+  HIP_OK(hipGetLastError());
+  t.state = 1;
+  return 0;
+}
+
+bool solute_on(const lbm_handle *h, int t) {
+  return h->p.nsubs == 2 && t >= h->p.sigma_t_on && t <= h->p.sigma_t_off;
+}
+
+// The number of steps (even, possibly 0) that one tile launch may take from
+// the next step on, of n left to run.
+int tile_steps(const lbm_handle *h, int n) {
+  const int t1 = h->time + 1;
+  if (!(t1 & 1)) return 0;
+  int len = std::min(n, h->tile.steps) & ~1;
+  while (len > 0) {
+    bool same = true;
+    for (int q = 1; q < len; q++) same = same && solute_on(h, t1 + q) == solute_on(h, t1);
+    if (same) break;
+    len -= 2;
+  }
+  return len;
+}
+
+int run_tile(lbm_handle *h, int steps, int write_macro) {
+  const lbm_params &p = h->p;
+  auto &t = h->tile;
+  TileArgs B{};
+  B.A = make_args<double, double>(h);
+  B.A.Fo = (double *)t.F2;
+  B.A.write_mv = write_macro;
+  B.A.ns = h->ns;
+  const bool sol = solute_on(h, h->time + 1);
+  B.A.solute_on = sol;
+  B.T = t.T;
+  B.gidx = t.gidx;
+  B.list = t.list;
+  B.cnt = t.cnt;
+  B.steps = steps;
+  B.shrink = t.shrink;
+  for (int side = 0; side < 2; side++) {
+    int which;
+    (void)row_condition(p, side, B.flow[side], which);
+    B.grad[side] = p.nsubs == 2 && (side == 0 ? p.zeroconcgrad_n : p.zeroconcgrad_s);
+    for (int k = 0; k < steps && B.flow[side]; k++) {
+      const int at = h->time + 1 + k;
+      B.val[side][k] = B.flow[side] == 2 ? p.rho_A[0] * bc_uy(h, which, at) : bc_rho(h, 0, which, at);
+    }
+  }
+  int rc;
+  if (p.nsubs == 1) rc = h->ns ? tile_launch<1, false, true>(h, B) : tile_launch<1, false, false>(h, B);
+  else if (sol) rc = h->ns ? tile_launch<2, true, true>(h, B) : tile_launch<2, true, false>(h, B);
+  else rc = h->ns ? tile_launch<2, false, true>(h, B) : tile_launch<2, false, false>(h, B);
+  if (rc) return rc;
+  std::swap(h->F, t.F2);
+  h->time += steps;
+  return 0;
+}
+
 }  // namespace
 
 extern "C" int lbm_run(lbm_handle *h, int nsteps, int write_macro_last) {
   if (need_lattice(h)) return 1;
   int q = 0;
+  if (nsteps >= 2 && !h->profile && plan_tiles(h)) return 1;
+  if (nsteps >= 2 && !h->profile && h->tile.state == 1) {
+    // a step that records the plane flux reads the state before it
+    const int keep = h->n_flux && write_macro_last ? 1 : 0;
+    while (q < nsteps) {
+      const int len = tile_steps(h, nsteps - q - keep);
+      if (len ? run_tile(h, len, q + len == nsteps ? write_macro_last : 0)
+              : do_step(h, q == nsteps - 1 ? write_macro_last : 0))
+        return 1;
+      q += len ? len : 1;
+    }
+    return sync(h);
+  }
   // the steps before the last in captured chunks where their launches repeat
   if (nsteps - 1 >= kChunk && chunkable(h, h->time + 1, h->time + nsteps - 1)) {
     while (nsteps - 1 - q >= kChunk) {

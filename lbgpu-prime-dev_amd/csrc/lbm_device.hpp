@@ -388,7 +388,13 @@ __device__ __forceinline__ CT cdotu(CT u0, CT u1, CT u2) {
 // WALSH: partial bounce-back (src/k_stream_collide_stream.c:129-135,183-192,
 // src/lattice.c:2936-2939): the momentum and the force enter u scaled by
 // kns = 1 - ns; the caller mixes the opposite pre-collision populations in.
-template <int Q, typename ST, typename CT, int SUBS, bool ODD, bool WALSH = false>
+// LEAN (FP64): the same values in fewer operations, for kernels that the
+// FP64 units bound.  The products by the velocity components 0 and +-1 are
+// exact, so skipping them changes no finite result; 0 * rho, added to each
+// momentum sum, keeps what they did to others (one infinite or NaN population
+// makes all of u NaN); x / 1 is x; and an opposite direction's 3 v and
+// 4.5 v v are the direction's own, negated and unchanged.
+template <int Q, typename ST, typename CT, int SUBS, bool ODD, bool WALSH = false, bool LEAN = false>
 __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (&f)[Q], CT (&u)[3],
                                         CT kns = (CT)1) {
   constexpr int D = Q == 9 ? 2 : 3;
@@ -409,6 +415,15 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
           u[2] = D == 3 ? add_c<CZ(A), CT>(u[2], f[A]) : u[2]),
          ...);
       }(std::make_integer_sequence<int, Q>{});
+    } else if constexpr (LEAN) {
+      [&]<int... A>(std::integer_sequence<int, A...>) {
+        ((u[0] = add_c<CX(A), CT>(u[0], f[A]), u[1] = add_c<CY(A), CT>(u[1], f[A]),
+          u[2] = D == 3 ? add_c<CZ(A), CT>(u[2], f[A]) : u[2]),
+         ...);
+      }(std::make_integer_sequence<int, Q>{});
+      const CT z = (CT)0 * rho;
+#pragma unroll
+      for (int d = 0; d < D; d++) u[d] += z;
     } else {
       // FP64: as written (the skipped form frees registers, and the flow +
       // solute odd step's second workgroup per CU then slows it by 5 % at
@@ -437,8 +452,10 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
 #pragma unroll
       for (int d = 0; d < D; d++) u[d] *= kns;
     }
+    if (!LEAN || A.rhoA != (CT)1) {
 #pragma unroll
-    for (int d = 0; d < D; d++) u[d] /= A.rhoA;
+      for (int d = 0; d < D; d++) u[d] /= A.rhoA;
+    }
     if constexpr (WALSH) {
 #pragma unroll
       for (int d = 0; d < D; d++) u[d] += kns * A.tau * A.g[d];
@@ -473,7 +490,7 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
   }
   const CT it = SUBS == 0 ? A.inv_tau : A.inv_tau_s;
   CT vd[Q];
-  if constexpr (sizeof(CT) == 4) {
+  if constexpr (sizeof(CT) == 4 || LEAN) {
     [&]<int... A>(std::integer_sequence<int, A...>) {
       ((vd[A] = cdotu<CX(A), CY(A), D == 3 ? CZ(A) : 0, CT>(u[0], u[1], u[2])), ...);
     }(std::make_integer_sequence<int, Q>{});
@@ -500,6 +517,27 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
       if (SUBS == 1) t = B * __builtin_fmaf((CT)3, v, (CT)1);
       else t = __builtin_fmaf(C, v * __builtin_fmaf((CT)4.5, v, (CT)3), B);
       f[a] = __builtin_fmaf(f[a], k1, w * t);
+    }
+  } else if constexpr (LEAN) {
+    const CT k1 = (CT)1 - it, s15 = (CT)1.5 * usq;
+    auto relax = [&](int a, CT v3, CT v45) {
+      CT fa = f[a] * k1;
+      const CT w = (CT)W<Q>(a);
+      if (SUBS == 1) {
+        fa += w * rho * ((CT)1 + v3) * it;
+      } else {
+        fa += w * rho * it;
+        fa += w * A.rhoA * (v3 + v45 - s15) * it;
+      }
+      f[a] = fa;
+    };
+    relax(0, SUBS == 1 ? (CT)0 * u[0] : (CT)0, (CT)0);
+#pragma unroll
+    for (int a = 1; a < Q; a += 2) {
+      const CT v3 = (CT)3 * vd[a];
+      const CT v45 = SUBS == 0 ? (CT)4.5 * vd[a] * vd[a] : (CT)0;
+      relax(a, v3, v45);
+      relax(a + 1, -v3, v45);
     }
   } else {
 #pragma unroll
@@ -812,16 +850,12 @@ __device__ __forceinline__ void bc_store(const BcArgs<ST, CT> &B, int idx, const
 // opp(a), where the pull reads it (as the 3-D faces do), instead of the
 // reference rows' own slot a (which leaves the bounced value in place and
 // hands the unknown to the interior node beside a side wall).
-template <int NS, typename ST, typename CT, int SUBS>
-__global__ void k_bc2d_pressure(BcArgs<ST, CT> B, int north, double rho_b, int velocity) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B.n) return;
-  const int idx = B.list[t];
-  int nb[9];
-  CT f[9];
-  bc_gather<9, NS, ST, CT, SUBS>(B, idx, nb, f);
+// Values of the three unknowns of a row node, in the order S, SE, SW (north)
+// or N, NE, NW (south).
+template <typename CT>
+__device__ __forceinline__ void bc2d_flow_values(const CT (&f)[9], bool north, double rho_b, CT rhoA, bool velocity,
+                                                 CT (&v)[3]) {
   enum { C_ = 0, E_, W_, N_, S_, NE_, SW_, NW_, SE_ };
-  const CT rhoA = SUBS == 0 ? B.A.rhoA : B.A.rhoA_s;
   if (north) {
     CT x = f[C_] + f[E_] + f[W_] + f[N_] + f[N_] + f[NE_] + f[NE_] + f[NW_] + f[NW_];
     if (velocity) {
@@ -832,12 +866,9 @@ __global__ void k_bc2d_pressure(BcArgs<ST, CT> B, int north, double rho_b, int v
       x -= (CT)rho_b;
       x += rhoA;
     }
-    CT vS = f[N_] - ((CT)(2. / 3.)) * x;
-    CT vSW = f[NE_] + ((CT)(1. / 2.)) * (f[E_] - f[W_]) - ((CT)(1. / 6.)) * x;
-    CT vSE = f[NW_] + ((CT)(1. / 2.)) * (f[W_] - f[E_]) - ((CT)(1. / 6.)) * x;
-    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, S_, vS, velocity);
-    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, SE_, vSE, velocity);
-    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, SW_, vSW, velocity);
+    v[0] = f[N_] - ((CT)(2. / 3.)) * x;
+    v[2] = f[NE_] + ((CT)(1. / 2.)) * (f[E_] - f[W_]) - ((CT)(1. / 6.)) * x;
+    v[1] = f[NW_] + ((CT)(1. / 2.)) * (f[W_] - f[E_]) - ((CT)(1. / 6.)) * x;
   } else {
     CT x = -f[C_] - f[E_] - f[W_] - f[S_] - f[S_] - f[SE_] - f[SE_] - f[SW_] - f[SW_];
     if (velocity) {
@@ -848,37 +879,63 @@ __global__ void k_bc2d_pressure(BcArgs<ST, CT> B, int north, double rho_b, int v
       x += (CT)rho_b;
       x -= rhoA;
     }
-    CT vN = f[S_] + ((CT)(2. / 3.)) * x;
-    CT vNE = f[SW_] + ((CT)(1. / 2.)) * (f[W_] - f[E_]) + ((CT)(1. / 6.)) * x;
-    CT vNW = f[SE_] + ((CT)(1. / 2.)) * (f[E_] - f[W_]) + ((CT)(1. / 6.)) * x;
-    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, N_, vN, velocity);
-    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, NW_, vNW, velocity);
-    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, NE_, vNE, velocity);
+    v[0] = f[S_] + ((CT)(2. / 3.)) * x;
+    v[1] = f[SW_] + ((CT)(1. / 2.)) * (f[W_] - f[E_]) + ((CT)(1. / 6.)) * x;
+    v[2] = f[SE_] + ((CT)(1. / 2.)) * (f[E_] - f[W_]) + ((CT)(1. / 6.)) * x;
+  }
+}
+
+template <int NS, typename ST, typename CT, int SUBS>
+__global__ void k_bc2d_pressure(BcArgs<ST, CT> B, int north, double rho_b, int velocity) {
+  int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= B.n) return;
+  const int idx = B.list[t];
+  int nb[9];
+  CT f[9], v[3];
+  bc_gather<9, NS, ST, CT, SUBS>(B, idx, nb, f);
+  bc2d_flow_values<CT>(f, north, rho_b, SUBS == 0 ? B.A.rhoA : B.A.rhoA_s, velocity, v);
+  // constant slots in both branches (a run-time slot would index the neighbour ranks in scratch memory)
+  if (north) {
+    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 4, v[0], velocity);
+    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 8, v[1], velocity);
+    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 6, v[2], velocity);
+  } else {
+    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 3, v[0], velocity);
+    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 7, v[2], velocity);
+    bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 5, v[1], velocity);
   }
 }
 
 // 2-D solute zero concentration gradient on the N or S row:
 // k_sysbound_zeroconcgrad_{n,s}_{1,2}, src/system_boundary_kernels.c:454-831
+template <typename CT>
+__device__ __forceinline__ void bc2d_zerograd_values(const CT (&f)[9], bool north, CT (&v)[3]) {
+  enum { C_ = 0, E_, W_, N_, S_, NE_, SW_, NW_, SE_ };
+  constexpr double w1 = W<9>(1), w2 = W<9>(5);
+  const CT c = north ? (f[N_] + f[NE_] + f[NW_]) / ((CT)(w1 + w2 + w2))
+                     : (f[S_] + f[SW_] + f[SE_]) / ((CT)(w1 + w2 + w2));
+  v[0] = (CT)w1 * c;
+  v[1] = (CT)w2 * c;
+  v[2] = (CT)w2 * c;
+}
+
 template <typename ST, typename CT>
 __global__ void k_bc2d_zerograd(BcArgs<ST, CT> B, int north) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= B.n) return;
   const int idx = B.list[t];
   int nb[9];
-  CT f[9];
+  CT f[9], v[3];
   bc_gather<9, 2, ST, CT, 1>(B, idx, nb, f);
-  enum { C_ = 0, E_, W_, N_, S_, NE_, SW_, NW_, SE_ };
-  constexpr double w1 = W<9>(1), w2 = W<9>(5);
+  bc2d_zerograd_values<CT>(f, north, v);
   if (north) {
-    CT c = (f[N_] + f[NE_] + f[NW_]) / ((CT)(w1 + w2 + w2));
-    bc_store<9, 2, ST, CT, 1>(B, idx, nb, S_, (CT)w1 * c, false);
-    bc_store<9, 2, ST, CT, 1>(B, idx, nb, SE_, (CT)w2 * c, false);
-    bc_store<9, 2, ST, CT, 1>(B, idx, nb, SW_, (CT)w2 * c, false);
+    bc_store<9, 2, ST, CT, 1>(B, idx, nb, 4, v[0], false);
+    bc_store<9, 2, ST, CT, 1>(B, idx, nb, 8, v[1], false);
+    bc_store<9, 2, ST, CT, 1>(B, idx, nb, 6, v[2], false);
   } else {
-    CT c = (f[S_] + f[SW_] + f[SE_]) / ((CT)(w1 + w2 + w2));
-    bc_store<9, 2, ST, CT, 1>(B, idx, nb, N_, (CT)w1 * c, false);
-    bc_store<9, 2, ST, CT, 1>(B, idx, nb, NW_, (CT)w2 * c, false);
-    bc_store<9, 2, ST, CT, 1>(B, idx, nb, NE_, (CT)w2 * c, false);
+    bc_store<9, 2, ST, CT, 1>(B, idx, nb, 3, v[0], false);
+    bc_store<9, 2, ST, CT, 1>(B, idx, nb, 7, v[2], false);
+    bc_store<9, 2, ST, CT, 1>(B, idx, nb, 5, v[1], false);
   }
 }
 

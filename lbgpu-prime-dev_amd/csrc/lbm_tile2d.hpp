@@ -1,0 +1,304 @@
+// Several D2Q9 time steps per launch (FP64 storage and collision).
+//
+// A single 2-D step is short of work for this GPU: the lattices that users
+// run (10^3 to 10^6 nodes) live in cache, and each step costs two to five
+// launches (the half-step and the boundary rows) and one read and one write
+// of every population.  k_tile2d advances a tile of the lattice by an even
+// number of steps inside one workgroup instead: it loads the tile's core and
+// a halo of nodes around it into LDS, runs the in-place AA half-steps there
+// (odd, even, odd, ...), boundary rows included, and stores the core into a
+// second population array.  The halo shrinks with every odd half-step, so
+// neighbouring tiles repeat each other's halo work and need no exchange.
+//
+// Validity of LDS locations (slot b of region node y), by the distance of y
+// from the region's edge: all are valid at the start (s = 0).  An odd
+// half-step at x reads and writes the locations (b, x - c_b): it can run
+// where dist(x) >= s + 1, and a location is valid afterwards where its
+// writer ran: dist >= s + 2.  An even half-step is node-local: it runs where
+// dist >= s.  A row condition whose source node is solid hands its value to
+// a neighbour's input (the reference's own-slot rule), which costs one more
+// node per odd half-step.  The halo is thus 2 (or 3) nodes per pair of steps.
+//
+// The arithmetic is collide() of the half-step kernel on the same values, so
+// results equal the step-by-step launches bit for bit.
+//
+// Measured per step, against half-steps and row launches one by one: 128^2
+// flow between walls 3.3 -> 1.3 us; 1088 x 1224 flow + solute with series rows
+// 58 -> 28 us; 600 x 500 with partial bounce-back 24 -> 7.8 us; 413 x 307
+// with rows 18.5 -> 3.6 us.  Small lattices are bound by the latency of a
+// step inside the workgroup (about 1 us: LDS gathers, the collision's serial
+// sums, the barrier), large ones by the loads of core and halo (1.7 times the
+// core at 25 x 25 with 4 steps) followed by the FP64 units, which one
+// workgroup per CU does not overlap.
+#pragma once
+
+#include "lbm_device.hpp"
+
+namespace lbm {
+
+constexpr int kTileSteps = 16;   // most steps of one launch
+constexpr int kTileHalo = 24;    // widest halo: 3 nodes per pair of steps
+constexpr int kTileRegion = 4096;  // most region nodes (12-bit region index)
+
+// list entry of a fluid region node: region index, bit 12 + a - 1 set when
+// x - c_a is fluid, and the boundary rows
+constexpr uint32_t kTileNorth = 1u << 20, kTileSouth = 1u << 21;
+
+struct TileGeo {
+  int ni, nj;
+  int cx, cy;      // core size
+  int tx, ty;      // tiles
+  int halo;        // H
+  int rx, rn;      // region row length cx + 2 H and node count
+  int tiles8;      // launched tiles / 8 (XCD mapping)
+};
+
+// core origin, core size and region size of tile t
+LBM_HD void tile_span(const TileGeo &T, int t, int &x0, int &y0, int &cw, int &ch) {
+  const int ty = t / T.tx, tx = t - ty * T.tx;
+  x0 = tx * T.cx;
+  y0 = ty * T.cy;
+  cw = T.ni - x0 < T.cx ? T.ni - x0 : T.cx;
+  ch = T.nj - y0 < T.cy ? T.nj - y0 : T.cy;
+}
+
+// Per tile: gidx[rn] (compact index of each region node, -1: solid or
+// outside), the list of its fluid nodes ordered by distance from the region's
+// edge (core first, then ring by ring inwards to outwards, each row-major),
+// and cnt[d] = number of list entries with distance >= d, d = 0..H.
+__global__ __launch_bounds__(256) void k_tile_build(Geo G, TileGeo T, int *gidx, uint32_t *list, int *cnt) {
+  __shared__ int wsum[4];
+  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int x0, y0, cw, ch;
+  tile_span(T, t, x0, y0, cw, ch);
+  const int rw = cw + 2 * T.halo, rh = ch + 2 * T.halo;
+  int *g = gidx + (long)t * T.rn;
+  uint32_t *l = list + (long)t * T.rn;
+  auto wrap = [](int v, int n) {
+    v %= n;
+    return v < 0 ? v + n : v;
+  };
+  for (int n = tid; n < T.rn; n += 256) {
+    const int ry = n / T.rx, rx = n - ry * T.rx;
+    g[n] = rx < rw && ry < rh ? rank_of(G, wrap(x0 - T.halo + rx, T.ni), wrap(y0 - T.halo + ry, T.nj)) : -1;
+  }
+  int run = 0;
+  for (int d = T.halo; d >= 0; d--) {
+    for (int base = 0; base < T.rn; base += 256) {
+      const int n = base + tid;
+      bool in = false;
+      int rx = 0, ry = 0;
+      if (n < T.rn) {
+        ry = n / T.rx;
+        rx = n - ry * T.rx;
+        int dist = rx < rw - 1 - rx ? rx : rw - 1 - rx;
+        dist = ry < dist ? ry : dist;
+        dist = rh - 1 - ry < dist ? rh - 1 - ry : dist;
+        dist = T.halo < dist ? T.halo : dist;
+        in = g[n] >= 0 && dist == d;
+      }
+      const uint64_t bal = __ballot(in);
+      if (lane == 0) wsum[wv] = __popcll(bal);
+      __syncthreads();
+      int at = run + __popcll(bal & ((1ull << lane) - 1ull));
+      for (int q = 0; q < wv; q++) at += wsum[q];
+      if (in) {
+        const int i = wrap(x0 - T.halo + rx, T.ni), j = wrap(y0 - T.halo + ry, T.nj);
+        uint32_t e = (uint32_t)n;
+#pragma unroll
+        for (int a = 1; a < 9; a++)
+          if (rank_of(G, wrap1(i - CX(a), T.ni), wrap1(j - CY(a), T.nj)) >= 0) e |= 1u << (11 + a);
+        if (j == T.nj - 1) e |= kTileNorth;
+        if (j == 0) e |= kTileSouth;
+        l[at] = e;
+      }
+      run += wsum[0] + wsum[1] + wsum[2] + wsum[3];
+      __syncthreads();
+    }
+    if (tid == 0) cnt[(long)t * (kTileHalo + 1) + d] = run;
+  }
+}
+
+struct TileArgs {
+  StepArgs<double, double> A;  // A.F: populations read, A.Fo: where they are written
+  TileGeo T;
+  const int *gidx;
+  const uint32_t *list;
+  const int *cnt;
+  int steps;             // even, the first one odd
+  int shrink;            // halo nodes an odd half-step uses up: 2, or 3 with handed-on row values
+  int flow[2];           // row condition of the flow, [0] north, [1] south: 0 none, 1 density, 2 y momentum
+  int grad[2];           // solute zero gradient
+  double val[2][kTileSteps];  // prescribed value per step
+};
+
+// the pair of one location in LDS
+template <int NS>
+using tile_t = double __attribute__((ext_vector_type(NS)));
+
+// Row conditions of one region node on the populations it has gathered; f
+// and gs hold what the node collides.  put(s, a, v, own_opp) takes the value
+// of unknown a of component s.
+template <int NS, typename Put>
+__device__ __forceinline__ void tile_rows(const TileArgs &B, uint32_t e, int step, const double (&f)[9],
+                                          const double (&gs)[9], Put &&put) {
+  auto side = [&](bool north, int q, int u0, int u1, int u2) {
+    double v[3];
+    if (B.flow[q]) {
+      bc2d_flow_values<double>(f, north, B.val[q][step], B.A.rhoA, B.flow[q] == 2, v);
+      put(0, u0, v[0], B.flow[q] == 2);
+      put(0, u1, v[1], B.flow[q] == 2);
+      put(0, u2, v[2], B.flow[q] == 2);
+    }
+    if (NS == 2 && B.grad[q]) {
+      bc2d_zerograd_values<double>(gs, north, v);
+      put(1, u0, v[0], false);
+      put(1, u1, v[1], false);
+      put(1, u2, v[2], false);
+    }
+  };
+  if (e & kTileNorth) side(true, 0, 4, 8, 6);
+  if (e & kTileSouth) side(false, 1, 3, 5, 7);
+}
+
+// the nine locations node n collides from: slot a of x - c_a (own slot
+// opp(a) when that node is solid) before an odd half-step, own slot opp(a)
+// before an even one; an odd half-step pushes f_a to location opp(a)
+template <bool ODD>
+__device__ __forceinline__ void tile_locs(const TileGeo &T, uint32_t e, int n, int (&loc)[9]) {
+  loc[0] = n;
+#pragma unroll
+  for (int a = 1; a < 9; a++) {
+    const int own = OPP(a) * T.rn + n;
+    loc[a] = ODD && ((e >> (11 + a)) & 1u) ? a * T.rn + n - CX(a) - CY(a) * T.rx : own;
+  }
+}
+
+// one half-step of one region node; LAST: the result goes to the output
+// array, else back to LDS
+template <int NS, bool SOL, bool WALSH, bool ODD, bool LAST>
+__device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<double, double> &A, tile_t<NS> *lds,
+                                          const int *g, uint32_t e, bool rows, int step) {
+  const int n = (int)(e & 4095u), rn = B.T.rn;
+  int loc[9];
+  tile_locs<ODD>(B.T, e, n, loc);
+  double f[9], gs[9], u[3];
+#pragma unroll
+  for (int a = 0; a < 9; a++) {
+    const tile_t<NS> v = lds[loc[a]];
+    f[a] = v[0];
+    if constexpr (NS == 2) gs[a] = v[NS - 1];
+  }
+  if (rows && (e & (kTileNorth | kTileSouth)))
+    tile_rows<NS>(B, e, step, f, gs, [&](int s, int a, double v, bool) {
+      if (s == 0) f[a] = v;
+      else gs[a] = v;
+      // a resting solute is not collided: its row values are stored
+      if constexpr (NS == 2 && !SOL && !LAST)
+        if (s == 1) lds[loc[a]][NS - 1] = v;
+    });
+  const int idx = (WALSH || LAST) ? g[n] : 0;
+  double ns = 0., kns = 1.;
+  if constexpr (WALSH) {
+    ns = A.ns[idx];
+    kns = 1. - ns;
+    double fp[9], gp[9];
+#pragma unroll
+    for (int a = 0; a < 9; a++) {
+      fp[a] = f[a];
+      if (SOL) gp[a] = gs[a];
+    }
+    collide<9, double, double, 0, ODD, true, true>(A, idx, f, u, kns);
+    if constexpr (SOL) collide<9, double, double, 1, ODD, true, true>(A, idx, gs, u, kns);
+    walsh_mix<9, double>(f, fp, ns, kns);
+    if constexpr (SOL) walsh_mix<9, double>(gs, gp, ns, kns);
+  } else {
+    collide<9, double, double, 0, ODD, false, true>(A, idx, f, u);
+    if constexpr (SOL) collide<9, double, double, 1, ODD, false, true>(A, idx, gs, u);
+  }
+#pragma unroll
+  for (int a = 0; a < 9; a++) {
+    // even: own slot a (a resting solute keeps its slot a, gathered as direction opp(a))
+    const int at = ODD ? loc[OPP(a)] : a * rn + n;
+    tile_t<NS> v;
+    v[0] = f[a];
+    if constexpr (NS == 2) v[NS - 1] = SOL ? gs[a] : gs[OPP(a)];
+    if constexpr (LAST)
+      *(tile_t<NS> *)(A.Fo + (size_t)foff<9, NS>(0, a, (uint32_t)idx)) = v;
+    else if constexpr (NS == 2 && !SOL)
+      lds[at][0] = v[0];
+    else
+      lds[at] = v;
+  }
+}
+
+template <int NS, bool SOL, bool WALSH, int NT>
+__global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
+  extern __shared__ __align__(16) char tile_lds[];
+  const int t = xcd_block(B.T.tiles8);
+  if (t >= B.T.tx * B.T.ty) return;
+  const int tid = threadIdx.x, rn = B.T.rn, H = B.T.halo;
+  tile_t<NS> *lds = (tile_t<NS> *)tile_lds;
+  uint32_t *lst = (uint32_t *)(lds + 9 * rn);
+  const int *g = B.gidx + (long)t * rn;
+  const int *cnt = B.cnt + (long)t * (kTileHalo + 1);
+  const int fluid = cnt[0], core = cnt[H];
+  if (core == 0) return;
+  for (int n = tid; n < rn; n += NT) {
+    const int idx = g[n];
+    if (n < fluid) lst[n] = B.list[(long)t * rn + n];
+    if (idx < 0) continue;
+    tile_t<NS> v[9];
+#pragma unroll
+    for (int a = 0; a < 9; a++) v[a] = *(const tile_t<NS> *)(B.A.F + (size_t)foff<9, NS>(0, a, (uint32_t)idx));
+#pragma unroll
+    for (int a = 0; a < 9; a++) lds[a * rn + n] = v[a];
+  }
+  __syncthreads();
+  const bool rows = B.flow[0] || B.flow[1] || (NS == 2 && (B.grad[0] || B.grad[1]));
+  const bool handed = B.shrink > 2;
+  StepArgs<double, double> A = B.A;
+  A.write_mv = 0;
+  int s = 0;
+  for (int k = 0; k < B.steps; k += 2) {
+    if (handed) {
+      // row values that go to a neighbour's input: stored before any node collides
+      const int act = cnt[s + 1];
+      for (int p = tid; p < act; p += NT) {
+        const uint32_t e = lst[p];
+        if (!(e & (kTileNorth | kTileSouth))) continue;
+        const int n = (int)(e & 4095u);
+        int loc[9];
+        tile_locs<true>(B.T, e, n, loc);
+        double f[9], gs[9];
+#pragma unroll
+        for (int a = 0; a < 9; a++) {
+          f[a] = lds[loc[a]][0];
+          if constexpr (NS == 2) gs[a] = lds[loc[a]][NS - 1];
+        }
+        // the rule of bc_store: own slot a (or opp(a)) when the source is solid
+        tile_rows<NS>(B, e, k, f, gs, [&](int s, int a, double v, bool own_opp) {
+          lds[(e >> (11 + a)) & 1u ? loc[a] : (own_opp ? OPP(a) : a) * rn + n][s ? NS - 1 : 0] = v;
+        });
+      }
+      __syncthreads();
+    }
+    const int odd = cnt[s + B.shrink - 1];
+    for (int p = tid; p < odd; p += NT)
+      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, g, lst[p], rows && !handed, k);
+    s += B.shrink;
+    __syncthreads();
+    if (k + 2 < B.steps) {
+      const int even = cnt[s];
+      for (int p = tid; p < even; p += NT)
+        tile_node<NS, SOL, WALSH, false, false>(B, A, lds, g, lst[p], rows, k + 1);
+      __syncthreads();
+    } else {
+      A.write_mv = B.A.write_mv;
+      for (int p = tid; p < core; p += NT)
+        tile_node<NS, SOL, WALSH, false, true>(B, A, lds, g, lst[p], rows, k + 1);
+    }
+  }
+}
+
+}  // namespace lbm
