@@ -16,6 +16,7 @@
 #include "lbm_device.hpp"
 #include "lbm_internal.h"
 #include "lbm_mi355x.h"
+#include "lbm_stage.hpp"
 #include "lbm_tile2d.hpp"
 
 using namespace lbm;
@@ -129,6 +130,7 @@ struct lbm_handle {
   int flux_valid = 0;
   int time = 0;
   hipStream_t stream = nullptr;
+  hipEvent_t stage_ev[kStageSlots] = {};  // host transfers (lbm_stage.hpp)
   double *scratch = nullptr;  // this device's address of the static staging array
   int profile = 0;
   std::vector<ProfPair> pending;
@@ -747,6 +749,7 @@ extern "C" int lbm_create(const lbm_params *p, lbm_handle **out) {
     return lbm_fail("velocity rows are 2-D conditions (3-D: zface_flow)");
   }
   lbm_handle *h = new lbm_handle();
+  stage_join();
   h->p = *p;
   if (p->dims == 2) h->p.nk = 1;
   if (p->dims == 3) {
@@ -792,6 +795,7 @@ extern "C" int lbm_create(const lbm_params *p, lbm_handle **out) {
   }
   h->p.c_bot_map = nullptr;
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
+    stage_leave();
     delete h;
     return lbm_fail("hipStreamCreate failed");
   }
@@ -838,6 +842,9 @@ extern "C" int lbm_destroy(lbm_handle *h) {
     (void)hipEventDestroy(pp.b);
   }
   for (auto e : h->pool) (void)hipEventDestroy(e);
+  for (auto e : h->stage_ev)
+    if (e) (void)hipEventDestroy(e);
+  stage_leave();
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return 0;
@@ -944,47 +951,44 @@ extern "C" int lbm_set_solids(lbm_handle *h, const uint8_t *mask) {
   return 0;
 }
 
+// Moves the pieces of a transfer through pinned memory (lbm_stage.hpp)
+template <typename Device, typename Host>
+static int move_pieces(lbm_handle *h, int comps, bool up, Device &&device, Host &&host) {
+  try {
+    const hipError_t e = staged(pieces_of(comps, h->N), up, h->stream, h->stage_ev, device, host);
+    if (e != hipSuccess) return lbm_fail("transfer: %s", hipGetErrorString(e));
+  } catch (const std::exception &x) {
+    return lbm_fail("transfer: %s", x.what());
+  }
+  return 0;
+}
+
 static int transfer_f(lbm_handle *h, int subs, double *f1d, int up) {
   if (need_lattice(h)) return 1;
   if (subs < 0 || subs >= h->p.nsubs) return lbm_fail("bad subs %d", subs);
   if (!f1d) return lbm_fail("null population array");
-  const int Q = h->Q, nf = h->nf;
-  std::vector<double> st((size_t)Q * nf);
-  double *dstage = nullptr;
-  HIP_OK(hipMalloc(&dstage, st.size() * sizeof(double)));
-  if (up) {
-    for (int a = 0; a < Q; a++)
-      for (int x = 0; x < nf; x++) st[(size_t)a * nf + x] = f1d[(long)a * h->N + h->node_host[x]];
-    HIP_OK(hipMemcpy(dstage, st.data(), st.size() * sizeof(double), hipMemcpyHostToDevice));
-  }
-  int rc = dispatch(h, [&]<int QQ, int NS, typename ST, typename CT>() -> int {
-    StepArgs<ST, CT> A = make_args<ST, CT>(h);
-    dim3 g(blocks_for(nf)), b(256);
-    if (up) {
-      if (subs == 0) hipLaunchKernelGGL((k_encode<QQ, NS, ST, CT, 0>), g, b, 0, h->stream, A, dstage);
-      else if constexpr (NS == 2) hipLaunchKernelGGL((k_encode<QQ, NS, ST, CT, 1>), g, b, 0, h->stream, A, dstage);
-    } else {
-      if (subs == 0) hipLaunchKernelGGL((k_decode<QQ, NS, ST, CT, 0>), g, b, 0, h->stream, A, dstage);
-      else if constexpr (NS == 2) hipLaunchKernelGGL((k_decode<QQ, NS, ST, CT, 1>), g, b, 0, h->stream, A, dstage);
-    }
-    HIP_OK(hipGetLastError());
-    return 0;
+  return dispatch(h, [&]<int Q, int NS, typename ST, typename CT>() -> int {
+    const StepArgs<ST, CT> A = make_args<ST, CT>(h);
+    auto device = [&](const Piece &p, double *slot) {
+      const dim3 g(blocks_for(p.nn), p.nc), b(256);
+      if (subs == 0) {
+        if (up) hipLaunchKernelGGL((k_dense_put<Q, NS, ST, CT, 0>), g, b, 0, h->stream, A, p.c0, p.n0, p.nn, slot);
+        else hipLaunchKernelGGL((k_dense_get<Q, NS, ST, CT, 0>), g, b, 0, h->stream, A, p.c0, p.n0, p.nn, slot);
+      } else if constexpr (NS == 2) {
+        if (up) hipLaunchKernelGGL((k_dense_put<Q, NS, ST, CT, 1>), g, b, 0, h->stream, A, p.c0, p.n0, p.nn, slot);
+        else hipLaunchKernelGGL((k_dense_get<Q, NS, ST, CT, 1>), g, b, 0, h->stream, A, p.c0, p.n0, p.nn, slot);
+      }
+      return hipGetLastError();
+    };
+    // the slots of one piece are consecutive in f1d
+    auto host = [&](const Piece &p, double *slot) {
+      double *mine = f1d + (long)p.c0 * h->N + p.n0;
+      const size_t bytes = (size_t)p.nc * p.nn * sizeof(double);
+      if (up) memcpy(slot, mine, bytes);
+      else memcpy(mine, slot, bytes);
+    };
+    return move_pieces(h, Q, up, device, host);
   });
-  if (!rc) {
-    hipError_t e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) rc = lbm_fail("transfer: %s", hipGetErrorString(e));
-  }
-  if (!rc && !up) {
-    hipError_t e = hipMemcpy(st.data(), dstage, st.size() * sizeof(double), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) rc = lbm_fail("transfer: %s", hipGetErrorString(e));
-    else {
-      memset(f1d, 0, sizeof(double) * Q * h->N);
-      for (int a = 0; a < Q; a++)
-        for (int x = 0; x < nf; x++) f1d[(long)a * h->N + h->node_host[x]] = st[(size_t)a * nf + x];
-    }
-  }
-  (void)hipFree(dstage);
-  return rc;
 }
 
 extern "C" int lbm_set_ns(lbm_handle *h, const double *ns) {
@@ -1025,10 +1029,10 @@ extern "C" int lbm_download_f_noalloc(lbm_handle *h, int subs, double *f1d) {
   double *stage = h->scratch;
   int rc = dispatch(h, [&]<int Q, int NS, typename ST, typename CT>() -> int {
     StepArgs<ST, CT> A = make_args<ST, CT>(h);
-    const dim3 g(blocks_for(h->N)), b(256);
-    if (subs == 0) hipLaunchKernelGGL((k_decode_dense<Q, NS, ST, CT, 0>), g, b, 0, h->stream, A, stage, (int)h->N);
+    const dim3 g(blocks_for(h->N), Q), b(256);
+    if (subs == 0) hipLaunchKernelGGL((k_dense_get<Q, NS, ST, CT, 0>), g, b, 0, h->stream, A, 0, 0L, h->N, stage);
     else if constexpr (NS == 2)
-      hipLaunchKernelGGL((k_decode_dense<Q, NS, ST, CT, 1>), g, b, 0, h->stream, A, stage, (int)h->N);
+      hipLaunchKernelGGL((k_dense_get<Q, NS, ST, CT, 1>), g, b, 0, h->stream, A, 0, 0L, h->N, stage);
     HIP_OK(hipGetLastError());
     return 0;
   });
@@ -1412,19 +1416,27 @@ extern "C" int lbm_halo_periodic(lbm_handle *h, int phase) {
 extern "C" int lbm_download_macro(lbm_handle *h, int subs, double *rho, double *ux, double *uy, double *uz) {
   if (need_lattice(h)) return 1;
   if (subs < 0 || subs >= h->p.nsubs) return lbm_fail("bad subs %d", subs);
-  HIP_OK(hipStreamSynchronize(h->stream));
   const int nf = h->nf, D = h->D;
-  std::vector<double> buf((size_t)(1 + D) * nf);
-  HIP_OK(hipMemcpy(buf.data(), h->mv + (long)subs * (1 + D) * nf, buf.size() * sizeof(double),
-                   hipMemcpyDeviceToHost));
+  const double *src = h->mv + (long)subs * (1 + D) * nf;
+  const Geo G = make_args<double, double>(h).G;
   double *dst[4] = {rho, ux, uy, uz};
-  for (int c = 0; c < 4; c++) {
-    if (!dst[c]) continue;
-    memset(dst[c], 0, sizeof(double) * h->N);
-    if (c > D) continue;
-    for (int x = 0; x < nf; x++) dst[c][h->node_host[x]] = buf[(size_t)c * nf + x];
-  }
-  return 0;
+  // components beyond the lattice's velocity are 0; null ones are skipped
+  auto device = [&](const Piece &p, double *slot) {
+    const int nc = std::min(p.nc, 1 + D - p.c0);
+    if (nc > 0)
+      hipLaunchKernelGGL(k_dense_field, dim3(blocks_for(p.nn), nc), dim3(256), 0, h->stream, G, src, nf, p.c0, p.n0,
+                         p.nn, slot);
+    return hipGetLastError();
+  };
+  auto host = [&](const Piece &p, double *slot) {
+    for (int c = 0; c < p.nc; c++) {
+      double *d = dst[p.c0 + c];
+      if (!d) continue;
+      if (p.c0 + c > D) memset(d + p.n0, 0, (size_t)p.nn * sizeof(double));
+      else memcpy(d + p.n0, slot + (size_t)c * p.nn, (size_t)p.nn * sizeof(double));
+    }
+  };
+  return move_pieces(h, 4, false, device, host);
 }
 
 extern "C" int lbm_sample_macro(lbm_handle *h, int subs, int npts, const long *nodes, double *out) {

@@ -6,43 +6,52 @@
 
 namespace lbm {
 
-// staging [Q][nf] doubles <-> storage rows of one subs
-template <int Q, int NS, typename ST, typename CT, int SUBS>
-__global__ void k_encode(StepArgs<ST, CT> A, const double *stage) {
-  int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= A.nf) return;
-#pragma unroll
-  for (int a = 0; a < Q; a++)
-    A.F[foff<Q, NS>(SUBS, a, idx)] =
-        Codec<ST, CT>::enc((CT)stage[(long)a * A.nf + idx], A.scale[SUBS], shift_of<Q, ST, CT, SUBS>(A, a));
+// Dense arrays at the boundary: blockIdx.y is a component of the piece that
+// is moved, nodes n0 .. n0 + nn of the lattice run along x; thread n finds its
+// compact index from the row words (-1: solid).  `host` is pinned memory, read
+// or written in place over the bus, which bounds all three: one 8-byte element
+// per lane, whole lines per wave.  Expanding here replaced per-node loops on
+// the host, whose scattered stores took 8 times the bus time (256^3, flow and
+// solute fields, 1.07 GB: 203 -> 24 ms, 46 GB/s; the bus itself 57 GB/s).
+
+// one node of a piece; false past its end
+__device__ __forceinline__ bool dense_node(const Geo &G, long n0, long nn, long &t, int &idx) {
+  t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nn) return false;
+  const uint32_t n = (uint32_t)(n0 + t), r = fdiv(n, G.div_ni);
+  idx = rank_of(G, (int)(n - r * (uint32_t)G.ni), (int)r);
+  return true;
 }
 
-template <int Q, int NS, typename ST, typename CT, int SUBS>
-__global__ void k_decode(StepArgs<ST, CT> A, double *stage) {
-  int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= A.nf) return;
-#pragma unroll
-  for (int a = 0; a < Q; a++)
-    stage[(long)a * A.nf + idx] = (double)Codec<ST, CT>::dec(A.F[foff<Q, NS>(SUBS, a, idx)], A.inv_scale[SUBS],
-                                                             shift_of<Q, ST, CT, SUBS>(A, a));
+// fields: host[c][n] = src[c][compact node], 0 at a solid node
+__global__ void k_dense_field(Geo G, const double *src, int nf, int c0, long n0, long nn, double *host) {
+  long t;
+  int idx;
+  if (!dense_node(G, n0, nn, t, idx)) return;
+  host[(long)blockIdx.y * nn + t] = idx < 0 ? 0.0 : src[(long)(c0 + blockIdx.y) * nf + idx];
 }
 
-// one distribution in the boundary's dense [Q][N] layout: thread n takes
-// dense node n, finds its compact index from the row words (-1: solid) and
-// writes its Q slots (0 at a solid node), so every element of out is
-// written and nothing of an earlier call's contents survives
+// populations of one subs: slots a0 + blockIdx.y; every element of out is
+// written (0 at a solid node), so nothing of an earlier call survives there
 template <int Q, int NS, typename ST, typename CT, int SUBS>
-__global__ void k_decode_dense(StepArgs<ST, CT> A, double *out, int n_nodes) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= n_nodes) return;
-  const int r = (int)fdiv((uint32_t)n, A.G.div_ni);
-  const int idx = rank_of(A.G, n - r * A.G.ni, r);
-#pragma unroll
-  for (int a = 0; a < Q; a++)
-    out[(long)a * n_nodes + n] =
-        idx < 0 ? 0.0
-                : (double)Codec<ST, CT>::dec(A.F[foff<Q, NS>(SUBS, a, idx)], A.inv_scale[SUBS],
-                                             shift_of<Q, ST, CT, SUBS>(A, a));
+__global__ void k_dense_get(StepArgs<ST, CT> A, int a0, long n0, long nn, double *out) {
+  long t;
+  int idx;
+  if (!dense_node(A.G, n0, nn, t, idx)) return;
+  const int a = a0 + (int)blockIdx.y;
+  out[(long)blockIdx.y * nn + t] =
+      idx < 0 ? 0.0
+              : (double)Codec<ST, CT>::dec(A.F[foff<Q, NS>(SUBS, a, idx)], A.inv_scale[SUBS],
+                                           shift_of<Q, ST, CT, SUBS>(A, a));
+}
+template <int Q, int NS, typename ST, typename CT, int SUBS>
+__global__ void k_dense_put(StepArgs<ST, CT> A, int a0, long n0, long nn, const double *in) {
+  long t;
+  int idx;
+  if (!dense_node(A.G, n0, nn, t, idx) || idx < 0) return;
+  const int a = a0 + (int)blockIdx.y;
+  A.F[foff<Q, NS>(SUBS, a, idx)] = Codec<ST, CT>::enc((CT)in[(long)blockIdx.y * nn + t], A.scale[SUBS],
+                                                      shift_of<Q, ST, CT, SUBS>(A, a));
 }
 
 // rest state: f~ = w rho (3 c.u + 4.5 (c.u)^2 - 1.5 u^2) = 0 at u = 0;

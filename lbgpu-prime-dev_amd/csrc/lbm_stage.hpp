@@ -1,0 +1,158 @@
+// Host arrays to and from the GPU through pinned memory.
+//
+// Fields and populations cross the C ABI as dense FP64 arrays in the
+// caller's ordinary memory.  The GPU expands or compacts them (k_dense_*)
+// while it writes or reads pinned slots directly, and a few host threads copy
+// between the slots and the caller's array, each with a slot of its own, so
+// that the bus and the copies (for a fresh array mostly the cost of its first
+// touch) run together.
+//
+// The slots are one allocation per process, made on first use, at most
+// kStageSlots * kStageSlot bytes, released with the last handle.  A transfer
+// holds them from start to end; transfers of other threads wait.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <string.h>
+
+#include <algorithm>
+#include <atomic>
+#include <mutex>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace lbm {
+
+constexpr int kStageSlots = 8;              // slots, and host threads at most
+constexpr size_t kStageSlot = 2u << 20;     // bytes of a slot
+// One thread (the caller's first) for each MiB: a thread costs about 20 us
+// to start and moves a MiB in 60 us (fields of 1.3 MB: 0.062 ms alone; 2.9 MB:
+// 0.109 ms with two, 0.13 alone, 0.147 with eight; 26 MB: 0.95 with eight).
+constexpr size_t kStageAlone = 1u << 20;
+
+struct Stage {
+  std::mutex mu;
+  int users = 0;
+  char *buf = nullptr;
+  size_t bytes = 0;
+};
+inline Stage &stage() {
+  static Stage s;
+  return s;
+}
+inline void stage_join() {
+  std::lock_guard<std::mutex> lock(stage().mu);
+  stage().users++;
+}
+inline void stage_leave() {
+  Stage &s = stage();
+  std::lock_guard<std::mutex> lock(s.mu);
+  if (--s.users > 0) return;
+  if (s.buf) (void)hipHostFree(s.buf);
+  s.buf = nullptr;
+  s.bytes = 0;
+}
+
+// One piece of a transfer: nc components of nn nodes from node n0, at most a
+// slot's worth; host moves it between the slot and the caller's memory,
+// device (when there is device work) launches the kernel on the slot.
+struct Piece {
+  int c0, nc;
+  long n0, nn;
+};
+
+// the pieces of comps components of N nodes each
+inline std::vector<Piece> pieces_of(int comps, long N) {
+  constexpr long most = (long)(kStageSlot / sizeof(double));
+  std::vector<Piece> v;
+  if (N <= most) {
+    const int group = (int)std::min<long>(comps, std::max<long>(1, most / N));
+    for (int c = 0; c < comps; c += group) v.push_back({c, std::min(group, comps - c), 0, N});
+  } else {
+    for (int c = 0; c < comps; c++)
+      for (long n = 0; n < N; n += most) v.push_back({c, 1, n, std::min(most, N - n)});
+  }
+  return v;
+}
+
+// Moves all pieces: device(piece, slot) launches on `stream` and returns a
+// hipError_t, host(piece, slot) copies; up: host memory to the GPU.  events:
+// kStageSlots events of the caller, created here when null.
+template <typename Device, typename Host>
+hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream, hipEvent_t *events, Device &&device,
+                  Host &&host) {
+  size_t total = 0, largest = 0;
+  for (const Piece &p : pieces) {
+    const size_t b = (size_t)p.nc * p.nn * sizeof(double);
+    total += b;
+    largest = std::max(largest, b);
+  }
+  if (!total) return hipSuccess;
+  const int n = (int)pieces.size();
+  const int workers = (int)std::max<size_t>(1, std::min<size_t>(std::min(kStageSlots, n), total / kStageAlone));
+  const size_t slot = (largest + 255) & ~(size_t)255;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  Stage &s = stage();
+  std::lock_guard<std::mutex> lock(s.mu);
+  if (s.bytes < slot * workers) {
+    if (s.buf) (void)hipHostFree(s.buf);
+    s.buf = nullptr;
+    s.bytes = 0;
+    // small transfers share one slot, others get all of them
+    const size_t want = slot * workers <= kStageSlot ? kStageSlot : kStageSlot * kStageSlots;
+    e = hipHostMalloc((void **)&s.buf, want, hipHostMallocPortable);
+    if (e != hipSuccess) {
+      s.buf = nullptr;
+      return e;
+    }
+    s.bytes = want;
+  }
+  for (int w = 0; w < workers; w++)
+    if (!events[w] && (e = hipEventCreateWithFlags(&events[w], hipEventDisableTiming)) != hipSuccess) return e;
+  std::atomic<int> next{0}, bad{(int)hipSuccess};
+  auto work = [&](int w) {
+    hipError_t r = hipSetDevice(dev);
+    char *const at = s.buf + w * slot;
+    bool busy = false;
+    for (int c; r == hipSuccess && bad.load() == (int)hipSuccess && (c = next.fetch_add(1)) < n;) {
+      const Piece &p = pieces[c];
+      if (up) {
+        if (busy) r = hipEventSynchronize(events[w]);
+        if (r == hipSuccess) host(p, (double *)at);
+      }
+      if (r == hipSuccess) r = device(p, (double *)at);
+      if (r == hipSuccess) r = hipEventRecord(events[w], stream);
+      busy = r == hipSuccess;
+      if (!up) {
+        if (r == hipSuccess) r = hipEventSynchronize(events[w]);
+        busy = false;
+        if (r == hipSuccess) host(p, (double *)at);
+      }
+    }
+    if (r != hipSuccess) bad.store((int)r);
+  };
+  {
+    // joins on every way out of this block
+    struct Pool {
+      std::vector<std::thread> t;
+      ~Pool() {
+        for (auto &x : t) x.join();
+      }
+    } pool;
+    try {
+      pool.t.reserve(workers);
+      for (int w = 1; w < workers; w++) pool.t.emplace_back(work, w);
+    } catch (const std::exception &) {
+      // fewer threads: the others take their pieces
+    }
+    work(0);
+  }
+  // the slots are free again once the GPU has read them
+  e = hipStreamSynchronize(stream);
+  return bad.load() != (int)hipSuccess ? (hipError_t)bad.load() : e;
+}
+
+}  // namespace lbm
