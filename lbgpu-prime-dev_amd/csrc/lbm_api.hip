@@ -1443,19 +1443,25 @@ extern "C" int lbm_sample_macro(lbm_handle *h, int subs, int npts, const long *n
   if (need_lattice(h)) return 1;
   if (subs < 0 || subs >= h->p.nsubs) return lbm_fail("bad subs %d", subs);
   if (npts < 0 || (npts && (!nodes || !out))) return lbm_fail("bad sample arguments");
-  HIP_OK(hipStreamSynchronize(h->stream));
-  const int nf = h->nf, D = h->D;
-  const double *mv = h->mv + (long)subs * (1 + D) * nf;
-  for (int q = 0; q < npts; q++) {
+  const int nf = h->nf, comps = 1 + h->D;
+  const double *mv = h->mv + (long)subs * comps * nf;
+  for (int q = 0; q < npts; q++)
     if (nodes[q] < 0 || nodes[q] >= h->N) return lbm_fail("sample node %ld outside the lattice", nodes[q]);
-    const int x = h->fid[nodes[q]];
-    for (int c = 0; c <= D; c++) {
-      double *dst = out + (long)q * (1 + D) + c;
-      if (x < 0)
-        *dst = 0.0;
-      else
-        HIP_OK(hipMemcpy(dst, mv + (long)c * nf + x, sizeof(double), hipMemcpyDeviceToHost));
-    }
+  if (!npts) return sync(h);
+  Stage &st = stage();
+  std::lock_guard<std::mutex> lock(st.mu);
+  HIP_OK(stage_hold(st, kStageSlot));
+  // a slot holds the values of `most` points, then their compact indices
+  const int most = (int)(kStageSlot / (sizeof(double) * comps + sizeof(int)));
+  double *val = (double *)st.buf;
+  int *at = (int *)(val + (size_t)most * comps);
+  for (int q0 = 0; q0 < npts; q0 += most) {
+    const int n = std::min(most, npts - q0);
+    for (int q = 0; q < n; q++) at[q] = h->fid[nodes[q0 + q]];
+    hipLaunchKernelGGL(k_sample_field, dim3(blocks_for(n)), dim3(256), 0, h->stream, mv, nf, comps, at, n, val);
+    HIP_OK(hipGetLastError());
+    HIP_OK(hipStreamSynchronize(h->stream));
+    memcpy(out + (long)q0 * comps, val, (size_t)n * comps * sizeof(double));
   }
   return 0;
 }

@@ -31,6 +31,17 @@ __global__ void k_dense_field(Geo G, const double *src, int nf, int c0, long n0,
   host[(long)blockIdx.y * nn + t] = idx < 0 ? 0.0 : src[(long)(c0 + blockIdx.y) * nf + idx];
 }
 
+// fields at single nodes: out[q][c] = src[c][at[q]], 0 where at[q] < 0 (solid);
+// at and out are pinned host memory.  One launch and one wait, against a
+// copy of about 12 us for every value (48 points of three values: 1.72 ms ->
+// 14 us).
+__global__ void k_sample_field(const double *src, int nf, int comps, const int *at, int n, double *out) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const int idx = at[q];
+  for (int c = 0; c < comps; c++) out[(long)q * comps + c] = idx < 0 ? 0.0 : src[(long)c * nf + idx];
+}
+
 // populations of one subs: slots a0 + blockIdx.y; every element of out is
 // written (0 at a solid node), so nothing of an earlier call survives there
 template <int Q, int NS, typename ST, typename CT, int SUBS>

@@ -54,6 +54,20 @@ inline void stage_leave() {
   s.bytes = 0;
 }
 
+// at least `bytes` (up to all slots) of pinned memory; s.mu is held
+inline hipError_t stage_hold(Stage &s, size_t bytes) {
+  if (s.bytes >= bytes) return hipSuccess;
+  if (s.buf) (void)hipHostFree(s.buf);
+  s.buf = nullptr;
+  s.bytes = 0;
+  // small transfers share one slot, others get all of them
+  const size_t want = bytes <= kStageSlot ? kStageSlot : kStageSlot * kStageSlots;
+  const hipError_t e = hipHostMalloc((void **)&s.buf, want, hipHostMallocPortable);
+  if (e != hipSuccess) s.buf = nullptr;
+  else s.bytes = want;
+  return e;
+}
+
 // One piece of a transfer: nc components of nn nodes from node n0, at most a
 // slot's worth; host moves it between the slot and the caller's memory,
 // device (when there is device work) launches the kernel on the slot.
@@ -97,19 +111,7 @@ hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream,
   if (e != hipSuccess) return e;
   Stage &s = stage();
   std::lock_guard<std::mutex> lock(s.mu);
-  if (s.bytes < slot * workers) {
-    if (s.buf) (void)hipHostFree(s.buf);
-    s.buf = nullptr;
-    s.bytes = 0;
-    // small transfers share one slot, others get all of them
-    const size_t want = slot * workers <= kStageSlot ? kStageSlot : kStageSlot * kStageSlots;
-    e = hipHostMalloc((void **)&s.buf, want, hipHostMallocPortable);
-    if (e != hipSuccess) {
-      s.buf = nullptr;
-      return e;
-    }
-    s.bytes = want;
-  }
+  if ((e = stage_hold(s, slot * workers)) != hipSuccess) return e;
   for (int w = 0; w < workers; w++)
     if (!events[w] && (e = hipEventCreateWithFlags(&events[w], hipEventDisableTiming)) != hipSuccess) return e;
   std::atomic<int> next{0}, bad{(int)hipSuccess};

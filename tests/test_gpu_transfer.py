@@ -47,6 +47,24 @@ def test_dense_round_trip(shape, storage):
     g.close()
 
 
+@pytest.mark.parametrize("points", [1, 64, 65, 50_000, 90_000])
+def test_samples_equal_fields(points):
+    """k_sample_field: values at listed nodes (repeats and solid nodes among
+    them; more than one pinned slot holds) equal the downloaded fields"""
+    L = _pkg.load()
+    rng = np.random.default_rng(points)
+    _, g = lattice(L, (19, 23, 29), 0, rng)
+    for s in range(2):
+        g.set_mv(s, *rng.standard_normal((4, g.N)))
+    at = rng.integers(0, g.N, points)
+    for s in range(2):
+        assert np.array_equal(g.sample_mv(s, at), np.stack(g.mv(s), 1)[at])
+    with pytest.raises(L.LbmError, match="outside the lattice"):
+        g.sample_mv(0, [0, g.N])
+    assert g.sample_mv(0, []).shape == (0, 4)
+    g.close()
+
+
 def test_transfers_from_several_threads():
     L = _pkg.load()
     bad = []
