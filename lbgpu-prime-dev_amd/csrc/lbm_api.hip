@@ -118,6 +118,8 @@ struct lbm_handle {
     size_t lds = 0;
     int *gidx = nullptr, *cnt = nullptr;
     uint32_t *list = nullptr;
+    int2 *tab = nullptr;  // k_sweep2d: strips instead of tiles
+    SweepGeo S{};
     void *F2 = nullptr;
   } tile;
   bool off64 = false;    // 64-bit element offsets at every size (LBM_OFFSET64=1)
@@ -358,7 +360,7 @@ void drop_chunks(lbm_handle *h) {
 }
 
 void free_tiles(lbm_handle *h) {
-  void *ptrs[] = {h->tile.gidx, h->tile.cnt, h->tile.list, h->tile.F2};
+  void *ptrs[] = {h->tile.gidx, h->tile.cnt, h->tile.list, h->tile.tab, h->tile.F2};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   h->tile = {};
@@ -1165,20 +1167,30 @@ bool row_condition(const lbm_params &p, int side, int &kind, int &which) {
 
 template <int NS, bool SOL, bool WALSH>
 int tile_launch(lbm_handle *h, const TileArgs &B) {
-  const dim3 grid(8 * B.T.tiles8);
-  auto go = [&](auto *fn, int nt) -> int {
-    // every handle asks for the same limit, the CU's whole LDS
+  auto &t = h->tile;
+  // every handle asks for the same limit, the CU's whole LDS
+  auto limit = [&](const void *fn) -> int {
     constexpr int bit = 1 << ((NS - 1) * 4 + SOL * 2 + WALSH);
-    if (!(h->tile.lds_set & bit)) {
-      HIP_OK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, h->lds_cu));
-      h->tile.lds_set |= bit;
-    }
-    hipLaunchKernelGGL(fn, grid, dim3(nt), h->tile.lds, h->stream, B);
+    if (t.lds_set & bit) return 0;
+    HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, h->lds_cu));
+    t.lds_set |= bit;
+    return 0;
+  };
+  auto tiles = [&](auto *fn) -> int {
+    if (limit((const void *)fn)) return 1;
+    hipLaunchKernelGGL(fn, dim3(8 * B.T.tiles8), dim3(t.threads), t.lds, h->stream, B);
     HIP_OK(hipGetLastError());
     return 0;
   };
-  if (h->tile.threads == 512) return go(k_tile2d<NS, SOL, WALSH, 512>, 512);
-  return go(k_tile2d<NS, SOL, WALSH, 1024>, 1024);
+  if constexpr (NS == 2)
+    if (t.tab) {
+      if (limit((const void *)k_sweep2d<SOL, WALSH>)) return 1;
+      hipLaunchKernelGGL((k_sweep2d<SOL, WALSH>), dim3(8 * t.S.blocks8), dim3(kSweepBlock), t.lds, h->stream, B, t.S,
+                         (const int2 *)t.tab);
+      HIP_OK(hipGetLastError());
+      return 0;
+    }
+  return t.threads == 512 ? tiles(k_tile2d<NS, SOL, WALSH, 512>) : tiles(k_tile2d<NS, SOL, WALSH, 1024>);
 }
 
 // Steps per launch, core and threads of k_tile2d for the handle's lattice.
@@ -1245,11 +1257,48 @@ int plan_tiles(lbm_handle *h) {
     }
   }
   t.shrink = handed ? 3 : 2;
+  const size_t sb = (size_t)h->tiles * p.nsubs * h->Q * kTile * h->st_bytes;
+  const StepArgs<double, double> A = make_args<double, double>(h);
+  auto off = [&]() {  // no memory: the steps are launched one by one
+    (void)hipGetLastError();
+    free_tiles(h);
+    h->tile.state = -1;
+    return 0;
+  };
+  t.T.ni = ni;
+  t.T.nj = nj;
+  // Strips (k_sweep2d) for flow + solute lattices of many tiles per CU, us per
+  // step, tiles -> strips: 1000^2 19.8 -> 19.6, 1088 x 1224 30.0 -> 24.2,
+  // 2100 x 1900 84.6 -> 63.4, below that tiles are faster (600 x 500 7.1
+  // against 9.2: short strips repeat their pipeline's start too often).  Flow
+  // alone keeps tiles (1088 x 1224 13.8 against 17.2, 2100 x 1900 45.0 against
+  // 41.9).  Rows that hand values to a neighbour need the tiles' barrier.
+  if (two && !handed && h->N >= 4500L * h->cus) {
+    SweepGeo &S = t.S;
+    const size_t col = (size_t)kSweepRows * (72 * p.nsubs + 8) + 8 * kSweepEntries;
+    const int most = (int)std::min<size_t>(kSweepCols, h->lds_cu / col) - 2 * kSweepHalo;
+    if (most < kSweepHalo) return 0;
+    S.strips = (ni + most - 1) / most;
+    S.cw = (ni + S.strips - 1) / S.strips;
+    S.strips = (ni + S.cw - 1) / S.cw;
+    S.rw = S.cw + 2 * kSweepHalo;
+    S.pieces = std::max(1, h->cus / S.strips);
+    S.ch = (nj + S.pieces - 1) / S.pieces;
+    S.pieces = (nj + S.ch - 1) / S.ch;
+    S.blocks8 = (S.strips * S.pieces + 7) / 8;
+    t.lds = col * S.rw;
+    t.steps = kSweepSteps;
+    t.threads = kSweepBlock;
+    const long n = (long)S.strips * nj * S.rw;
+    if (hipMalloc(&t.tab, (size_t)n * sizeof(int2)) != hipSuccess || hipMalloc(&t.F2, sb) != hipSuccess) return off();
+    hipLaunchKernelGGL(k_sweep_build, dim3(blocks_for(n)), dim3(256), 0, h->stream, A.G, S, t.tab);
+    HIP_OK(hipGetLastError());
+    t.state = 1;
+    return 0;
+  }
   tile_shape(h, t.shrink, t.steps, t.T.cx, t.T.cy, t.threads);
   const int cx = t.T.cx, cy = t.T.cy;
   TileGeo &T = t.T;
-  T.ni = ni;
-  T.nj = nj;
   T.halo = t.shrink * t.steps / 2;
   T.tx = (ni + cx - 1) / cx;
   T.ty = (nj + cy - 1) / cy;
@@ -1263,17 +1312,11 @@ int plan_tiles(lbm_handle *h) {
   t.lds = (size_t)T.rn * (72 * p.nsubs + 4);
   if (T.rn > kTileRegion || t.lds > (size_t)h->lds_cu) return 0;
   const long n = (long)T.tx * T.ty;
-  const size_t sb = (size_t)h->tiles * p.nsubs * h->Q * kTile * h->st_bytes;
   if (hipMalloc(&t.gidx, (size_t)n * T.rn * sizeof(int)) != hipSuccess ||
       hipMalloc(&t.list, (size_t)n * T.rn * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&t.cnt, (size_t)n * (kTileHalo + 1) * sizeof(int)) != hipSuccess ||
-      hipMalloc(&t.F2, sb) != hipSuccess) {
-    (void)hipGetLastError();
-    free_tiles(h);
-    h->tile.state = -1;
-    return 0;
-  }
-  const StepArgs<double, double> A = make_args<double, double>(h);
+      hipMalloc(&t.F2, sb) != hipSuccess)
+    return off();
   hipLaunchKernelGGL(k_tile_build, dim3((unsigned)n), dim3(256), 0, h->stream, A.G, T, t.gidx, t.list, t.cnt);
   HIP_OK(hipGetLastError());
   t.state = 1;

@@ -161,27 +161,38 @@ __device__ __forceinline__ void tile_rows(const TileArgs &B, uint32_t e, int ste
   if (e & kTileSouth) side(false, 1, 3, 5, 7);
 }
 
-// the nine locations node n collides from: slot a of x - c_a (own slot
+// Where a node's populations lie in LDS: slot a of the node is element
+// a * plane + n0; the same column in the rows below and above is dm and dp
+// elements away (all but n0 the same for the whole wave).
+struct TileAt {
+  int plane, n0, dm, dp;
+};
+
+// the nine locations a node collides from: slot a of x - c_a (own slot
 // opp(a) when that node is solid) before an odd half-step, own slot opp(a)
-// before an even one; an odd half-step pushes f_a to location opp(a)
+// before an even one; an odd half-step pushes f_a to location opp(a).  The
+// two choices differ by a wave-uniform distance, added under the node's bit
+// (three integer operations a direction).
 template <bool ODD>
-__device__ __forceinline__ void tile_locs(const TileGeo &T, uint32_t e, int n, int (&loc)[9]) {
-  loc[0] = n;
+__device__ __forceinline__ void tile_locs(const TileAt &P, uint32_t e, int (&loc)[9]) {
+  loc[0] = P.n0;
 #pragma unroll
   for (int a = 1; a < 9; a++) {
-    const int own = OPP(a) * T.rn + n;
-    loc[a] = ODD && ((e >> (11 + a)) & 1u) ? a * T.rn + n - CX(a) - CY(a) * T.rx : own;
+    loc[a] = OPP(a) * P.plane + P.n0;
+    if (ODD) {
+      const int row = CY(a) == 0 ? 0 : (CY(a) > 0 ? P.dm : P.dp);
+      loc[a] += ((int)(e << (20 - a)) >> 31) & ((a - OPP(a)) * P.plane + row - CX(a));
+    }
   }
 }
 
-// one half-step of one region node; LAST: the result goes to the output
-// array, else back to LDS
+// one half-step of one node; LAST: the result goes to the output array (the
+// node's compact index is idx), else back to LDS; ns: partial bounce-back
 template <int NS, bool SOL, bool WALSH, bool ODD, bool LAST>
 __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<double, double> &A, tile_t<NS> *lds,
-                                          const int *g, uint32_t e, bool rows, int step) {
-  const int n = (int)(e & 4095u), rn = B.T.rn;
+                                          const TileAt &P, int idx, double ns, uint32_t e, bool rows, int step) {
   int loc[9];
-  tile_locs<ODD>(B.T, e, n, loc);
+  tile_locs<ODD>(P, e, loc);
   double f[9], gs[9], u[3];
 #pragma unroll
   for (int a = 0; a < 9; a++) {
@@ -197,11 +208,8 @@ __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<doub
       if constexpr (NS == 2 && !SOL && !LAST)
         if (s == 1) lds[loc[a]][NS - 1] = v;
     });
-  const int idx = (WALSH || LAST) ? g[n] : 0;
-  double ns = 0., kns = 1.;
   if constexpr (WALSH) {
-    ns = A.ns[idx];
-    kns = 1. - ns;
+    const double kns = 1. - ns;
     double fp[9], gp[9];
 #pragma unroll
     for (int a = 0; a < 9; a++) {
@@ -219,7 +227,7 @@ __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<doub
 #pragma unroll
   for (int a = 0; a < 9; a++) {
     // even: own slot a (a resting solute keeps its slot a, gathered as direction opp(a))
-    const int at = ODD ? loc[OPP(a)] : a * rn + n;
+    const int at = ODD ? loc[OPP(a)] : a * P.plane + P.n0;
     tile_t<NS> v;
     v[0] = f[a];
     if constexpr (NS == 2) v[NS - 1] = SOL ? gs[a] : gs[OPP(a)];
@@ -260,6 +268,10 @@ __global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
   StepArgs<double, double> A = B.A;
   A.write_mv = 0;
   int s = 0;
+  auto at = [&](uint32_t e) {
+    const int n = (int)(e & 4095u);
+    return TileAt{rn, n, -B.T.rx, B.T.rx};
+  };
   for (int k = 0; k < B.steps; k += 2) {
     if (handed) {
       // row values that go to a neighbour's input: stored before any node collides
@@ -269,7 +281,7 @@ __global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
         if (!(e & (kTileNorth | kTileSouth))) continue;
         const int n = (int)(e & 4095u);
         int loc[9];
-        tile_locs<true>(B.T, e, n, loc);
+        tile_locs<true>(at(e), e, loc);
         double f[9], gs[9];
 #pragma unroll
         for (int a = 0; a < 9; a++) {
@@ -284,20 +296,200 @@ __global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
       __syncthreads();
     }
     const int odd = cnt[s + B.shrink - 1];
-    for (int p = tid; p < odd; p += NT)
-      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, g, lst[p], rows && !handed, k);
+    for (int p = tid; p < odd; p += NT) {
+      const uint32_t e = lst[p];
+      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, at(e), 0, WALSH ? A.ns[g[e & 4095u]] : 0., e, rows && !handed, k);
+    }
     s += B.shrink;
     __syncthreads();
     if (k + 2 < B.steps) {
       const int even = cnt[s];
-      for (int p = tid; p < even; p += NT)
-        tile_node<NS, SOL, WALSH, false, false>(B, A, lds, g, lst[p], rows, k + 1);
+      for (int p = tid; p < even; p += NT) {
+        const uint32_t e = lst[p];
+        tile_node<NS, SOL, WALSH, false, false>(B, A, lds, at(e), 0, WALSH ? A.ns[g[e & 4095u]] : 0., e, rows, k + 1);
+      }
       __syncthreads();
     } else {
       A.write_mv = B.A.write_mv;
-      for (int p = tid; p < core; p += NT)
-        tile_node<NS, SOL, WALSH, false, true>(B, A, lds, g, lst[p], rows, k + 1);
+      for (int p = tid; p < core; p += NT) {
+        const uint32_t e = lst[p];
+        const int idx = g[e & 4095u];
+        tile_node<NS, SOL, WALSH, false, true>(B, A, lds, at(e), idx, WALSH ? A.ns[idx] : 0., e, rows, k + 1);
+      }
     }
+  }
+}
+
+// ---- large lattices: strips swept along y ----------------------------------
+//
+// A lattice of several tiles per CU spends most of a tile's time on loading
+// it, and 25 x 25 cores load 1.7 times their populations.  k_sweep2d gives a
+// workgroup a strip of columns and sweeps it along y: the rows enter LDS one
+// by one, and four stages follow each other two rows apart, so that one
+// iteration advances
+//   odd half-step 1 on row i, even 2 on row i - 2, odd 3 on row i - 4, even 4
+//   on row i - 6 (stored to the output array),
+// with one barrier.  An odd stage on row r touches rows r - 1 .. r + 1 and
+// needs them to have passed the stage before, which they have; the rows the
+// stages touch are disjoint.  Nine rows are live (i - 6 .. i + 1 and the row
+// i + 2 being filled).  Populations are loaded two iterations before they are
+// written to LDS and their indices two more, and the barrier orders LDS only,
+// so the loads stay in flight across it.  The halo is kSweepHalo columns on
+// either side and, once per strip piece, rows at either end.
+//
+// Measured (flow + solute, porosity 0.7, row conditions), us per step, tiles
+// -> strips: 1088 x 1224 30.0 -> 24.2, 2100 x 1900 84.6 -> 63.4.  An iteration
+// takes 1.7 us: 0.9 us without the collision (LDS traffic and latency of two
+// waves per SIMD, which is all that 160 KB of rows feed), 0.1 us of it waiting
+// for the global loads; solid columns leave 30 % of the lanes idle.
+constexpr int kSweepSteps = 4, kSweepHalo = 4, kSweepRows = 9;
+constexpr int kSweepEntries = 16;  // rows whose table entries are in LDS (i - 6 .. i + 4)
+
+struct SweepGeo {
+  int cw, strips;   // core columns of a strip
+  int rw;           // table row length cw + 2 kSweepHalo
+  int ch, pieces;   // rows of a piece, pieces of a strip
+  int blocks8;      // launched workgroups / 8
+};
+
+// tab[strip][row][column] = {compact index (-1 solid or past the strip),
+// entry bits of the node}
+__global__ __launch_bounds__(256) void k_sweep_build(Geo G, SweepGeo S, int2 *tab) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (long)S.strips * G.nj * S.rw) return;
+  const int x = (int)(t % S.rw), j = (int)(t / S.rw % G.nj), strip = (int)(t / S.rw / G.nj);
+  const int x0 = strip * S.cw, cw = G.ni - x0 < S.cw ? G.ni - x0 : S.cw;
+  int2 v = {-1, 0};
+  if (x < cw + 2 * kSweepHalo) {
+    int i = (x0 - kSweepHalo + x) % G.ni;
+    if (i < 0) i += G.ni;
+    v.x = rank_of(G, i, j);
+    uint32_t e = 0;
+#pragma unroll
+    for (int a = 1; a < 9; a++)
+      if (rank_of(G, wrap1(i - CX(a), G.ni), wrap1(j - CY(a), G.nj)) >= 0) e |= 1u << (11 + a);
+    if (j == G.nj - 1) e |= kTileNorth;
+    if (j == 0) e |= kTileSouth;
+    v.y = (int)e;
+  }
+  tab[t] = v;
+}
+
+// barrier that orders LDS accesses only
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// one thread per column and stage
+constexpr int kSweepCols = 128, kSweepBlock = 4 * kSweepCols;
+
+template <bool SOL, bool WALSH>
+__global__ __launch_bounds__(kSweepBlock) void k_sweep2d(TileArgs B, SweepGeo S, const int2 *tab) {
+  extern __shared__ __align__(16) char sweep_lds[];
+  constexpr int NS = 2, R = kSweepRows, H = kSweepHalo;
+  const int t = xcd_block(S.blocks8);
+  if (t >= S.strips * S.pieces) return;
+  const int strip = t % S.strips, piece = t / S.strips;
+  const int ni = B.T.ni, nj = B.T.nj;
+  const int cw = ni - strip * S.cw < S.cw ? ni - strip * S.cw : S.cw;
+  const int y0 = piece * S.ch, ch = nj - y0 < S.ch ? nj - y0 : S.ch;
+  const int rw = cw + 2 * H, stride = S.rw, plane = R * stride;
+  tile_t<NS> *lds = (tile_t<NS> *)sweep_lds;
+  int2 *ent = (int2 *)(lds + 9 * plane);
+  double *nsl = (double *)(ent + kSweepEntries * stride);
+  // a thread computes column n of one stage (a SIMD's two waves take an odd
+  // and an even stage); the threads of stages 0 to 2 also load column n of
+  // slots 3 stage .. 3 stage + 2.  Those of stage 3, which store the results,
+  // do not load: waiting for a load would wait for the stores before it.
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int stage = (wv & 3) ^ (wv >> 2);
+  const int n = ((int)threadIdx.x & 63) + 64 * (wv >> 2);
+  const bool rows = B.flow[0] || B.flow[1] || (NS == 2 && (B.grad[0] || B.grad[1]));
+  const bool last = stage == B.steps - 1;
+  const int first = last ? H : 1 + stage;  // distance from the strip's edge and ends
+  const bool on = stage < B.steps && n >= first && n < rw - first;
+  StepArgs<double, double> A = B.A;
+  A.write_mv = last ? B.A.write_mv : 0;
+
+  // row y0 - H + q has number q and lies in slot q % R; iteration k has stage
+  // 0 on number k + 1, with numbers k .. k + 2 in LDS
+  const int iters = ch + 2 * H - 2 + 2 * (B.steps - 1) - (H - 1), most = ch + 2 * H - 1;
+  auto compute = [&](int k, bool stores) __attribute__((always_inline)) {
+    const int c = k + 1 - 2 * stage;  // this stage's row number
+    if (!on || c < first || c > most - first) return;
+    const int s0 = c % R, sm = (c + R - 1) % R, sp = (c + 1) % R;
+    const int2 en = ent[(c & (kSweepEntries - 1)) * stride + n];
+    if (en.x < 0) return;
+    const TileAt P{plane, s0 * stride + n, (sm - s0) * stride, (sp - s0) * stride};
+    const double ns = WALSH ? nsl[s0 * stride + n] : 0.;
+    if (!stores && !(stage & 1))
+      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, P, en.x, ns, (uint32_t)en.y, rows, stage);
+    else if (stores || last) tile_node<NS, SOL, WALSH, false, true>(B, A, lds, P, en.x, ns, (uint32_t)en.y, rows, stage);
+    else tile_node<NS, SOL, WALSH, false, false>(B, A, lds, P, en.x, ns, (uint32_t)en.y, rows, stage);
+  };
+  if (stage == 3) {
+    lds_barrier();
+    for (int k = 0; k < iters; k++) {
+      compute(k, true);
+      lds_barrier();
+    }
+    return;
+  }
+
+  // loads are issued by every thread in every iteration (clamped, so that
+  // their number is known and only the oldest are waited for)
+  const int2 *mine = tab + (long)strip * nj * stride + (n < rw ? n : rw - 1);
+  auto entry = [&](int q) __attribute__((always_inline)) -> int2 {
+    int r = (y0 - H + (q < most ? q : most)) % nj;
+    r = r < 0 ? r + nj : r;
+    return mine[(long)r * stride];
+  };
+  struct Rows {
+    tile_t<NS> v[3];
+    double ns;
+  };
+  auto load = [&](Rows &q, int2 e, int number) __attribute__((always_inline)) {
+    if (stage == 0 && n < rw) ent[(number & (kSweepEntries - 1)) * stride + n] = e;
+    const uint32_t idx = e.x < 0 ? 0u : (uint32_t)e.x;
+    const double *p = B.A.F + (size_t)foff<9, NS>(0, 3 * stage, idx);
+#pragma unroll
+    for (int k = 0; k < 3; k++) q.v[k] = *(const tile_t<NS> *)(p + k * kTile * NS);
+    if (WALSH) q.ns = A.ns[idx];
+  };
+  auto fill = [&](const Rows &q, int number) __attribute__((always_inline)) {
+    if (number > most || n >= rw) return;
+    const int at = number % R * stride + n;
+#pragma unroll
+    for (int k = 0; k < 3; k++) lds[(3 * stage + k) * plane + at] = q.v[k];
+    if (WALSH && stage == 0) nsl[at] = q.ns;
+  };
+  Rows q0, q1;
+  {
+    const int2 e0 = entry(0), e1 = entry(1), e2 = entry(2);
+    Rows q2;
+    load(q0, e0, 0);
+    load(q1, e1, 1);
+    load(q2, e2, 2);
+    fill(q0, 0);
+    fill(q1, 1);
+    fill(q2, 2);
+  }
+  load(q0, entry(3), 3);
+  load(q1, entry(4), 4);
+  int2 e0 = entry(5), e1 = entry(6);
+  lds_barrier();
+  auto iterate = [&](int k, Rows &q, int2 &e) __attribute__((always_inline)) {
+    fill(q, k + 3);
+    load(q, e, k + 5);
+    e = entry(k + 7);
+    compute(k, false);
+    lds_barrier();
+  };
+  for (int k = 0; k < iters; k += 2) {
+    iterate(k, q0, e0);
+    if (k + 1 < iters) iterate(k + 1, q1, e1);
   }
 }
 
