@@ -39,20 +39,6 @@ struct AdjArgs {
                                // solute concentration per node); null on other steps
 };
 
-// slot offset a half-step reads for direction a (the pull) / writes (the push)
-template <bool ODD>
-__device__ __forceinline__ uint32_t pull_off(const int (&nb)[19], int s, int a, int idx) {
-  if (a == 0) return foff<19, 2>(s, 0, idx);
-  if (ODD) return nb[a] >= 0 ? foff<19, 2>(s, a, nb[a]) : foff<19, 2>(s, OPP(a), idx);
-  return foff<19, 2>(s, OPP(a), idx);
-}
-template <bool ODD>
-__device__ __forceinline__ uint32_t push_off(const int (&nb)[19], int s, int a, int idx) {
-  if (a == 0) return foff<19, 2>(s, 0, idx);
-  if (ODD) return nb[OPP(a)] >= 0 ? foff<19, 2>(s, OPP(a), nb[OPP(a)]) : foff<19, 2>(s, a, idx);
-  return foff<19, 2>(s, a, idx);
-}
-
 // Threads per workgroup of the adjoint step: one wave.  With one or two
 // waves per SIMD (the register counts below) a workgroup of four waves
 // holds its CU's slots until its slowest wave ends; one-wave workgroups are
@@ -89,11 +75,11 @@ struct AdjMoments {
 
 // the adjoint at the push positions (where the forward half-step wrote)
 template <bool ODD, bool OFF32>
-__device__ __forceinline__ void adj_load(const AdjArgs &J, const int (&nb)[19], int idx, double (&lam)[19],
+__device__ __forceinline__ void adj_load(const AdjArgs &J, const uint32_t (&loc)[19], double (&lam)[19],
                                          double (&mu)[19], AdjMoments &m) {
 #pragma unroll
   for (int a = 0; a < 19; a++) {
-    const pair_t<double> v = ld_stream<!ODD>((const pair_t<double> *)elem<OFF32>(J.L, push_off<ODD>(nb, 0, a, idx)));
+    const pair_t<double> v = ld_stream<!ODD>((const pair_t<double> *)at_loc<OFF32>(J.L, loc[OPP(a)]));
     lam[a] = v.x;
     mu[a] = v.y;
     const double wl = W<19>(a) * v.x, wm = W<19>(a) * v.y;
@@ -150,13 +136,13 @@ __device__ __forceinline__ void adj_state_arrays(AdjState &st, const double (&f)
 // leave the L2 to the adjoint's read-then-written lines (adjoint kernels of
 // a 128^3 sweep: 289 -> 286 ms with them in the odd step too).
 template <int A_, int END, bool ODD, bool OFF32>
-__device__ __forceinline__ void adj_state_stream(AdjState &st, const AdjArgs &J, const int (&nb)[19], int idx,
+__device__ __forceinline__ void adj_state_stream(AdjState &st, const AdjArgs &J, const uint32_t (&loc)[19],
                                                  const double (&lam)[19], const double (&mu)[19]) {
   if constexpr (A_ < END) {
     const pair_t<double> v =
-        ld_stream<true>((const pair_t<double> *)elem<OFF32>(J.A.F, pull_off<ODD>(nb, 0, A_, idx)));
+        ld_stream<true>((const pair_t<double> *)at_loc<OFF32>(J.A.F, loc[A_]));
     adj_state_add<A_>(st, v.x, v.y, lam[A_], mu[A_]);
-    adj_state_stream<A_ + 1, END, ODD, OFF32>(st, J, nb, idx, lam, mu);
+    adj_state_stream<A_ + 1, END, ODD, OFF32>(st, J, loc, lam, mu);
   }
 }
 
@@ -222,7 +208,7 @@ __device__ __forceinline__ void adj_new(const AdjArgs &J, const AdjOut &o, doubl
 
 template <int B_, bool ODD, bool OFF32>
 __device__ __forceinline__ void adj_store_all(const AdjArgs &J, const AdjOut &o, double seed, double oseed,
-                                              const int (&nb)[19], int idx, const double (&lam)[19],
+                                              const uint32_t (&loc)[19], const double (&lam)[19],
                                               const double (&mu)[19]) {
   if constexpr (B_ < 19) {
     double nl, nm;
@@ -230,8 +216,8 @@ __device__ __forceinline__ void adj_store_all(const AdjArgs &J, const AdjOut &o,
     pair_t<double> v;
     v.x = nl;
     v.y = nm;
-    st_stream<!ODD>((pair_t<double> *)elem<OFF32>(J.L, pull_off<ODD>(nb, 0, B_, idx)), v);
-    adj_store_all<B_ + 1, ODD, OFF32>(J, o, seed, oseed, nb, idx, lam, mu);
+    st_stream<!ODD>((pair_t<double> *)at_loc<OFF32>(J.L, loc[B_]), v);
+    adj_store_all<B_ + 1, ODD, OFF32>(J, o, seed, oseed, loc, lam, mu);
   }
 }
 
@@ -245,16 +231,24 @@ __device__ __forceinline__ void adj_new_all(const AdjArgs &J, const AdjOut &o, d
   }
 }
 
-template <bool ODD>
-__device__ __forceinline__ void adj_neighbours(const StepArgs<double, double> &A, int idx, int (&nb)[19], int &k) {
-  nb[0] = idx;
+template <bool ODD, bool OFF32>
+__device__ __forceinline__ void adj_locs(const StepArgs<double, double> &A, int idx, uint32_t (&loc)[19], int &k) {
+  constexpr uint32_t U = loc_unit<2, double, OFF32>();
   int i, j;
   coords<3>(A.G, (uint32_t)A.G.node[idx], i, j, k);
-  if (ODD) {
-    int r[18];
-    neighbors_rows<3>(A.G, i, j, k, r);
-#pragma unroll
-    for (int a = 1; a < 19; a++) nb[a] = r[a - 1];
+  if constexpr (ODD) odd_locs<19, U>(A.G, idx, i, j, k, loc);
+  else even_locs<19, U>(idx, loc);
+}
+
+// An even step's locations lie at constant distances from the node's own:
+// formed anew for each of its three passes over them (the empty asm keeps
+// the compiler from carrying all 19 through; 356 -> 212 bytes of spills per
+// lane, all in the face blocks).
+template <bool ODD, bool OFF32>
+__device__ __forceinline__ void adj_locs_again(int idx, uint32_t (&loc)[19]) {
+  if constexpr (!ODD) {
+    asm("" : "+v"(idx));
+    even_locs<19, loc_unit<2, double, OFF32>()>(idx, loc);
   }
 }
 
@@ -362,15 +356,17 @@ __device__ __forceinline__ void adj_face_block(const AdjArgs &J, long slot, int 
   if (t < nface) {
     const int idx = t < nlo ? t : A.zb.hi_begin + (t - nlo);
     const bool top = idx >= A.zb.hi_begin;
-    int nb[19], k;
-    adj_neighbours<ODD>(A, idx, nb, k);
+    uint32_t loc[19];
+    int k;
+    adj_locs<ODD, OFF32>(A, idx, loc, k);
     double lam[19], mu[19];
     AdjMoments m;
-    adj_load<ODD, OFF32>(J, nb, idx, lam, mu, m);
+    adj_load<ODD, OFF32>(J, loc, lam, mu, m);
     double f[19], g[19];
+    adj_locs_again<ODD, OFF32>(idx, loc);
 #pragma unroll
     for (int a = 0; a < 19; a++) {
-      const pair_t<double> v = *(const pair_t<double> *)elem<OFF32>(A.F, pull_off<ODD>(nb, 0, a, idx));
+      const pair_t<double> v = *(const pair_t<double> *)at_loc<OFF32>(A.F, loc[a]);
       f[a] = v.x;
       g[a] = v.y;
     }
@@ -380,6 +376,7 @@ __device__ __forceinline__ void adj_face_block(const AdjArgs &J, long slot, int 
     const AdjOut o = adj_collide(J, m, st);
     double lb[19], mb[19];
     adj_new_all<0>(J, o, k == J.zf ? J.seed : 0.0, J.obs ? J.obs[idx] : 0.0, lam, mu, lb, mb);
+    adj_locs_again<ODD, OFF32>(idx, loc);
     // the adjoint runs with pressure on both faces (or none) and a
     // Dirichlet inlet with a zero-gradient outlet (or none)
     if (A.zb.flow[0] != kZNone) adj_zface_flow(top, lb);
@@ -392,7 +389,7 @@ __device__ __forceinline__ void adj_face_block(const AdjArgs &J, long slot, int 
       pair_t<double> v;
       v.x = lb[b];
       v.y = mb[b];
-      *(pair_t<double> *)elem<OFF32>(J.L, pull_off<ODD>(nb, 0, b, idx)) = v;
+      *(pair_t<double> *)at_loc<OFF32>(J.L, loc[b]) = v;
     }
 #pragma unroll
     for (int q = 0; q < 5; q++) acc[q] = o.acc[q];
@@ -419,15 +416,18 @@ void k_adjoint_step(AdjArgs J, int nfb) {
   const int idx = lb * kAdjBlock + (int)threadIdx.x;
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (idx < J.A.nf && !zface_node<19>(J.A, idx)) {
-    int nb[19], k;
-    adj_neighbours<ODD>(J.A, idx, nb, k);
+    uint32_t loc[19];
+    int k;
+    adj_locs<ODD, OFF32>(J.A, idx, loc, k);
     double lam[19], mu[19];
     AdjMoments m;
-    adj_load<ODD, OFF32>(J, nb, idx, lam, mu, m);
+    adj_load<ODD, OFF32>(J, loc, lam, mu, m);
     AdjState st;
-    adj_state_stream<0, 19, ODD, OFF32>(st, J, nb, idx, lam, mu);
+    adj_locs_again<ODD, OFF32>(idx, loc);
+    adj_state_stream<0, 19, ODD, OFF32>(st, J, loc, lam, mu);
     const AdjOut o = adj_collide(J, m, st);
-    adj_store_all<0, ODD, OFF32>(J, o, k == J.zf ? J.seed : 0.0, J.obs ? J.obs[idx] : 0.0, nb, idx, lam, mu);
+    adj_locs_again<ODD, OFF32>(idx, loc);
+    adj_store_all<0, ODD, OFF32>(J, o, k == J.zf ? J.seed : 0.0, J.obs ? J.obs[idx] : 0.0, loc, lam, mu);
 #pragma unroll
     for (int q = 0; q < 5; q++) acc[q] = o.acc[q];
   }
@@ -448,9 +448,11 @@ __device__ __forceinline__ void adj_face(double *L, const int (&nb)[19], int s, 
                                         double &dcb) {
   constexpr int UP[5] = {9, 11, 13, 15, 17};
   constexpr int DN[5] = {10, 12, 14, 16, 18};
+  // element of the pull of each direction
   uint32_t loc[19];
 #pragma unroll
-  for (int a = 0; a < 19; a++) loc[a] = pull_off<ODD>(nb, s, a, idx);
+  for (int a = 0; a < 19; a++)
+    loc[a] = ODD && a && nb[a] >= 0 ? foff<19, 2>(s, a, nb[a]) : foff<19, 2>(s, OPP(a), idx);
   double lu[5], dl[19];
 #pragma unroll
   for (int a = 0; a < 19; a++) dl[a] = 0.0;

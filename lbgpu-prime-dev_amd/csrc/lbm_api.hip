@@ -489,16 +489,11 @@ int upload_band_map(lbm_handle *h, int bs, long nb, long per, int **dst) {
   return 0;
 }
 
-// the odd half-step's workgroup size for the handle's kind, and the LDS a
-// half-step workgroup reserves
+// the odd half-step's workgroup size for the handle's kind
 int odd_block(const lbm_handle *h) {
   return dispatch(h, [&]<int Q, int NS, typename ST, typename CT>() -> int {
-    return StepShape<true, NS, ST, CT>::block;
+    return step_shape<NS, ST, CT>(true, h->nf).block;
   });
-}
-template <bool ODD, int NS, typename ST, typename CT>
-size_t step_pad(const lbm_handle *h) {
-  return step_lds_pad(StepShape<ODD, NS, ST, CT>::per_cu, h->lds_cu);
 }
 
 // The 3-D lattice's block maps.  Odd half-step (blocks of odd_block()):
@@ -514,7 +509,7 @@ int build_band_maps(lbm_handle *h) {
   // the odd step's node block for this kind
   const int bso = odd_block(h);
   const long nbo = blocks_for(h->nf, bso);
-  if ((double)h->nf / h->p.nk / 8.0 >= 3.0 * kBlockOdd) {
+  if ((double)h->nf / h->p.nk / 8.0 >= 3.0 * 512) {
     const long per = (nbo + 7) / 8;
     if (int rc = upload_band_map(h, bso, nbo, per, &h->bmap)) return rc;
     h->bmap8 = (int)per;
@@ -544,10 +539,11 @@ int launch_half(lbm_handle *h, int odd, int t, int write_mv, bool fuse_bc = fals
     A.solute_on = NS == 2 && t >= h->p.sigma_t_on && t <= h->p.sigma_t_off;
     Prof pr(h, odd ? 0 : 1);
     const bool off32 = !h->off64 && (size_t)h->tiles * NS * Q * kTile * sizeof(ST) <= 0xffffffffull;
-    const int bs = odd ? half_step_block<true, NS, ST, CT>() : half_step_block<false, NS, ST, CT>();
+    const StepShape shape = step_shape<NS, ST, CT>(odd, h->nf);
+    const int bs = shape.block;
     A.nblk8 = (int)((blocks_for(h->nf, bs) + 7) / 8);
     const dim3 grid = odd ? odd_grid(h, A, bs) : dim3(8 * A.nblk8), block(bs);
-    const size_t lds = odd ? step_pad<true, NS, ST, CT>(h) : step_pad<false, NS, ST, CT>(h);
+    const size_t lds = step_lds_pad(shape.per_cu, h->lds_cu);
     if (h->ns) {
       // Walsh partial bounce-back
       A.ns = h->ns;
@@ -2079,8 +2075,9 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
       if (fz) set_zb(h, A);
       A.Fo = (double *)rp[q];
       A.solute_on = 1;
-      const int bs = (t & 1) ? half_step_block<true, 2, double, double>() : half_step_block<false, 2, double, double>();
-      const size_t lds = (t & 1) ? step_pad<true, 2, double, double>(h) : step_pad<false, 2, double, double>(h);
+      const StepShape shape = step_shape<2, double, double>(t & 1, h->nf);
+      const int bs = shape.block;
+      const size_t lds = step_lds_pad(shape.per_cu, h->lds_cu);
       A.nblk8 = (int)((blocks_for(h->nf, bs) + 7) / 8);
       const dim3 grid = (t & 1) ? odd_grid(h, A, bs) : dim3(8 * A.nblk8), block(bs);
       Prof pr(h, (t & 1) ? 0 : 1);

@@ -27,52 +27,43 @@
 namespace lbm {
 
 constexpr int kBlock = 256;
-// Workgroup size of the odd (pull/push) half-step of the kinds that run at
-// full occupancy (FP64 flow, FP32 storage with the FP32 collision): 8-wave
-// workgroups keep more of its 19 gathers per node in flight on a CU (flow
-// FP64 at 256^3, porosity 0.40: 0.437 ms at 512 threads against 0.457 ms at
-// 256 and 0.491 ms at 1024, contiguous block order).  FP16 storage runs 256
-// threads in the row-band order with 256-node blocks (0.242 against 0.267 ms
-// at 256^3 in the contiguous order; 512 threads gained 4 % at 256^3 but lost
-// 4 % at 192^3).  StepShape below gives every kind's shape.
-constexpr int kBlockOdd = 512;
-// Launch shape of a half-step kernel instantiation: threads per workgroup,
-// and the number of its workgroups one CU may hold (0: as many as the
-// registers allow; otherwise each workgroup reserves LDS it does not use,
-// lds_per_cu / (per_cu + 1/2) rounded down, so that no more fit).
+// Launch shape of a half-step: threads per workgroup, and the number of its
+// workgroups one CU may hold (0: as many as the registers allow; otherwise
+// each workgroup reserves LDS it does not use, lds_per_cu / (per_cu + 1/2)
+// rounded down, so that no more fit).
+//
 // With FP64 storage and collision the half-steps run at low occupancy in
 // small workgroups: fewer requests in flight per XCD let its L2 serve the
 // lines that neighbouring waves share (and the read-then-write of each line)
 // before they leave it, and small workgroups retire wave by wave instead of
-// waiting for their slowest wave.  Measured at 256^3 (porosity 0.40, odd
-// step in the row-band order), odd / even half-step:
-//   flow + solute: odd in one-wave workgroups, at most 6 per CU (1.5 waves
-//   per SIMD): 0.793 ms against 0.830 with 512 threads (two waves per SIMD,
-//   registers allow no more), 0.841 with 256 (three per SIMD), 0.806 / 0.833
-//   / 0.814 with at most 8 / 4 / 10 one-wave workgroups; even in two-wave
-//   workgroups, at most 2 per CU (one wave per SIMD): 0.642 ms against 0.666
-//   with 256 threads uncapped, 0.648 with one-wave workgroups at most 3-6
-//   per CU, 0.659 with 256 threads at most 2-3 per CU;
-//   flow: odd stays at 512 threads uncapped (0.395 ms; capped or smaller,
-//   0.42-0.54); even in two-wave workgroups at most 3 per CU: 0.328 against
-//   0.338 ms.
-// FP32 storage with the FP64 collision (flow + solute; 141 / 178 registers:
-// at most three / two waves per SIMD) takes the small workgroups without a
-// cap: odd in one-wave workgroups 0.420 ms against 0.441 with 512 threads,
-// even in two-wave workgroups 0.307 against 0.331 with 256 (capped at 1.5
-// or 1 wave per SIMD both were slower: 0.46-0.70 / 0.32-0.36 ms).
-// FP32 storage with the FP32 collision and FP16 storage keep 512 / 256
-// threads uncapped: smaller workgroups or caps made them 1-70 % slower.
-template <bool ODD, int NS, typename ST, typename CT>
+// waiting for their slowest wave.  A lattice that gives a CU few waves (below
+// kFewNodes fluid nodes) is bound by latency and by the last workgroups
+// instead: it runs one-wave workgroups with every odd-step wave resident.
+// Measured, us per step (odd and even averaged; sphere packs of 38k, 157k,
+// 913k, 3.2M and 7.0M fluid nodes; former shapes -> these):
+//   flow FP64        6.0 11.2 48.7 164.4 347.1 -> 4.8 9.6 47.8 162.3 346.9
+//     (odd 512 threads, even 128 capped at 3 -> 256 capped at 3, 128 at 3)
+//   flow + solute    6.5 19.4 89.8 326.3 713.7 -> 6.3 18.5 same (64 at 6, 128 at 2)
+//   FP32             6.2 12.0 49.4 165.3 353.6 -> 5.4 10.0 48.7 163.5 352.5
+//     (512, 256 -> 256, 128 capped at 4)
+//   FP32, FP64 collision  5.9 10.7 49.3 165.4 356.1 -> 5.6 10.3 same (64, 128)
+// FP16 storage keeps 256 threads uncapped: 64 and 128 threads measured within
+// 1 % below 3.2M nodes and 2-4 % slower at 7.0M, caps 3-70 % slower.
+constexpr int kFewNodes = 1 << 18;
+constexpr int kStepBlock = 256;  // largest workgroup of a half-step
 struct StepShape {
-  static constexpr bool f64 = sizeof(ST) == 8 && sizeof(CT) == 8;
-  static constexpr bool f32_f64 = NS == 2 && sizeof(ST) == 4 && sizeof(CT) == 8;
-  static constexpr int block = ODD ? (NS == 2 && (f64 || f32_f64) ? 64 : (sizeof(ST) >= 4 ? kBlockOdd : kBlock))
-                                   : (f64 || f32_f64 ? 128 : kBlock);
-  static constexpr int per_cu = !f64 ? 0 : (ODD ? (NS == 2 ? 6 : 0) : (NS == 2 ? 2 : 3));
+  int block, per_cu;
 };
-template <bool ODD, int NS, typename ST, typename CT>
-constexpr int half_step_block() { return StepShape<ODD, NS, ST, CT>::block; }
+template <int NS, typename ST, typename CT>
+StepShape step_shape(bool odd, int nf) {
+  constexpr bool f64 = sizeof(ST) == 8 && sizeof(CT) == 8, f32_f64 = NS == 2 && sizeof(ST) == 4 && sizeof(CT) == 8;
+  if (sizeof(ST) == 2) return {256, 0};
+  if (nf < kFewNodes) return {64, f64 && !odd ? 6 : 0};
+  if (f64 && NS == 2) return odd ? StepShape{64, 6} : StepShape{128, 2};
+  if (f64) return odd ? StepShape{256, 3} : StepShape{128, 3};
+  if (f32_f64) return odd ? StepShape{64, 0} : StepShape{128, 0};
+  return odd ? StepShape{256, 0} : StepShape{128, 4};
+}
 // LDS a half-step workgroup reserves to cap the workgroups per CU
 inline size_t step_lds_pad(int per_cu, int lds_per_cu) {
   if (per_cu <= 0 || lds_per_cu <= 0) return 0;
@@ -123,14 +114,10 @@ struct Codec<double, float> {
   static __device__ __forceinline__ double enc(float v, float, float) { return (double)v; }
 };
 
-// Population element e of the tile array.  OFF32: the array is smaller
-// than 4 GiB, so the byte offset is a 32-bit value added to the uniform
-// base (saddr + voffset addressing, half the address registers).
-template <bool OFF32, typename T>
-__device__ __forceinline__ T *elem(T *F, uint32_t e) {
-  if (OFF32) return (T *)((char *)F + (uint32_t)(e * (uint32_t)sizeof(T)));
-  return F + e;
-}
+// Locations are 32-bit.  OFF32: the array is smaller than 4 GiB, so a location
+// is a byte offset added to the uniform base (saddr + voffset addressing,
+// half the address registers); otherwise it counts elements.
+//
 // Loads and stores of populations.  The even half-step streams whole
 // tiles and uses non-temporal accesses; the odd half-step's gathers and
 // scatters share partial lines between neighbouring waves, which must stay
@@ -209,22 +196,61 @@ __device__ __forceinline__ void neighbors(const Geo &G, int x, int (&nb)[Q]) {
   for (int a = 1; a < Q; a++) nb[a] = r[a - 1];
 }
 
-// Gather the Q populations one half-step collides.
-template <int Q, int NS, typename ST, typename CT, int SUBS, bool ODD, bool OFF32 = false>
-__device__ __forceinline__ void gather(const StepArgs<ST, CT> &A, int idx, const int (&nb)[Q],
-                                       CT (&f)[Q]) {
+// The locations one half-step collides from, loc[a] for direction a: before
+// an odd one slot a of x - c_a, or the own slot opp(a) when that node is
+// solid; before an even one the own slot opp(a).  The half-step stores f_a at
+// loc[opp(a)], so one set of offsets serves its loads and its stores.  Units:
+// bytes from the array's start (OFF32) or elements.
+template <int NS, typename ST, bool OFF32>
+__host__ __device__ constexpr uint32_t loc_unit() {
+  return OFF32 ? NS * sizeof(ST) : NS;
+}
+
+template <int Q, uint32_t U>
+__device__ __forceinline__ void even_locs(int x, uint32_t (&loc)[Q]) {
 #pragma unroll
-  for (int a = 0; a < Q; a++) {
-    uint32_t off;
-    if (a == 0)
-      off = foff<Q, NS>(SUBS, 0, idx);
-    else if (ODD)
-      off = nb[a] >= 0 ? foff<Q, NS>(SUBS, a, nb[a]) : foff<Q, NS>(SUBS, OPP(a), idx);
-    else
-      off = foff<Q, NS>(SUBS, OPP(a), idx);
-    f[a] = Codec<ST, CT>::dec(ld_stream<!ODD>(elem<OFF32>(A.F, off)),
-                              A.inv_scale[SUBS], shift_of<Q, ST, CT, SUBS>(A, a));
+  for (int a = 0; a < Q; a++) loc[a] = loc_at<Q, U>(OPP(a), (uint32_t)x);
+}
+
+template <int Q, uint32_t U>
+__device__ __forceinline__ void odd_locs(const Geo &G, int x, int i, int j, int k, uint32_t (&loc)[Q]) {
+  int rank[Q - 1];
+  bool fluid[Q - 1];
+  neighbors_core<Q == 9 ? 2 : 3>(G, i, j, k, rank, fluid);
+  loc[0] = loc_at<Q, U>(0, (uint32_t)x);
+#pragma unroll
+  for (int a = 1; a < Q; a++) {
+    const uint32_t nb = loc_at<Q, U>(a, (uint32_t)rank[a - 1]);
+    const uint32_t own = loc[0] + (uint32_t)OPP(a) * (kTile * U);
+    loc[a] = fluid[a - 1] ? nb : own;
   }
+}
+
+template <int Q, uint32_t U, bool ODD>
+__device__ __forceinline__ void step_locs(const Geo &G, int x, uint32_t (&loc)[Q]) {
+  if constexpr (ODD) {
+    int i, j, k;
+    coords<Q == 9 ? 2 : 3>(G, (uint32_t)G.node[x], i, j, k);
+    odd_locs<Q, U>(G, x, i, j, k, loc);
+  } else {
+    even_locs<Q, U>(x, loc);
+  }
+}
+
+// the population of component s at a location
+template <bool OFF32, typename T>
+__device__ __forceinline__ T *at_loc(T *F, uint32_t loc, int s = 0) {
+  if (OFF32) return (T *)((char *)F + (uint32_t)(loc + (uint32_t)(s * sizeof(T))));
+  return F + loc + s;
+}
+
+// Gather the Q populations one half-step collides.
+template <int Q, typename ST, typename CT, int SUBS, bool ODD, bool OFF32>
+__device__ __forceinline__ void gather(const StepArgs<ST, CT> &A, const uint32_t (&loc)[Q], CT (&f)[Q]) {
+#pragma unroll
+  for (int a = 0; a < Q; a++)
+    f[a] = Codec<ST, CT>::dec(ld_stream<!ODD>(at_loc<OFF32>(A.F, loc[a], SUBS)), A.inv_scale[SUBS],
+                              shift_of<Q, ST, CT, SUBS>(A, a));
 }
 
 // ---- FP16 stores with stochastic rounding ----------------------------------
@@ -281,30 +307,23 @@ __device__ __forceinline__ _Float16 sr_one(float x, uint32_t r) {
   return v.x;
 }
 
-template <int Q, int NS, typename ST, typename CT, int SUBS, bool ODD, bool OFF32 = false>
-__device__ __forceinline__ void scatter(const StepArgs<ST, CT> &A, int idx, const int (&nb)[Q],
+template <int Q, typename ST, typename CT, int SUBS, bool ODD, bool OFF32>
+__device__ __forceinline__ void scatter(const StepArgs<ST, CT> &A, int idx, const uint32_t (&loc)[Q],
                                         const CT (&f)[Q]) {
   [[maybe_unused]] uint32_t seed = 0;
   if constexpr (sizeof(ST) == 2) seed = sr_seed(idx, (float)f[0], (float)f[1]);
 #pragma unroll
   for (int a = 0; a < Q; a++) {
     [[maybe_unused]] constexpr int kPartner[19] = {1, 2, 1, 4, 3, 6, 5, 8, 7, 10, 9, 12, 11, 14, 13, 16, 15, 18, 17};
-    uint32_t off;
-    if (a == 0)
-      off = foff<Q, NS>(SUBS, 0, idx);
-    else if (ODD)
-      off = nb[OPP(a)] >= 0 ? foff<Q, NS>(SUBS, OPP(a), nb[OPP(a)]) : foff<Q, NS>(SUBS, a, idx);
-    else
-      off = foff<Q, NS>(SUBS, a, idx);
+    ST *const to = at_loc<OFF32>(A.Fo, loc[OPP(a)], SUBS);
     if constexpr (sizeof(ST) == 2) {
       // the partner's value: another slot of the node (its opposite)
       const int b = kPartner[a];
       const float y = (float)((f[a] - shift_of<Q, ST, CT, SUBS>(A, a)) * A.scale[SUBS]);
       const float yb = (float)((f[b] - shift_of<Q, ST, CT, SUBS>(A, b)) * A.scale[SUBS]);
-      st_stream<!ODD>(elem<OFF32>(A.Fo, off), (ST)sr_one(y, sr_rand(yb, seed)));
+      st_stream<!ODD>(to, (ST)sr_one(y, sr_rand(yb, seed)));
     } else {
-      st_stream<!ODD>(
-          elem<OFF32>(A.Fo, off), Codec<ST, CT>::enc(f[a], A.scale[SUBS], shift_of<Q, ST, CT, SUBS>(A, a)));
+      st_stream<!ODD>(to, Codec<ST, CT>::enc(f[a], A.scale[SUBS], shift_of<Q, ST, CT, SUBS>(A, a)));
     }
   }
 }
@@ -316,37 +335,22 @@ using pair_t = ST __attribute__((ext_vector_type(2)));
 
 // NT: streaming loads also in the odd half-step (out-of-place steps)
 template <int Q, typename ST, typename CT, bool ODD, bool OFF32, bool NT = false>
-__device__ __forceinline__ void gather2(const StepArgs<ST, CT> &A, int idx, const int (&nb)[Q], CT (&f)[Q],
-                                        CT (&g)[Q]) {
+__device__ __forceinline__ void gather2(const StepArgs<ST, CT> &A, const uint32_t (&loc)[Q], CT (&f)[Q], CT (&g)[Q]) {
 #pragma unroll
   for (int a = 0; a < Q; a++) {
-    uint32_t off;
-    if (a == 0)
-      off = foff<Q, 2>(0, 0, idx);
-    else if (ODD)
-      off = nb[a] >= 0 ? foff<Q, 2>(0, a, nb[a]) : foff<Q, 2>(0, OPP(a), idx);
-    else
-      off = foff<Q, 2>(0, OPP(a), idx);
-    const pair_t<ST> v = ld_stream<!ODD || NT>((const pair_t<ST> *)elem<OFF32>(A.F, off));
+    const pair_t<ST> v = ld_stream<!ODD || NT>((const pair_t<ST> *)at_loc<OFF32>(A.F, loc[a]));
     f[a] = Codec<ST, CT>::dec(v.x, A.inv_scale[0], (CT)0);
     g[a] = Codec<ST, CT>::dec(v.y, A.inv_scale[1], shift_of<Q, ST, CT, 1>(A, a));
   }
 }
 
 template <int Q, typename ST, typename CT, bool ODD, bool OFF32>
-__device__ __forceinline__ void scatter2(const StepArgs<ST, CT> &A, int idx, const int (&nb)[Q],
+__device__ __forceinline__ void scatter2(const StepArgs<ST, CT> &A, int idx, const uint32_t (&loc)[Q],
                                          const CT (&f)[Q], const CT (&g)[Q]) {
   [[maybe_unused]] uint32_t seed = 0;
   if constexpr (sizeof(ST) == 2) seed = sr_seed(idx, (float)f[0], (float)g[0]);
 #pragma unroll
   for (int a = 0; a < Q; a++) {
-    uint32_t off;
-    if (a == 0)
-      off = foff<Q, 2>(0, 0, idx);
-    else if (ODD)
-      off = nb[OPP(a)] >= 0 ? foff<Q, 2>(0, OPP(a), nb[OPP(a)]) : foff<Q, 2>(0, a, idx);
-    else
-      off = foff<Q, 2>(0, a, idx);
     pair_t<ST> v;
     if constexpr (sizeof(ST) == 2) {
       const half2_sr h = sr_pair((float)(f[a] * A.scale[0]),
@@ -357,7 +361,7 @@ __device__ __forceinline__ void scatter2(const StepArgs<ST, CT> &A, int idx, con
       v.x = Codec<ST, CT>::enc(f[a], A.scale[0], (CT)0);
       v.y = Codec<ST, CT>::enc(g[a], A.scale[1], shift_of<Q, ST, CT, 1>(A, a));
     }
-    st_stream<!ODD>((pair_t<ST> *)elem<OFF32>(A.Fo, off), v);
+    st_stream<!ODD>((pair_t<ST> *)at_loc<OFF32>(A.Fo, loc[OPP(a)]), v);
   }
 }
 
@@ -388,13 +392,14 @@ __device__ __forceinline__ CT cdotu(CT u0, CT u1, CT u2) {
 // WALSH: partial bounce-back (src/k_stream_collide_stream.c:129-135,183-192,
 // src/lattice.c:2936-2939): the momentum and the force enter u scaled by
 // kns = 1 - ns; the caller mixes the opposite pre-collision populations in.
-// LEAN (FP64): the same values in fewer operations, for kernels that the
-// FP64 units bound.  The products by the velocity components 0 and +-1 are
-// exact, so skipping them changes no finite result; 0 * rho, added to each
-// momentum sum, keeps what they did to others (one infinite or NaN population
-// makes all of u NaN); x / 1 is x; and an opposite direction's 3 v and
-// 4.5 v v are the direction's own, negated and unchanged.
-template <int Q, typename ST, typename CT, int SUBS, bool ODD, bool WALSH = false, bool LEAN = false>
+// The values are those of the written order in fewer operations.  The
+// products by the velocity components 0 and +-1 are exact, so skipping them
+// changes no finite result; 0 * rho, added to each momentum sum in FP64, keeps
+// what they did to others (one infinite or NaN population makes all of u NaN);
+// x / 1 is x; and an opposite direction's 3 v and 4.5 v v are the direction's
+// own, negated and unchanged.  (FP64 against the products written out: 2-D
+// tiles 8-10 % faster, 3-D steps 2-5 % below 10^6 nodes, 0-1 % above.)
+template <int Q, typename ST, typename CT, int SUBS, bool ODD, bool WALSH = false>
 __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (&f)[Q], CT (&u)[3],
                                         CT kns = (CT)1) {
   constexpr int D = Q == 9 ? 2 : 3;
@@ -407,52 +412,33 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
     u[0] = (CT)0;
     u[1] = (CT)0;
     u[2] = (CT)0;
-    if constexpr (sizeof(CT) == 4) {
-      // FP32 collision: the zero terms skipped (same values; 16 % fewer
-      // instructions: FP16 odd step 3 % faster)
-      [&]<int... A>(std::integer_sequence<int, A...>) {
-        ((u[0] = add_c<CX(A), CT>(u[0], f[A]), u[1] = add_c<CY(A), CT>(u[1], f[A]),
-          u[2] = D == 3 ? add_c<CZ(A), CT>(u[2], f[A]) : u[2]),
-         ...);
-      }(std::make_integer_sequence<int, Q>{});
-    } else if constexpr (LEAN) {
-      [&]<int... A>(std::integer_sequence<int, A...>) {
-        ((u[0] = add_c<CX(A), CT>(u[0], f[A]), u[1] = add_c<CY(A), CT>(u[1], f[A]),
-          u[2] = D == 3 ? add_c<CZ(A), CT>(u[2], f[A]) : u[2]),
-         ...);
-      }(std::make_integer_sequence<int, Q>{});
+    [&]<int... A>(std::integer_sequence<int, A...>) {
+      ((u[0] = add_c<CX(A), CT>(u[0], f[A]), u[1] = add_c<CY(A), CT>(u[1], f[A]),
+        u[2] = D == 3 ? add_c<CZ(A), CT>(u[2], f[A]) : u[2]),
+       ...);
+    }(std::make_integer_sequence<int, Q>{});
+    if constexpr (sizeof(CT) == 8) {
       const CT z = (CT)0 * rho;
 #pragma unroll
       for (int d = 0; d < D; d++) u[d] += z;
-    } else {
-      // FP64: as written (the skipped form frees registers, and the flow +
-      // solute odd step's second workgroup per CU then slows it by 5 % at
-      // 256^3)
-#pragma unroll
-      for (int a = 0; a < Q; a++) {
-        u[0] += ((CT)CX(a)) * f[a];
-        u[1] += ((CT)CY(a)) * f[a];
-        if (D == 3) u[2] += ((CT)CZ(a)) * f[a];
-      }
     }
     if constexpr (sizeof(CT) == 4 && sizeof(ST) >= 4) {
 #pragma unroll
       for (int d = 0; d < D; d++) jpre[d] = u[d];
     }
   } else if constexpr (sizeof(CT) == 4 && sizeof(ST) >= 4) {
-#pragma unroll
-    for (int a = 1; a < Q; a++) {
-      jpre[0] += ((CT)CX(a)) * f[a];
-      jpre[1] += ((CT)CY(a)) * f[a];
-      if (D == 3) jpre[2] += ((CT)CZ(a)) * f[a];
-    }
+    [&]<int... A>(std::integer_sequence<int, A...>) {
+      ((jpre[0] = add_c<CX(A), CT>(jpre[0], f[A]), jpre[1] = add_c<CY(A), CT>(jpre[1], f[A]),
+        jpre[2] = D == 3 ? add_c<CZ(A), CT>(jpre[2], f[A]) : jpre[2]),
+       ...);
+    }(std::make_integer_sequence<int, Q>{});
   }
   if (SUBS == 0) {
     if constexpr (WALSH) {
 #pragma unroll
       for (int d = 0; d < D; d++) u[d] *= kns;
     }
-    if (!LEAN || A.rhoA != (CT)1) {
+    if (A.rhoA != (CT)1) {
 #pragma unroll
       for (int d = 0; d < D; d++) u[d] /= A.rhoA;
     }
@@ -490,17 +476,9 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
   }
   const CT it = SUBS == 0 ? A.inv_tau : A.inv_tau_s;
   CT vd[Q];
-  if constexpr (sizeof(CT) == 4 || LEAN) {
-    [&]<int... A>(std::integer_sequence<int, A...>) {
-      ((vd[A] = cdotu<CX(A), CY(A), D == 3 ? CZ(A) : 0, CT>(u[0], u[1], u[2])), ...);
-    }(std::make_integer_sequence<int, Q>{});
-  } else {
-#pragma unroll
-    for (int a = 0; a < Q; a++) {
-      vd[a] = ((CT)CX(a)) * u[0] + ((CT)CY(a)) * u[1];
-      if (D == 3) vd[a] += ((CT)CZ(a)) * u[2];
-    }
-  }
+  [&]<int... A>(std::integer_sequence<int, A...>) {
+    ((vd[A] = cdotu<CX(A), CY(A), D == 3 ? CZ(A) : 0, CT>(u[0], u[1], u[2])), ...);
+  }(std::make_integer_sequence<int, Q>{});
   if constexpr (sizeof(CT) == 4) {
     // FP32 collision, the same update factored per node and fused
     // (FP32 and FP16 storage have no FP64 parity to keep): flow
@@ -518,7 +496,7 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
       else t = __builtin_fmaf(C, v * __builtin_fmaf((CT)4.5, v, (CT)3), B);
       f[a] = __builtin_fmaf(f[a], k1, w * t);
     }
-  } else if constexpr (LEAN) {
+  } else {
     const CT k1 = (CT)1 - it, s15 = (CT)1.5 * usq;
     auto relax = [&](int a, CT v3, CT v45) {
       CT fa = f[a] * k1;
@@ -538,20 +516,6 @@ __device__ __forceinline__ void collide(const StepArgs<ST, CT> &A, int idx, CT (
       const CT v45 = SUBS == 0 ? (CT)4.5 * vd[a] * vd[a] : (CT)0;
       relax(a, v3, v45);
       relax(a + 1, -v3, v45);
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < Q; a++) {
-      CT fa = f[a] * ((CT)1 - it);
-      const CT vdotu = vd[a];
-      const CT w = (CT)W<Q>(a);
-      if (SUBS == 1) {
-        fa += w * rho * ((CT)1 + (CT)3 * vdotu) * it;
-      } else {
-        fa += w * rho * it;
-        fa += w * A.rhoA * ((CT)3 * vdotu + (CT)4.5 * vdotu * vdotu - (CT)1.5 * usq) * it;
-      }
-      f[a] = fa;
     }
   }
   if constexpr (sizeof(CT) == 4 && sizeof(ST) >= 4) {
@@ -734,16 +698,15 @@ __device__ __forceinline__ void walsh_mix(CT (&f)[Q], const CT (&fp)[Q], CT ns, 
 }
 
 template <int Q, int NS, typename ST, typename CT, bool ODD, bool OFF32, bool WALSH = false>
-__global__ __launch_bounds__((half_step_block<ODD, NS, ST, CT>())) void k_half_step(StepArgs<ST, CT> A) {
+__global__ __launch_bounds__(kStepBlock) void k_half_step(StepArgs<ST, CT> A) {
   // node block: from the row-band map when the launch carries one, else the
   // XCD-contiguous remap
   const int lb = A.bmap ? A.bmap[blockIdx.x] : xcd_block(A.nblk8);
   if (lb < 0) return;
-  const int idx = lb * half_step_block<ODD, NS, ST, CT>() + (int)threadIdx.x;
+  const int idx = lb * (int)blockDim.x + (int)threadIdx.x;
   if (idx >= A.nf) return;
-  int nb[Q];
-  nb[0] = idx;
-  if (ODD) neighbors<Q>(A.G, idx, nb);
+  uint32_t loc[Q];
+  step_locs<Q, loc_unit<NS, ST, OFF32>(), ODD>(A.G, idx, loc);
   CT f[Q], u[3];
   CT ns = (CT)0, kns = (CT)1;
   if constexpr (WALSH) {
@@ -759,10 +722,10 @@ __global__ __launch_bounds__((half_step_block<ODD, NS, ST, CT>())) void k_half_s
       // streaming loads leave the L2 to the lines it writes (128^3 flow +
       // solute: replay 202 -> 188 ms per sweep, objective run with kept
       // states 188 -> 183 ms; in-place steps unchanged).
-      if (A.Fo != A.F) gather2<Q, ST, CT, ODD, OFF32, true>(A, idx, nb, f, g);
-      else gather2<Q, ST, CT, ODD, OFF32>(A, idx, nb, f, g);
+      if (A.Fo != A.F) gather2<Q, ST, CT, ODD, OFF32, true>(A, loc, f, g);
+      else gather2<Q, ST, CT, ODD, OFF32>(A, loc, f, g);
     } else {
-      gather2<Q, ST, CT, ODD, OFF32>(A, idx, nb, f, g);
+      gather2<Q, ST, CT, ODD, OFF32>(A, loc, f, g);
     }
     if constexpr (Q == 19)
       if (zface_node<Q>(A, idx)) zface_fix<ST, CT, true>(A, idx, f, g);
@@ -781,11 +744,11 @@ __global__ __launch_bounds__((half_step_block<ODD, NS, ST, CT>())) void k_half_s
       collide<Q, ST, CT, 0, ODD>(A, idx, f, u);
       collide<Q, ST, CT, 1, ODD>(A, idx, g, u);
     }
-    scatter2<Q, ST, CT, ODD, OFF32>(A, idx, nb, f, g);
+    scatter2<Q, ST, CT, ODD, OFF32>(A, idx, loc, f, g);
     return;
   }
   // flow alone (the solute, when present, is outside its active time window)
-  gather<Q, NS, ST, CT, 0, ODD, OFF32>(A, idx, nb, f);
+  gather<Q, ST, CT, 0, ODD, OFF32>(A, loc, f);
   if constexpr (Q == 19)
     if (zface_node<Q>(A, idx)) zface_fix<ST, CT, false>(A, idx, f, f);
   if constexpr (WALSH) {
@@ -797,7 +760,7 @@ __global__ __launch_bounds__((half_step_block<ODD, NS, ST, CT>())) void k_half_s
   } else {
     collide<Q, ST, CT, 0, ODD>(A, idx, f, u);
   }
-  scatter<Q, NS, ST, CT, 0, ODD, OFF32>(A, idx, nb, f);
+  scatter<Q, ST, CT, 0, ODD, OFF32>(A, idx, loc, f);
 }
 
 // ---- boundary conditions ------------------------------------------------
@@ -813,11 +776,12 @@ struct BcArgs {
 template <int Q, int NS, typename ST, typename CT, int SUBS>
 __device__ __forceinline__ void bc_gather(const BcArgs<ST, CT> &B, int idx, int (&nb)[Q], CT (&f)[Q]) {
   nb[0] = idx;
-  if (B.phase == 1) {
-    neighbors<Q>(B.A.G, idx, nb);
-    gather<Q, NS, ST, CT, SUBS, true>(B.A, idx, nb, f);
-  } else {
-    gather<Q, NS, ST, CT, SUBS, false>(B.A, idx, nb, f);
+  if (B.phase == 1) neighbors<Q>(B.A.G, idx, nb);
+#pragma unroll
+  for (int a = 0; a < Q; a++) {
+    const uint32_t own = foff<Q, NS>(SUBS, OPP(a), idx);
+    const uint32_t off = B.phase == 1 && nb[a] >= 0 ? foff<Q, NS>(SUBS, a, nb[a]) : own;
+    f[a] = Codec<ST, CT>::dec(B.A.F[off], B.A.inv_scale[SUBS], shift_of<Q, ST, CT, SUBS>(B.A, a));
   }
 }
 
@@ -893,13 +857,15 @@ __global__ void k_bc2d_pressure(BcArgs<ST, CT> B, int north, double rho_b, int v
   int nb[9];
   CT f[9], v[3];
   bc_gather<9, NS, ST, CT, SUBS>(B, idx, nb, f);
-  bc2d_flow_values<CT>(f, north, rho_b, SUBS == 0 ? B.A.rhoA : B.A.rhoA_s, velocity, v);
-  // constant slots in both branches (a run-time slot would index the neighbour ranks in scratch memory)
+  const CT rhoA = SUBS == 0 ? B.A.rhoA : B.A.rhoA_s;
+  // both branches whole, so that every index is a constant
   if (north) {
+    bc2d_flow_values<CT>(f, true, rho_b, rhoA, velocity, v);
     bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 4, v[0], velocity);
     bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 8, v[1], velocity);
     bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 6, v[2], velocity);
   } else {
+    bc2d_flow_values<CT>(f, false, rho_b, rhoA, velocity, v);
     bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 3, v[0], velocity);
     bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 7, v[2], velocity);
     bc_store<9, NS, ST, CT, SUBS>(B, idx, nb, 5, v[1], velocity);
@@ -927,12 +893,13 @@ __global__ void k_bc2d_zerograd(BcArgs<ST, CT> B, int north) {
   int nb[9];
   CT f[9], v[3];
   bc_gather<9, 2, ST, CT, 1>(B, idx, nb, f);
-  bc2d_zerograd_values<CT>(f, north, v);
   if (north) {
+    bc2d_zerograd_values<CT>(f, true, v);
     bc_store<9, 2, ST, CT, 1>(B, idx, nb, 4, v[0], false);
     bc_store<9, 2, ST, CT, 1>(B, idx, nb, 8, v[1], false);
     bc_store<9, 2, ST, CT, 1>(B, idx, nb, 6, v[2], false);
   } else {
+    bc2d_zerograd_values<CT>(f, false, v);
     bc_store<9, 2, ST, CT, 1>(B, idx, nb, 3, v[0], false);
     bc_store<9, 2, ST, CT, 1>(B, idx, nb, 7, v[2], false);
     bc_store<9, 2, ST, CT, 1>(B, idx, nb, 5, v[1], false);

@@ -92,6 +92,13 @@ LBM_HD uint32_t foff(int s, int a, uint32_t x) {
   return (x / kTile) * (uint32_t)(Q * kTile) + (uint32_t)(a * kTile) + (x % kTile);
 }
 
+// The same location in units of U per node (U = NS elements, or the NS
+// populations' bytes) with one multiplication.
+template <int Q, uint32_t U>
+LBM_HD uint32_t loc_at(int a, uint32_t x) {
+  return x * U + (x / kTile) * ((uint32_t)(Q - 1) * kTile * U) + (uint32_t)a * (kTile * U);
+}
+
 // fluid test and compact index of node (i, row r): one 16-byte load and
 // no branch, so the loads of all neighbours can be in flight together
 LBM_HD int rank_of(const Geo &G, int i, int r) {
@@ -207,100 +214,98 @@ LBM_HD void neighbors_of(const Geo &G, int i, int j, int k, const int (&dx)[K], 
 // nodes i-1, i, i+1 of a row come from the word holding i, its bitmask and
 // the ranks of the row's nodes just outside the word (dprev / dnext, which
 // also carry the periodic wrap at the row ends).  Every load is issued
-// before any rank is formed.  out[a-1] = compact index of x - c_a.
+// before any rank is formed.  For a = 1..Q-1: rank[a-1] = compact index of
+// x - c_a where fluid[a-1], else of no meaning.
+//
+// The half-steps of the narrow storage types are bound by the number of
+// vector instructions they issue (FP16 odd step, 192^3: 1312 of them, at 4
+// cycles a wave 106 of its 112 us), so a row costs one popcount (the ranks of
+// i - 1 and i + 1 follow from it by the bits of i - 1 and i) and one rotation
+// that brings those three bits down, everything else is selects, and the halo
+// form runs only in halo mode.
 template <int D>
-LBM_HD void neighbors_rows(const Geo &G, int i, int j, int k, int (&out)[D == 2 ? 8 : 18]) {
+LBM_HD void neighbors_core(const Geo &G, int i, int j, int k, int (&rank)[D == 2 ? 8 : 18],
+                           bool (&fluid)[D == 2 ? 8 : 18]) {
   // lattice rows (dy, dz) of the nodes x - c_a, in the reference order
-  constexpr int R = D == 2 ? 3 : 9;
+  constexpr int R = D == 2 ? 3 : 9, M = D == 2 ? 8 : 18;
   constexpr int rdy[9] = {0, -1, 1, 0, 0, -1, 1, 1, -1};
   constexpr int rdz[9] = {0, 0, 0, -1, 1, -1, 1, -1, 1};
+  // row and column offset of x - c_a
+  constexpr int row2[8] = {0, 0, 1, 2, 1, 2, 1, 2}, col2[8] = {-1, 1, 0, 0, -1, 1, 1, -1};
+  constexpr int row3[18] = {0, 0, 1, 2, 1, 2, 1, 2, 3, 4, 3, 4, 3, 4, 5, 6, 7, 8};
+  constexpr int col3[18] = {-1, 1, 0, 0, -1, 1, 1, -1, 0, 0, -1, 1, 1, -1, 0, 0, 0, 0};
   const int b = i & 63, w = i >> 6;
-  const int wend = (G.ni - 64 * w) < 64 ? (G.ni - 64 * w) : 64;  // valid bits of the word
-  uint64_t bits[R];
-  int base[R], dp[R], dn[R], gh[R];
-  bool cross[R];
+  const bool left = b == 0, right = b == 63 || i == G.ni - 1;  // no such node in the word
+  const uint32_t s = (uint32_t)(b + 63) & 63u;                 // rotation: bits i-1, i, i+1 become 0, 1, 2
+  const uint64_t below = (1ull << b) - 1ull;
   const RowWord *ptr[R];
 #pragma unroll
   for (int q = 0; q < R; q++) {
-    int last, lastw, row, p;
-    if (D == 2) {
-      last = j + rdy[q];
-      lastw = wrap1(last, G.nj);
-      row = lastw;
-      p = 0;
-    } else {
-      const int jj = wrap1(j + rdy[q], G.nj);
-      last = k + rdz[q];
-      lastw = wrap1(last, G.nk);
-      row = jj + G.nj * lastw;
-      p = G.ni * jj;
-    }
+    const int last = D == 2 ? j + rdy[q] : k + rdz[q];
+    const int lastw = wrap1(last, D == 2 ? G.nj : G.nk);
+    const int row = D == 2 ? lastw : wrap1(j + rdy[q], G.nj) + G.nj * lastw;
     ptr[q] = G.rw + ((long)row * G.W + w);
-    cross[q] = G.halo && last != lastw;
-    gh[q] = G.ghost + (last < 0 ? 0 : G.E) + p;  // + the column below
   }
+  int at[R], base[R];     // rank of the first fluid node at or after i, of the word's first
+  uint32_t near[R];       // bits 0..2: nodes i-1, i, i+1 (within the word)
+  int dp[R], dn[R];
 #pragma unroll
   for (int q = 0; q < R; q++) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const uint4 v = *reinterpret_cast<const uint4 *>(ptr[q]);
-    bits[q] = (uint64_t)v.x | ((uint64_t)v.y << 32);
+    const uint32_t x0 = s & 32u ? v.y : v.x, x1 = s & 32u ? v.x : v.y;
+    near[q] = __builtin_amdgcn_alignbit(x1, x0, s);
     base[q] = (int)v.z;
+    at[q] = base[q] + __popc(v.x & (uint32_t)below) + __popc(v.y & (uint32_t)(below >> 32));
     dp[q] = (int)(int16_t)(v.w & 0xffffu);
-    dn[q] = (int)(int16_t)(v.w >> 16);
+    dn[q] = (int)v.w >> 16;
 #else
-    bits[q] = ptr[q]->bits;
-    base[q] = ptr[q]->base;
-    dp[q] = ptr[q]->dprev;
-    dn[q] = ptr[q]->dnext;
+    const RowWord &v = *ptr[q];
+    near[q] = (uint32_t)(s ? (v.bits >> s) | (v.bits << (64 - s)) : v.bits);
+    base[q] = v.base;
+    at[q] = v.base + popc64(v.bits & below);
+    dp[q] = v.dprev;
+    dn[q] = v.dnext;
 #endif
   }
-  // rank of column offset dx in row q
-  auto rank = [&](int q, int dx) -> int {
-    int r;
+#pragma unroll
+  for (int a = 0; a < M; a++) {
+    const int q = D == 2 ? row2[a & 7] : row3[a], dx = D == 2 ? col2[a & 7] : col3[a];
     if (dx == 0) {
-      r = ((bits[q] >> b) & 1ull) ? base[q] + popc64(bits[q] & ((1ull << b) - 1ull)) : -1;
+      fluid[a] = near[q] & 2u;
+      rank[a] = at[q];
     } else if (dx < 0) {
-      const int bb = b - 1;
-      const int in = ((bits[q] >> (bb & 63)) & 1ull) ? base[q] + popc64(bits[q] & ((1ull << (bb & 63)) - 1ull)) : -1;
-      r = b > 0 ? in : (dp[q] == kSolidRank ? -1 : base[q] + dp[q]);
+      const int in = at[q] - 1, out = base[q] + dp[q];
+      const bool fin = near[q] & 1u, fout = dp[q] != kSolidRank;
+      fluid[a] = left ? fout : fin;
+      rank[a] = left ? out : in;
     } else {
-      const int bb = b + 1;
-      const int in = ((bits[q] >> (bb & 63)) & 1ull) ? base[q] + popc64(bits[q] & ((1ull << (bb & 63)) - 1ull)) : -1;
-      r = bb < wend ? in : (dn[q] == kSolidRank ? -1 : base[q] + dn[q]);
+      const int in = at[q] + (int)((near[q] >> 1) & 1u), out = base[q] + dn[q];
+      const bool fin = near[q] & 4u, fout = dn[q] != kSolidRank;
+      fluid[a] = right ? fout : fin;
+      rank[a] = right ? out : in;
     }
-    const int col = wrap1(i + dx, G.ni);
-    return (cross[q] && r >= 0) ? gh[q] + col : r;
-  };
-  if (D == 2) {
-    // a: 1 E, 2 W, 3 N, 4 S, 5 NE, 6 SW, 7 NW, 8 SE; x - c_a
-    out[0] = rank(0, -1);
-    out[1] = rank(0, 1);
-    out[2] = rank(1, 0);
-    out[3] = rank(2, 0);
-    out[4] = rank(1, -1);
-    out[5] = rank(2, 1);
-    out[6] = rank(1, 1);
-    out[7] = rank(2, -1);
-  } else {
-    out[0] = rank(0, -1);   // 1  (+1, 0, 0)
-    out[1] = rank(0, 1);    // 2  (-1, 0, 0)
-    out[2] = rank(1, 0);    // 3  (0, +1, 0)
-    out[3] = rank(2, 0);    // 4  (0, -1, 0)
-    out[4] = rank(1, -1);   // 5  (+1, +1, 0)
-    out[5] = rank(2, 1);    // 6  (-1, -1, 0)
-    out[6] = rank(1, 1);    // 7  (-1, +1, 0)
-    out[7] = rank(2, -1);   // 8  (+1, -1, 0)
-    out[8] = rank(3, 0);    // 9  (0, 0, +1)
-    out[9] = rank(4, 0);    // 10 (0, 0, -1)
-    out[10] = rank(3, -1);  // 11 (+1, 0, +1)
-    out[11] = rank(4, 1);   // 12 (-1, 0, -1)
-    out[12] = rank(3, 1);   // 13 (-1, 0, +1)
-    out[13] = rank(4, -1);  // 14 (+1, 0, -1)
-    out[14] = rank(5, 0);   // 15 (0, +1, +1)
-    out[15] = rank(6, 0);   // 16 (0, -1, -1)
-    out[16] = rank(7, 0);   // 17 (0, -1, +1)
-    out[17] = rank(8, 0);   // 18 (0, +1, -1)
   }
+  if (G.halo) {
+    // across the last axis: ghost entries, as solid as the periodic image
+#pragma unroll
+    for (int a = 0; a < M; a++) {
+      const int q = D == 2 ? row2[a & 7] : row3[a], dx = D == 2 ? col2[a & 7] : col3[a];
+      const int last = D == 2 ? j + rdy[q] : k + rdz[q];
+      const int col = wrap1(i + dx, G.ni) + (D == 2 ? 0 : G.ni * wrap1(j + rdy[q], G.nj));
+      const int gh = G.ghost + (last < 0 ? 0 : G.E) + col;
+      rank[a] = last != wrap1(last, D == 2 ? G.nj : G.nk) ? gh : rank[a];
+    }
+  }
+}
+
+// out[a-1] = compact index of x - c_a, -1 when solid
+template <int D>
+LBM_HD void neighbors_rows(const Geo &G, int i, int j, int k, int (&out)[D == 2 ? 8 : 18]) {
+  bool fluid[D == 2 ? 8 : 18];
+  neighbors_core<D>(G, i, j, k, out, fluid);
+#pragma unroll
+  for (int a = 0; a < (D == 2 ? 8 : 18); a++) out[a] = fluid[a] ? out[a] : -1;
 }
 
 // Host: fill the row words from the dense -> compact map (fid[n] = -1 for

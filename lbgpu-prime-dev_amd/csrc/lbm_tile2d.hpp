@@ -216,13 +216,13 @@ __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<doub
       fp[a] = f[a];
       if (SOL) gp[a] = gs[a];
     }
-    collide<9, double, double, 0, ODD, true, true>(A, idx, f, u, kns);
-    if constexpr (SOL) collide<9, double, double, 1, ODD, true, true>(A, idx, gs, u, kns);
+    collide<9, double, double, 0, ODD, true>(A, idx, f, u, kns);
+    if constexpr (SOL) collide<9, double, double, 1, ODD, true>(A, idx, gs, u, kns);
     walsh_mix<9, double>(f, fp, ns, kns);
     if constexpr (SOL) walsh_mix<9, double>(gs, gp, ns, kns);
   } else {
-    collide<9, double, double, 0, ODD, false, true>(A, idx, f, u);
-    if constexpr (SOL) collide<9, double, double, 1, ODD, false, true>(A, idx, gs, u);
+    collide<9, double, double, 0, ODD>(A, idx, f, u);
+    if constexpr (SOL) collide<9, double, double, 1, ODD>(A, idx, gs, u);
   }
 #pragma unroll
   for (int a = 0; a < 9; a++) {
