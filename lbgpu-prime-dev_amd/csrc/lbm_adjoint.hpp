@@ -55,13 +55,6 @@ constexpr int kAdjBlock = 64;
 // launch at 128^3).  The odd step, with its neighbour ranks, runs at one
 // wave (344 registers): squeezed to two (256 registers and 356 B of spills
 // per lane) the adjoint kernels of a 128^3 sweep took 313 ms instead of 303.
-#ifndef LBM_ADJ_WAVES_ODD
-#define LBM_ADJ_WAVES_ODD 1
-#endif
-#ifndef LBM_ADJ_WAVES_EVEN
-#define LBM_ADJ_WAVES_EVEN 2
-#endif
-
 // Weighted moments of the adjoint of one node:
 //   Lr = sum w lam, L1 = sum w lam c, L2 = sum w lam c c^T (xx yy zz xy xz yz),
 //   M0 = sum w mu,  M1 = sum w mu c.
@@ -405,8 +398,8 @@ __device__ __forceinline__ void adj_face_block(const AdjArgs &J, long slot, int 
 // 8 * nblk8 blocks) when there is one, else from the XCD-contiguous remap.
 // Gradient partials: slot b of face block b, slot nfb + node block of the
 // others (so the block order does not change the sums).
-template <bool ODD, bool OFF32>
-__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(ODD ? LBM_ADJ_WAVES_ODD : LBM_ADJ_WAVES_EVEN)))
+template <bool ODD, bool OFF32, bool FEW>
+__global__ __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(ODD || FEW ? 1 : 2)))
 void k_adjoint_step(AdjArgs J, int nfb) {
   if ((int)blockIdx.x < nfb) {
     adj_face_block<ODD, OFF32>(J, blockIdx.x, blockIdx.x);

@@ -279,6 +279,10 @@ bool zface_fused(const lbm_handle *h, int t) {
   return true;
 }
 
+// Whether step t leaves the state it reads untouched when it runs out of
+// place: no separate boundary launch stores into it.
+bool plain_state(const lbm_handle *h, int t) { return zface_fused(h, t) || !zface_any(h); }
+
 template <typename ST, typename CT>
 void set_zb(const lbm_handle *h, StepArgs<ST, CT> &A) {
   A.zb.on = 1;
@@ -1880,8 +1884,13 @@ extern "C" int lbm_objective_run(lbm_handle *h, int nsteps, int window, int ever
   const double *mv_c = h->mv + (long)1 * (1 + h->D) * h->nf;  // solute concentration
   int ob = 0;
   void *const live = h->F;
-  // the kept steps run out of place: kept[i] -> kept[i + 1], the last one
-  // into the lattice's own array
+  // Steps run in place in the lattice's own array, except that a step whose
+  // result is saved writes it straight into the checkpoint or the first kept
+  // state, the step after a checkpoint reads it there and writes the own
+  // array again, and the kept steps run kept[i] -> kept[i + 1], the last one
+  // into the own array.  A copy is left for the run's first state and where a
+  // separate boundary launch writes into the state it reads (a saved state is
+  // the one before its step's boundary conditions).
   struct Restore {
     lbm_handle *h;
     void *F;
@@ -1890,15 +1899,19 @@ extern "C" int lbm_objective_run(lbm_handle *h, int nsteps, int window, int ever
       h->Fout = nullptr;
     }
   } restore{h, live};
+  // where the state before step q is saved, or null
+  auto saved = [&](int q) -> void * {
+    if (q >= kept_from) return q < nsteps ? o.kept[q - kept_from] : nullptr;
+    return q % every == 0 ? o.ckpt[q / every] : nullptr;
+  };
   for (int q = 0; q < nsteps; q++) {
-    if (q < kept_from && q % every == 0)
-      HIP_OK(hipMemcpyAsync(o.ckpt[q / every], h->F, sb, hipMemcpyDeviceToDevice, h->stream));
-    if (q >= kept_from) {
-      const int i = q - kept_from;
-      if (i == 0) HIP_OK(hipMemcpyAsync(o.kept[0], live, sb, hipMemcpyDeviceToDevice, h->stream));
-      h->F = o.kept[i];
-      h->Fout = i + 1 < (int)P ? o.kept[i + 1] : live;
+    void *const to = saved(q);
+    if (to && h->F != to) {
+      HIP_OK(hipMemcpyAsync(to, h->F, sb, hipMemcpyDeviceToDevice, h->stream));
+      if (q >= kept_from) h->F = to;
     }
+    void *const next = saved(q + 1);
+    h->Fout = next && (q + 1 >= kept_from || plain_state(h, t0 + q + 2)) ? next : live;
     const bool in_window = q >= nsteps - window;
     int oe = ob;
     while (oe < nobs && o.o_step[oe] == q + 1) oe++;
@@ -1921,6 +1934,7 @@ extern "C" int lbm_objective_run(lbm_handle *h, int nsteps, int window, int ever
       HIP_OK(hipGetLastError());
     }
     ob = oe;
+    h->F = h->Fout;
   }
   h->F = live;
   h->Fout = nullptr;
@@ -2057,20 +2071,25 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
     // the states before the segment's steps, after their BCs: kept by the
     // objective run, or replayed from the segment's checkpoint
     void *const *sp = sgi >= nrep ? h->obj.kept.data() + ((long)sgi * K - h->obj.kept_from) : rp;
-    if (sgi < nrep && (e = hipMemcpyAsync(rp[0], h->obj.ckpt[sgi], sb, hipMemcpyDeviceToDevice, h->stream)) !=
-                          hipSuccess) {
+    // the checkpoint itself serves as the segment's first state unless a
+    // separate boundary launch would write into it
+    void *const first = sgi < nrep && plain_state(h, ts + 1) ? h->obj.ckpt[sgi] : sp[0];
+    if (sgi < nrep && first == rp[0] &&
+        (e = hipMemcpyAsync(rp[0], h->obj.ckpt[sgi], sb, hipMemcpyDeviceToDevice, h->stream)) != hipSuccess) {
       fail("checkpoint restore", e);
       break;
     }
     // replay the segment out of place, keeping every state after its BCs
+    // (the state after its last step belongs to the next segment)
     for (int q = 1; q <= len && !rc && sgi < nrep; q++) {
       const int t = ts + q;
-      h->F = rp[q - 1];
+      h->F = q == 1 ? first : rp[q - 1];
       const bool fz = zface_fused(h, t);
       if (!fz && launch_bcs(h, (t & 1) ? 1 : 2, t)) {
         rc = 1;
         break;
       }
+      if (q == len) break;
       StepArgs<double, double> A = make_args<double, double>(h);
       if (fz) set_zb(h, A);
       A.Fo = (double *)rp[q];
@@ -2095,7 +2114,7 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
       const int t = ts + q;
       const bool odd = t & 1;
       AdjArgs J;
-      h->F = sp[q - 1];
+      h->F = q == 1 ? first : sp[q - 1];
       const bool fz = zface_fused(h, t);
       J.A = make_args<double, double>(h);
       J.amap = h->amap;
@@ -2133,12 +2152,15 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
       const int fb = fz ? nfb : 0;
       dim3 grid(nblk + fb), block(kAdjBlock);
       Prof pr(h, 5);
+      // (few nodes are always below 4 GiB unless 64-bit offsets are forced)
+      const bool few = h->nf < kFewNodes && off32;
       if (odd) {
-        if (off32) hipLaunchKernelGGL((k_adjoint_step<true, true>), grid, block, 0, h->stream, J, fb);
-        else hipLaunchKernelGGL((k_adjoint_step<true, false>), grid, block, 0, h->stream, J, fb);
+        if (off32) hipLaunchKernelGGL((k_adjoint_step<true, true, false>), grid, block, 0, h->stream, J, fb);
+        else hipLaunchKernelGGL((k_adjoint_step<true, false, false>), grid, block, 0, h->stream, J, fb);
       } else {
-        if (off32) hipLaunchKernelGGL((k_adjoint_step<false, true>), grid, block, 0, h->stream, J, fb);
-        else hipLaunchKernelGGL((k_adjoint_step<false, false>), grid, block, 0, h->stream, J, fb);
+        if (few) hipLaunchKernelGGL((k_adjoint_step<false, true, true>), grid, block, 0, h->stream, J, fb);
+        else if (off32) hipLaunchKernelGGL((k_adjoint_step<false, true, false>), grid, block, 0, h->stream, J, fb);
+        else hipLaunchKernelGGL((k_adjoint_step<false, false, false>), grid, block, 0, h->stream, J, fb);
       }
       if ((e = hipGetLastError()) != hipSuccess) {
         fail("adjoint step", e);
