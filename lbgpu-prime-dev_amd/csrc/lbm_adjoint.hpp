@@ -55,6 +55,10 @@ constexpr int kAdjBlock = 64;
 // launch at 128^3).  The odd step, with its neighbour ranks, runs at one
 // wave (344 registers): squeezed to two (256 registers and 356 B of spills
 // per lane) the adjoint kernels of a 128^3 sweep took 313 ms instead of 303.
+// The adjoint's own sums are contracted to fused multiply-adds (nothing has to
+// match them bit for bit; 626 -> 478 FP64 instructions of the even step: 72 x
+// 68 x 80 33.97 -> 33.46 us a step, 128^3 138.8 -> 136.6).
+
 // Weighted moments of the adjoint of one node:
 //   Lr = sum w lam, L1 = sum w lam c, L2 = sum w lam c c^T (xx yy zz xy xz yz),
 //   M0 = sum w mu,  M1 = sum w mu c.
@@ -70,6 +74,7 @@ struct AdjMoments {
 template <bool ODD, bool OFF32>
 __device__ __forceinline__ void adj_load(const AdjArgs &J, const uint32_t (&loc)[19], double (&lam)[19],
                                          double (&mu)[19], AdjMoments &m) {
+#pragma clang fp contract(fast)
 #pragma unroll
   for (int a = 0; a < 19; a++) {
     const pair_t<double> v = ld_stream<!ODD>((const pair_t<double> *)at_loc<OFF32>(J.L, loc[OPP(a)]));
@@ -107,6 +112,7 @@ struct AdjState {
 
 template <int A_>
 __device__ __forceinline__ void adj_state_add(AdjState &st, double f, double g, double lam, double mu) {
+#pragma clang fp contract(fast)
   st.drho += f;
   if (CX(A_) != 0) st.j[0] += CX(A_) > 0 ? f : -f;
   if (CY(A_) != 0) st.j[1] += CY(A_) > 0 ? f : -f;
@@ -148,6 +154,7 @@ struct AdjOut {
 };
 
 __device__ __forceinline__ AdjOut adj_collide(const AdjArgs &J, const AdjMoments &m, const AdjState &st) {
+#pragma clang fp contract(fast)
   const StepArgs<double, double> &A = J.A;
   const double rhoA = A.rhoA, tau = A.tau, om = A.inv_tau, oms = A.inv_tau_s;
   double u[3];
@@ -189,6 +196,7 @@ __device__ __forceinline__ AdjOut adj_collide(const AdjArgs &J, const AdjMoments
 template <int B_>
 __device__ __forceinline__ void adj_new(const AdjArgs &J, const AdjOut &o, double seed, double oseed, double lam,
                                         double mu, double &lb, double &mb) {
+#pragma clang fp contract(fast)
   const double om = J.A.inv_tau, oms = J.A.inv_tau_s;
   lb = (1.0 - om) * lam + om * o.Lr;
   if (CX(B_) != 0) lb += CX(B_) > 0 ? o.Gr[0] : -o.Gr[0];
@@ -245,11 +253,44 @@ __device__ __forceinline__ void adj_locs_again(int idx, uint32_t (&loc)[19]) {
   }
 }
 
-__device__ __forceinline__ void adj_block_sum(const AdjArgs &J, long slot, double (&acc)[5]) {
-  __shared__ double red[5];
-  const int kinds[5] = {0, 0, 0, 0, 0};
-  block_reduce<5, kAdjBlock / 64>(acc, kinds, red);
-  if (threadIdx.x < 5) J.gacc[slot * 5 + threadIdx.x] += red[threadIdx.x];
+// The parameter terms of a one-wave workgroup, added to its slot.  The slot's
+// old values are loaded before the node's own loads and the wave sums by
+// data-parallel moves, so that the wave ends soon after its stores (a load at
+// the end and sums through LDS: 48 x 40 x 60 14.62 -> 14.35 us a step, 128^3
+// 136.6 -> 135.9).
+struct AdjSlot {
+  double v[5];
+};
+__device__ __forceinline__ AdjSlot adj_slot_load(const AdjArgs &J, long slot) {
+  AdjSlot o;
+#pragma unroll
+  for (int q = 0; q < 5; q++) o.v[q] = J.gacc[slot * 5 + q];
+  return o;
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t u = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+// lane 63: the sum over the wave (a lane without a source adds 0)
+__device__ __forceinline__ double wave_sum_last(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: each row's last lane has its sum
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
+  return dpp_add<0x143, 0xc>(v);
+}
+__device__ __forceinline__ void adj_slot_add(const AdjArgs &J, long slot, const AdjSlot &old, double (&acc)[5]) {
+  static_assert(kAdjBlock == 64, "one wave");
+#pragma unroll
+  for (int q = 0; q < 5; q++) acc[q] = wave_sum_last(acc[q]);
+  if (threadIdx.x == 63) {
+#pragma unroll
+    for (int q = 0; q < 5; q++) J.gacc[slot * 5 + q] = old.v[q] + acc[q];
+  }
 }
 
 // transpose of the flow z-face condition on the new adjoint of a face node:
@@ -344,6 +385,7 @@ template <bool ODD, bool OFF32>
 __device__ __forceinline__ void adj_face_block(const AdjArgs &J, long slot, int fb) {
   const StepArgs<double, double> &A = J.A;
   const int t = fb * kAdjBlock + (int)threadIdx.x;
+  const AdjSlot old = adj_slot_load(J, slot);
   const int nlo = A.zb.lo_end, nface = nlo + (A.nf - A.zb.hi_begin);
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (t < nface) {
@@ -387,7 +429,7 @@ __device__ __forceinline__ void adj_face_block(const AdjArgs &J, long slot, int 
 #pragma unroll
     for (int q = 0; q < 5; q++) acc[q] = o.acc[q];
   }
-  adj_block_sum(J, slot, acc);
+  adj_slot_add(J, slot, old, acc);
 }
 
 // Adjoint of one half-step.  With A.zb.on the first nfb blocks (a multiple
@@ -407,6 +449,7 @@ void k_adjoint_step(AdjArgs J, int nfb) {
   }
   const int lb = J.amap ? J.amap[blockIdx.x - nfb] : xcd_block(J.A.nblk8, (int)blockIdx.x - nfb);
   const int idx = lb * kAdjBlock + (int)threadIdx.x;
+  const AdjSlot old = adj_slot_load(J, nfb + (long)lb);
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (idx < J.A.nf && !zface_node<19>(J.A, idx)) {
     uint32_t loc[19];
@@ -424,7 +467,7 @@ void k_adjoint_step(AdjArgs J, int nfb) {
 #pragma unroll
     for (int q = 0; q < 5; q++) acc[q] = o.acc[q];
   }
-  adj_block_sum(J, nfb + (long)lb, acc);
+  adj_slot_add(J, nfb + (long)lb, old, acc);
 }
 
 // Transpose of the z-face conditions of k_bc_zface for one face.
