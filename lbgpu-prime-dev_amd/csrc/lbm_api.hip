@@ -114,6 +114,7 @@ struct lbm_handle {
     int state = 0;  // 0 not planned, 1 ready, -1 not for this lattice
     TileGeo T{};
     int steps = 0, shrink = 0, threads = 0;
+    bool keep = false;  // one tile per CU, one node per thread
     int lds_set = 0;  // kernels whose LDS limit has been raised
     size_t lds = 0;
     int *gidx = nullptr, *cnt = nullptr;
@@ -1190,23 +1191,26 @@ int tile_launch(lbm_handle *h, const TileArgs &B) {
       HIP_OK(hipGetLastError());
       return 0;
     }
-  return t.threads == 512 ? tiles(k_tile2d<NS, SOL, WALSH, 512>) : tiles(k_tile2d<NS, SOL, WALSH, 1024>);
+  return t.keep ? tiles(k_tile2d<NS, SOL, WALSH, true>) : tiles(k_tile2d<NS, SOL, WALSH, false>);
 }
 
-// Steps per launch, core and threads of k_tile2d for the handle's lattice.
+// Steps per launch and core of k_tile2d for the handle's lattice.
 // A lattice that one tile per CU covers takes the smallest square core that
 // does: its time is launch (2 us) and per-step latency (1 us), so it takes
 // as many steps a launch as the halo's work allows, 8 (two components with
-// cores above 12: 6; cores above 20: 4).  Measured, us per step, flow | flow +
-// solute with row conditions: 128^2 8 x 8 cores 1.54 | 1.94 (4 steps 1.74 |
-// 2.06), 200 x 170 12 x 12 cores 1.64 | 2.07 (4 steps 1.9 | 2.19), 300 x 310
-// 20 x 20 cores 1.97 with 8 steps | 2.71 with 6 (4 steps: 2.3 | 2.86).
+// cores above 12: 6; cores above 20: 4).  Measured when the kernel was first
+// tuned, us per step, flow | flow + solute with row conditions: 128^2 8 x 8
+// cores 1.54 | 1.94 (4 steps 1.74 | 2.06), 200 x 170 12 x 12 cores 1.64 | 2.07
+// (4 steps 1.9 | 2.19), 300 x 310 20 x 20 cores 1.97 with 8 steps | 2.71 with 6
+// (4 steps: 2.3 | 2.86).
 // Larger lattices run several tiles per CU and are bound by the loads of the
 // halo and the FP64 units together: 4 steps, flow in 32 x 16 cores of which a
 // CU holds two (1000^2 10.8, 2100 x 1900 44.9 us; 30 x 30 cores with 8 steps
 // 11.3, 43.7), flow + solute in the largest square core that LDS holds, 25 x
 // 25 (19.7, 85.3 us; 32 x 16 20.4, 91.4; 20 x 20 with 6 steps 22.2, 94.9).
-void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy, int &threads) {
+// Now, with entries in registers: 1.30 | 1.77, 1.38 | 1.91, 1.93 | 2.67 us;
+// 1000^2 9.8 | 18.2, 2100 x 1900 41.0 us.
+void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy) {
   const int ns = h->p.nsubs;
   const double per_cu = (double)h->N / h->cus;
   int s = 8;
@@ -1215,8 +1219,8 @@ void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy, i
   auto most = [&](int k) {  // largest square core of k steps
     int c = 0;
     const int halo = shrink * k / 2;
-    while (c + 1 + 2 * halo <= 64 && (size_t)(c + 1 + 2 * halo) * (c + 1 + 2 * halo) * (72 * ns + 4) <= (size_t)h->lds_cu)
-      c++;
+    auto fits = [&](int r) { return r * r <= kTileRegion && (size_t)r * r * 72 * ns <= (size_t)h->lds_cu; };
+    while (fits(c + 1 + 2 * halo)) c++;
     return c;
   };
   if (most(steps) < s) steps = 4;
@@ -1225,8 +1229,6 @@ void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy, i
     cx = 32;
     cy = 16;
   }
-  const int halo = shrink * steps / 2;
-  threads = (cx + 2 * halo) * (cy + 2 * halo) > 800 && !(s > 20 && ns == 1) ? 1024 : 512;
 }
 
 // Plans the tiles of the handle's lattice on first use; h->tile.state tells
@@ -1268,10 +1270,10 @@ int plan_tiles(lbm_handle *h) {
   t.T.ni = ni;
   t.T.nj = nj;
   // Strips (k_sweep2d) for flow + solute lattices of many tiles per CU, us per
-  // step, tiles -> strips: 1000^2 19.8 -> 19.6, 1088 x 1224 30.0 -> 24.2,
-  // 2100 x 1900 84.6 -> 63.4, below that tiles are faster (600 x 500 7.1
+  // step, tiles -> strips: 1000^2 18.2 -> 19.6, 1088 x 1224 28 -> 23.8,
+  // 2100 x 1900 80 -> 62, below that tiles are faster (600 x 500 6.7
   // against 9.2: short strips repeat their pipeline's start too often).  Flow
-  // alone keeps tiles (1088 x 1224 13.8 against 17.2, 2100 x 1900 45.0 against
+  // alone keeps tiles (1088 x 1224 12.4 against 17.2, 2100 x 1900 41.0 against
   // 41.9).  Rows that hand values to a neighbour need the tiles' barrier.
   if (two && !handed && h->N >= 4500L * h->cus) {
     SweepGeo &S = t.S;
@@ -1296,7 +1298,7 @@ int plan_tiles(lbm_handle *h) {
     t.state = 1;
     return 0;
   }
-  tile_shape(h, t.shrink, t.steps, t.T.cx, t.T.cy, t.threads);
+  tile_shape(h, t.shrink, t.steps, t.T.cx, t.T.cy);
   const int cx = t.T.cx, cy = t.T.cy;
   TileGeo &T = t.T;
   T.halo = t.shrink * t.steps / 2;
@@ -1309,12 +1311,16 @@ int plan_tiles(lbm_handle *h) {
   T.rx = T.cx + 2 * T.halo;
   T.rn = T.rx * (T.cy + 2 * T.halo);
   T.tiles8 = (T.tx * T.ty + 7) / 8;
-  t.lds = (size_t)T.rn * (72 * p.nsubs + 4);
+  t.lds = (size_t)T.rn * 72 * p.nsubs;
+  t.threads = std::min(kTileThreads, (T.rn + 63) / 64 * 64);
+  t.keep = T.rn <= kTileThreads && T.tx * T.ty <= h->cus;
+  // two workgroups of a CU fit its registers with 512 threads each
+  if (!t.keep && 2 * t.lds <= (size_t)h->lds_cu) t.threads = std::max(512, (T.rn / 2 + 63) / 64 * 64);
   if (T.rn > kTileRegion || t.lds > (size_t)h->lds_cu) return 0;
   const long n = (long)T.tx * T.ty;
   if (hipMalloc(&t.gidx, (size_t)n * T.rn * sizeof(int)) != hipSuccess ||
       hipMalloc(&t.list, (size_t)n * T.rn * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&t.cnt, (size_t)n * (kTileHalo + 1) * sizeof(int)) != hipSuccess ||
+      hipMalloc(&t.cnt, (size_t)n * sizeof(int)) != hipSuccess ||
       hipMalloc(&t.F2, sb) != hipSuccess)
     return off();
   hipLaunchKernelGGL(k_tile_build, dim3((unsigned)n), dim3(256), 0, h->stream, A.G, T, t.gidx, t.list, t.cnt);

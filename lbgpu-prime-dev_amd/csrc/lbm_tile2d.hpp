@@ -23,9 +23,9 @@
 // results equal the step-by-step launches bit for bit.
 //
 // Measured per step, against half-steps and row launches one by one: 128^2
-// flow between walls 3.3 -> 1.3 us; 1088 x 1224 flow + solute with series rows
-// 58 -> 28 us; 600 x 500 with partial bounce-back 24 -> 7.8 us; 413 x 307
-// with rows 18.5 -> 3.6 us.  Small lattices are bound by the latency of a
+// flow between walls 3.3 -> 1.1 us; 1088 x 1224 flow + solute with series rows
+// 58 -> 28 us (strips, below: 23.8); 600 x 500 with partial bounce-back 24 ->
+// 7.5 us; 413 x 307 with rows 18.5 -> 3.3 us.  Small lattices are bound by the latency of a
 // step inside the workgroup (about 1 us: LDS gathers, the collision's serial
 // sums, the barrier), large ones by the loads of core and halo (1.7 times the
 // core at 25 x 25 with 4 steps) followed by the FP64 units, which one
@@ -38,11 +38,14 @@ namespace lbm {
 
 constexpr int kTileSteps = 16;   // most steps of one launch
 constexpr int kTileHalo = 24;    // widest halo: 3 nodes per pair of steps
-constexpr int kTileRegion = 4096;  // most region nodes (12-bit region index)
+constexpr int kTileRegion = 2048;  // most region nodes (below 4096: 12-bit region index)
 
 // list entry of a fluid region node: region index, bit 12 + a - 1 set when
-// x - c_a is fluid, and the boundary rows
+// x - c_a is fluid, the boundary rows, and from bit 22 its distance from the
+// region's edge (at most the halo)
 constexpr uint32_t kTileNorth = 1u << 20, kTileSouth = 1u << 21;
+constexpr int kTileDist = 22;
+constexpr int kTileThreads = 1024;  // most threads of k_tile2d, which take at most two nodes each
 
 struct TileGeo {
   int ni, nj;
@@ -64,8 +67,8 @@ LBM_HD void tile_span(const TileGeo &T, int t, int &x0, int &y0, int &cw, int &c
 
 // Per tile: gidx[rn] (compact index of each region node, -1: solid or
 // outside), the list of its fluid nodes ordered by distance from the region's
-// edge (core first, then ring by ring inwards to outwards, each row-major),
-// and cnt[d] = number of list entries with distance >= d, d = 0..H.
+// edge (core first, then ring by ring inwards to outwards, each row-major,
+// so that whole waves fall idle as the halo shrinks), and their number.
 __global__ __launch_bounds__(256) void k_tile_build(Geo G, TileGeo T, int *gidx, uint32_t *list, int *cnt) {
   __shared__ int wsum[4];
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(256) void k_tile_build(Geo G, TileGeo T, int *gidx,
       for (int q = 0; q < wv; q++) at += wsum[q];
       if (in) {
         const int i = wrap(x0 - T.halo + rx, T.ni), j = wrap(y0 - T.halo + ry, T.nj);
-        uint32_t e = (uint32_t)n;
+        uint32_t e = (uint32_t)n | (uint32_t)d << kTileDist;
 #pragma unroll
         for (int a = 1; a < 9; a++)
           if (rank_of(G, wrap1(i - CX(a), T.ni), wrap1(j - CY(a), T.nj)) >= 0) e |= 1u << (11 + a);
@@ -115,8 +118,8 @@ __global__ __launch_bounds__(256) void k_tile_build(Geo G, TileGeo T, int *gidx,
       run += wsum[0] + wsum[1] + wsum[2] + wsum[3];
       __syncthreads();
     }
-    if (tid == 0) cnt[(long)t * (kTileHalo + 1) + d] = run;
   }
+  if (tid == 0) cnt[t] = run;
 }
 
 struct TileArgs {
@@ -186,13 +189,12 @@ __device__ __forceinline__ void tile_locs(const TileAt &P, uint32_t e, int (&loc
   }
 }
 
-// one half-step of one node; LAST: the result goes to the output array (the
-// node's compact index is idx), else back to LDS; ns: partial bounce-back
+// one half-step of one node, which collides from loc; LAST: the result goes to
+// the output array (the node's compact index is idx), else back to LDS; ns:
+// partial bounce-back
 template <int NS, bool SOL, bool WALSH, bool ODD, bool LAST>
 __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<double, double> &A, tile_t<NS> *lds,
-                                          const TileAt &P, int idx, double ns, uint32_t e, bool rows, int step) {
-  int loc[9];
-  tile_locs<ODD>(P, e, loc);
+                                          const int (&loc)[9], int idx, double ns, uint32_t e, bool rows, int step) {
   double f[9], gs[9], u[3];
 #pragma unroll
   for (int a = 0; a < 9; a++) {
@@ -227,7 +229,7 @@ __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<doub
 #pragma unroll
   for (int a = 0; a < 9; a++) {
     // even: own slot a (a resting solute keeps its slot a, gathered as direction opp(a))
-    const int at = ODD ? loc[OPP(a)] : a * P.plane + P.n0;
+    const int at = loc[OPP(a)];
     tile_t<NS> v;
     v[0] = f[a];
     if constexpr (NS == 2) v[NS - 1] = SOL ? gs[a] : gs[OPP(a)];
@@ -240,21 +242,25 @@ __device__ __forceinline__ void tile_node(const TileArgs &B, const StepArgs<doub
   }
 }
 
-template <int NS, bool SOL, bool WALSH, int NT>
-__global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
+// A thread takes list entry tid and keeps what it needs in every step, its
+// locations among it, in registers (KEEP: lattices of one tile per CU, whose
+// steps are bound by their latency; with the list in LDS, counts in global
+// memory and locations formed in every step, 128^2 took 1.55 us a step instead
+// of 1.33).  Larger lattices want the registers for a second workgroup on the
+// CU: they take entry tid + blockDim.x too and form locations as they go.
+template <int NS, bool SOL, bool WALSH, bool KEEP>
+__global__ __launch_bounds__(kTileThreads) void k_tile2d(TileArgs B) {
+  constexpr int PER = KEEP ? 1 : 2;
   extern __shared__ __align__(16) char tile_lds[];
   const int t = xcd_block(B.T.tiles8);
   if (t >= B.T.tx * B.T.ty) return;
-  const int tid = threadIdx.x, rn = B.T.rn, H = B.T.halo;
+  const int tid = threadIdx.x, nt = blockDim.x, rn = B.T.rn;
   tile_t<NS> *lds = (tile_t<NS> *)tile_lds;
-  uint32_t *lst = (uint32_t *)(lds + 9 * rn);
   const int *g = B.gidx + (long)t * rn;
-  const int *cnt = B.cnt + (long)t * (kTileHalo + 1);
-  const int fluid = cnt[0], core = cnt[H];
-  if (core == 0) return;
-  for (int n = tid; n < rn; n += NT) {
+  const uint32_t *list = B.list + (long)t * rn;
+  const int fluid = B.cnt[t];
+  for (int n = tid; n < rn; n += nt) {
     const int idx = g[n];
-    if (n < fluid) lst[n] = B.list[(long)t * rn + n];
     if (idx < 0) continue;
     tile_t<NS> v[9];
 #pragma unroll
@@ -262,26 +268,53 @@ __global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
 #pragma unroll
     for (int a = 0; a < 9; a++) lds[a * rn + n] = v[a];
   }
+  uint32_t e[PER];
+  int dist[PER], idx[PER], keep_odd[9], keep_even[9];
+  double ns[PER];
+  const TileAt at0{rn, 0, -B.T.rx, B.T.rx};
+#pragma unroll
+  for (int q = 0; q < PER; q++) {
+    const int p = tid + q * nt;
+    e[q] = p < fluid ? list[p] : 0u;
+    dist[q] = p < fluid ? (int)(e[q] >> kTileDist) : -1;
+    const int n = (int)(e[q] & 4095u);
+    idx[q] = p < fluid && (KEEP || WALSH) ? g[n] : 0;
+    ns[q] = WALSH ? B.A.ns[idx[q]] : 0.;
+  }
+  auto at = [&](int q) {
+    TileAt P = at0;
+    P.n0 = (int)(e[q] & 4095u);
+    return P;
+  };
+  if constexpr (KEEP) {
+    tile_locs<true>(at(0), e[0], keep_odd);
+    tile_locs<false>(at(0), e[0], keep_even);
+  }
+  auto locs = [&](auto odd, int q, int (&loc)[9]) __attribute__((always_inline)) {
+    if constexpr (!KEEP) {
+      asm("" : "+v"(e[q]));  // formed here, not ahead of the loop
+      tile_locs<decltype(odd)::value>(at(q), e[q], loc);
+    } else {
+#pragma unroll
+      for (int a = 0; a < 9; a++) loc[a] = decltype(odd)::value ? keep_odd[a] : keep_even[a];
+    }
+  };
+  using Odd = std::true_type;
+  using Even = std::false_type;
   __syncthreads();
   const bool rows = B.flow[0] || B.flow[1] || (NS == 2 && (B.grad[0] || B.grad[1]));
   const bool handed = B.shrink > 2;
   StepArgs<double, double> A = B.A;
   A.write_mv = 0;
   int s = 0;
-  auto at = [&](uint32_t e) {
-    const int n = (int)(e & 4095u);
-    return TileAt{rn, n, -B.T.rx, B.T.rx};
-  };
   for (int k = 0; k < B.steps; k += 2) {
     if (handed) {
       // row values that go to a neighbour's input: stored before any node collides
-      const int act = cnt[s + 1];
-      for (int p = tid; p < act; p += NT) {
-        const uint32_t e = lst[p];
-        if (!(e & (kTileNorth | kTileSouth))) continue;
-        const int n = (int)(e & 4095u);
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        if (dist[q] < s + 1 || !(e[q] & (kTileNorth | kTileSouth))) continue;
         int loc[9];
-        tile_locs<true>(at(e), e, loc);
+        locs(Odd(), q, loc);
         double f[9], gs[9];
 #pragma unroll
         for (int a = 0; a < 9; a++) {
@@ -289,33 +322,41 @@ __global__ __launch_bounds__(NT) void k_tile2d(TileArgs B) {
           if constexpr (NS == 2) gs[a] = lds[loc[a]][NS - 1];
         }
         // the rule of bc_store: own slot a (or opp(a)) when the source is solid
-        tile_rows<NS>(B, e, k, f, gs, [&](int s, int a, double v, bool own_opp) {
-          lds[(e >> (11 + a)) & 1u ? loc[a] : (own_opp ? OPP(a) : a) * rn + n][s ? NS - 1 : 0] = v;
+        tile_rows<NS>(B, e[q], k, f, gs, [&](int c, int a, double v, bool own_opp) {
+          const int own = (own_opp ? OPP(a) : a) * rn + (int)(e[q] & 4095u);
+          lds[(e[q] >> (11 + a)) & 1u ? loc[a] : own][c ? NS - 1 : 0] = v;
         });
       }
       __syncthreads();
     }
-    const int odd = cnt[s + B.shrink - 1];
-    for (int p = tid; p < odd; p += NT) {
-      const uint32_t e = lst[p];
-      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, at(e), 0, WALSH ? A.ns[g[e & 4095u]] : 0., e, rows && !handed, k);
-    }
+#pragma unroll
+    for (int q = 0; q < PER; q++)
+      if (dist[q] >= s + B.shrink - 1) {
+        int loc[9];
+        locs(Odd(), q, loc);
+        tile_node<NS, SOL, WALSH, true, false>(B, A, lds, loc, 0, ns[q], e[q], rows && !handed, k);
+      }
     s += B.shrink;
     __syncthreads();
     if (k + 2 < B.steps) {
-      const int even = cnt[s];
-      for (int p = tid; p < even; p += NT) {
-        const uint32_t e = lst[p];
-        tile_node<NS, SOL, WALSH, false, false>(B, A, lds, at(e), 0, WALSH ? A.ns[g[e & 4095u]] : 0., e, rows, k + 1);
-      }
+#pragma unroll
+      for (int q = 0; q < PER; q++)
+        if (dist[q] >= s) {
+          int loc[9];
+          locs(Even(), q, loc);
+          tile_node<NS, SOL, WALSH, false, false>(B, A, lds, loc, 0, ns[q], e[q], rows, k + 1);
+        }
       __syncthreads();
     } else {
       A.write_mv = B.A.write_mv;
-      for (int p = tid; p < core; p += NT) {
-        const uint32_t e = lst[p];
-        const int idx = g[e & 4095u];
-        tile_node<NS, SOL, WALSH, false, true>(B, A, lds, at(e), idx, WALSH ? A.ns[idx] : 0., e, rows, k + 1);
-      }
+#pragma unroll
+      for (int q = 0; q < PER; q++)
+        if (dist[q] >= B.T.halo) {
+          int loc[9];
+          locs(Even(), q, loc);
+          tile_node<NS, SOL, WALSH, false, true>(B, A, lds, loc, KEEP ? idx[q] : g[e[q] & 4095u], ns[q], e[q], rows,
+                                                 k + 1);
+        }
     }
   }
 }
@@ -424,10 +465,13 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep2d(TileArgs B, SweepGeo S,
     if (en.x < 0) return;
     const TileAt P{plane, s0 * stride + n, (sm - s0) * stride, (sp - s0) * stride};
     const double ns = WALSH ? nsl[s0 * stride + n] : 0.;
+    int loc[9];
+    if (!stores && !(stage & 1)) tile_locs<true>(P, (uint32_t)en.y, loc);
+    else tile_locs<false>(P, (uint32_t)en.y, loc);
     if (!stores && !(stage & 1))
-      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, P, en.x, ns, (uint32_t)en.y, rows, stage);
-    else if (stores || last) tile_node<NS, SOL, WALSH, false, true>(B, A, lds, P, en.x, ns, (uint32_t)en.y, rows, stage);
-    else tile_node<NS, SOL, WALSH, false, false>(B, A, lds, P, en.x, ns, (uint32_t)en.y, rows, stage);
+      tile_node<NS, SOL, WALSH, true, false>(B, A, lds, loc, en.x, ns, (uint32_t)en.y, rows, stage);
+    else if (stores || last) tile_node<NS, SOL, WALSH, false, true>(B, A, lds, loc, en.x, ns, (uint32_t)en.y, rows, stage);
+    else tile_node<NS, SOL, WALSH, false, false>(B, A, lds, loc, en.x, ns, (uint32_t)en.y, rows, stage);
   };
   if (stage == 3) {
     lds_barrier();
