@@ -7,9 +7,10 @@
 // that the bus and the copies (for a fresh array mostly the cost of its first
 // touch) run together.
 //
-// The slots are one allocation per process, made on first use, at most
-// kStageSlots * kStageSlot bytes, released with the last handle.  A transfer
-// holds them from start to end; transfers of other threads wait.
+// Slots and threads are one set per process, made on first use, at most
+// kStageSlots * kStageSlot bytes and kStageSlots - 1 threads, released with the
+// last handle.  A transfer holds them from start to end; transfers of other
+// threads wait.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -17,8 +18,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
+#include <functional>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -26,20 +28,81 @@ namespace lbm {
 
 constexpr int kStageSlots = 8;              // slots, and host threads at most
 constexpr size_t kStageSlot = 2u << 20;     // bytes of a slot
-// One thread (the caller's first) for each MiB: a thread costs about 20 us
-// to start and moves a MiB in 60 us (fields of 1.3 MB: 0.062 ms alone; 2.9 MB:
-// 0.109 ms with two, 0.13 alone, 0.147 with eight; 26 MB: 0.95 with eight).
+// One thread (the caller's first) for each MiB: a thread moves a MiB in 60 us
+// (fields of 1.3 MB: 0.062 ms alone; 2.9 MB: 0.109 ms with two, 0.13 alone).
+// 1 GB of fields: 20 GB/s with two threads, 33 with four, 44 with six, 47 with
+// eight.
 constexpr size_t kStageAlone = 1u << 20;
 
 struct Stage {
-  std::mutex mu;
+  std::mutex mu;   // held for a whole transfer
   int users = 0;
   char *buf = nullptr;
   size_t bytes = 0;
+
+  // Helper threads, started by the first transfer that wants them, asleep
+  // between transfers, ended with the last handle.  The caller works too and
+  // waits only for helpers that have begun: on a machine whose cores are all
+  // busy (a BLAS pool still spinning after the caller's last product) a
+  // thread that has to be started or joined costs a scheduler tick, 4 ms a
+  // transfer where 18 MB take 0.7.
+  std::mutex jm;
+  std::condition_variable wake, idle;
+  std::vector<std::thread> threads;
+  const std::function<void(int)> *job = nullptr;
+  int next = 0, most = 0, begun = 0;  // slots given out and to give, helpers at work
+  bool stop = false;
+
+  void helper() {
+    std::unique_lock<std::mutex> lock(jm);
+    for (;;) {
+      wake.wait(lock, [&] { return stop || (job && next < most); });
+      if (stop) return;
+      const std::function<void(int)> *const mine = job;
+      const int slot = next++;
+      begun++;
+      lock.unlock();
+      (*mine)(slot);
+      lock.lock();
+      if (--begun == 0) idle.notify_all();
+    }
+  }
+  // fn(0) here, fn(1) .. fn(workers - 1) on helpers that come in time
+  void run(const std::function<void(int)> &fn, int workers) {
+    if (workers > 1) {
+      std::lock_guard<std::mutex> lock(jm);
+      try {
+        while ((int)threads.size() < workers - 1) threads.emplace_back([this] { helper(); });
+      } catch (const std::exception &) {
+        // fewer helpers: the others take their share
+      }
+      job = &fn;
+      next = 1;
+      most = workers;
+    }
+    if (workers > 1) wake.notify_all();
+    fn(0);
+    if (workers > 1) {
+      std::unique_lock<std::mutex> lock(jm);
+      job = nullptr;
+      idle.wait(lock, [&] { return begun == 0; });
+    }
+  }
+  void end_threads() {
+    {
+      std::lock_guard<std::mutex> lock(jm);
+      stop = true;
+    }
+    wake.notify_all();
+    for (auto &t : threads) t.join();
+    threads.clear();
+    stop = false;
+  }
 };
+// never destroyed: a process may end with handles open
 inline Stage &stage() {
-  static Stage s;
-  return s;
+  static Stage *const s = new Stage;
+  return *s;
 }
 inline void stage_join() {
   std::lock_guard<std::mutex> lock(stage().mu);
@@ -49,6 +112,7 @@ inline void stage_leave() {
   Stage &s = stage();
   std::lock_guard<std::mutex> lock(s.mu);
   if (--s.users > 0) return;
+  s.end_threads();
   if (s.buf) (void)hipHostFree(s.buf);
   s.buf = nullptr;
   s.bytes = 0;
@@ -136,22 +200,7 @@ hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream,
     }
     if (r != hipSuccess) bad.store((int)r);
   };
-  {
-    // joins on every way out of this block
-    struct Pool {
-      std::vector<std::thread> t;
-      ~Pool() {
-        for (auto &x : t) x.join();
-      }
-    } pool;
-    try {
-      pool.t.reserve(workers);
-      for (int w = 1; w < workers; w++) pool.t.emplace_back(work, w);
-    } catch (const std::exception &) {
-      // fewer threads: the others take their pieces
-    }
-    work(0);
-  }
+  s.run(work, workers);
   // the slots are free again once the GPU has read them
   e = hipStreamSynchronize(stream);
   return bad.load() != (int)hipSuccess ? (hipError_t)bad.load() : e;
