@@ -162,6 +162,7 @@ struct StepArgs {
   int nf;         // fluid nodes
   int nblk8;      // launched blocks / 8
   const int *bmap; // node block of each launched block (-1: none), or null
+  const uint32_t *ltab;  // [Q-1][nf] odd_locs of every node (OFF32), or null
   double *mv;     // [nsubs][1+D][nf]
   int write_mv;
   int solute_on;
@@ -226,15 +227,37 @@ __device__ __forceinline__ void odd_locs(const Geo &G, int x, int i, int j, int 
   }
 }
 
-template <int Q, uint32_t U, bool ODD>
-__device__ __forceinline__ void step_locs(const Geo &G, int x, uint32_t (&loc)[Q]) {
-  if constexpr (ODD) {
+// Small lattices keep the odd step's locations in a table: one level of
+// coalesced loads instead of two dependent ones (node index, row words) and
+// the rank arithmetic.  us per step, computed -> table: 20 x 24 x 22 flow +
+// solute FP64 4.22 -> 3.83, 40 x 36 x 44 6.40 -> 5.99, flow 4.79 -> 4.38, FP32
+// 5.28 -> 4.86; at 105k fluid nodes the 4 (Q - 1) bytes a node begin to cost
+// what they save.
+constexpr int kTableNodes = 1 << 16;
+
+template <int Q, uint32_t U, bool ODD, bool TAB = false>
+__device__ __forceinline__ void step_locs(const Geo &G, const uint32_t *ltab, int nf, int x, uint32_t (&loc)[Q]) {
+  if constexpr (!ODD) {
+    even_locs<Q, U>(x, loc);
+  } else if constexpr (TAB) {
+    loc[0] = loc_at<Q, U>(0, (uint32_t)x);
+#pragma unroll
+    for (int a = 1; a < Q; a++) loc[a] = ltab[(a - 1) * nf + x];
+  } else {
     int i, j, k;
     coords<Q == 9 ? 2 : 3>(G, (uint32_t)G.node[x], i, j, k);
     odd_locs<Q, U>(G, x, i, j, k, loc);
-  } else {
-    even_locs<Q, U>(x, loc);
   }
+}
+
+template <int Q, uint32_t U>
+__global__ void k_loc_table(Geo G, int nf, uint32_t *ltab) {
+  const int x = blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= nf) return;
+  uint32_t loc[Q];
+  step_locs<Q, U, true>(G, nullptr, nf, x, loc);
+#pragma unroll
+  for (int a = 1; a < Q; a++) ltab[(a - 1) * nf + x] = loc[a];
 }
 
 // the population of component s at a location
@@ -697,7 +720,7 @@ __device__ __forceinline__ void walsh_mix(CT (&f)[Q], const CT (&fp)[Q], CT ns, 
   }
 }
 
-template <int Q, int NS, typename ST, typename CT, bool ODD, bool OFF32, bool WALSH = false>
+template <int Q, int NS, typename ST, typename CT, bool ODD, bool OFF32, bool WALSH = false, bool TAB = false>
 __global__ __launch_bounds__(kStepBlock) void k_half_step(StepArgs<ST, CT> A) {
   // node block: from the row-band map when the launch carries one, else the
   // XCD-contiguous remap
@@ -706,7 +729,7 @@ __global__ __launch_bounds__(kStepBlock) void k_half_step(StepArgs<ST, CT> A) {
   const int idx = lb * (int)blockDim.x + (int)threadIdx.x;
   if (idx >= A.nf) return;
   uint32_t loc[Q];
-  step_locs<Q, loc_unit<NS, ST, OFF32>(), ODD>(A.G, idx, loc);
+  step_locs<Q, loc_unit<NS, ST, OFF32>(), ODD, TAB>(A.G, A.ltab, A.nf, idx, loc);
   CT f[Q], u[3];
   CT ns = (CT)0, kns = (CT)1;
   if constexpr (WALSH) {
