@@ -1229,8 +1229,8 @@ int tile_launch(lbm_handle *h, const TileArgs &B) {
 // Steps per launch and core of k_tile2d for the handle's lattice.
 // A lattice that one tile per CU covers takes the smallest square core that
 // does: its time is launch (2 us) and per-step latency (1 us), so it takes
-// as many steps a launch as the halo's work allows, 8 (two components with
-// cores above 12: 6; cores above 20: 4).  Measured when the kernel was first
+// as many steps a launch as the halo's work allows, 8 (flow with cores up to
+// 10: 10; two components with cores above 12: 6).  Measured when the kernel was first
 // tuned, us per step, flow | flow + solute with row conditions: 128^2 8 x 8
 // cores 1.54 | 1.94 (4 steps 1.74 | 2.06), 200 x 170 12 x 12 cores 1.64 | 2.07
 // (4 steps 1.9 | 2.19), 300 x 310 20 x 20 cores 1.97 with 8 steps | 2.71 with 6
@@ -1240,14 +1240,17 @@ int tile_launch(lbm_handle *h, const TileArgs &B) {
 // CU holds two (1000^2 10.8, 2100 x 1900 44.9 us; 30 x 30 cores with 8 steps
 // 11.3, 43.7), flow + solute in the largest square core that LDS holds, 25 x
 // 25 (19.7, 85.3 us; 32 x 16 20.4, 91.4; 20 x 20 with 6 steps 22.2, 94.9).
-// Now, with entries in registers: 1.30 | 1.77, 1.38 | 1.91, 1.93 | 2.67 us;
-// 1000^2 9.8 | 18.2, 2100 x 1900 41.0 us.
+// Now, with entries in registers: 1.26 (10 steps; 8: 1.31) | 1.77, 1.38 | 1.91,
+// 1.82 | 2.61 us; 413 x 307 flow, 23 x 23 cores with 8 steps, 2.05 (32 x 16
+// cores with 4: 3.02); 1000^2 9.8 | 18.2, 2100 x 1900 41.0 us.
 void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy) {
   const int ns = h->p.nsubs;
   const double per_cu = (double)h->N / h->cus;
   int s = 8;
   while ((double)s * s < per_cu && s < 64) s++;
-  steps = s <= 12 ? 8 : (s <= 20 ? (ns == 1 ? 8 : 6) : 4);
+  // most one-tile cores: what LDS holds with 8 (flow) and 6 steps
+  const int one = ns == 1 ? 29 : 20;
+  steps = s <= 10 && ns == 1 ? 10 : (s <= 12 ? 8 : (s <= one ? (ns == 1 ? 8 : 6) : 4));
   auto most = [&](int k) {  // largest square core of k steps
     int c = 0;
     const int halo = shrink * k / 2;
@@ -1257,7 +1260,7 @@ void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy) {
   };
   if (most(steps) < s) steps = 4;
   cx = cy = std::min(s, most(steps));
-  if (s > 20 && ns == 1) {
+  if (s > one && ns == 1) {
     cx = 32;
     cy = 16;
   }
@@ -1370,7 +1373,9 @@ bool solute_on(const lbm_handle *h, int t) {
 int tile_steps(const lbm_handle *h, int n) {
   const int t1 = h->time + 1;
   if (!(t1 & 1)) return 0;
-  int len = std::min(n, h->tile.steps) & ~1;
+  // as few launches as possible, of nearly equal length
+  const int even = n & ~1, launches = (even + h->tile.steps - 1) / h->tile.steps;
+  int len = launches ? ((even + launches - 1) / launches + 1) & ~1 : 0;
   while (len > 0) {
     bool same = true;
     for (int q = 1; q < len; q++) same = same && solute_on(h, t1 + q) == solute_on(h, t1);
@@ -2156,7 +2161,10 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
       h->F = q == 1 ? first : sp[q - 1];
       const bool fz = zface_fused(h, t);
       J.A = make_args<double, double>(h);
-      J.amap = h->amap;
+      // few nodes: every block is resident at once, and in node order their
+      // lines are shared sooner (48 x 40 x 60 14.3 -> 13.6 us a step, 72 x 68 x
+      // 80 33.6 -> 32.8; 128^3 136 -> 143, which keeps the bands)
+      J.amap = h->nf < kFewNodes ? nullptr : h->amap;
       J.A.nblk8 = h->anblk8;
       if (fz) set_zb(h, J.A);
       J.L = L;

@@ -37,7 +37,6 @@
 namespace lbm {
 
 constexpr int kTileSteps = 16;   // most steps of one launch
-constexpr int kTileHalo = 24;    // widest halo: 3 nodes per pair of steps
 constexpr int kTileRegion = 2048;  // most region nodes (below 4096: 12-bit region index)
 
 // list entry of a fluid region node: region index, bit 12 + a - 1 set when
