@@ -867,13 +867,15 @@ extern "C" int lbm_destroy(lbm_handle *h) {
 static int build_lattice(lbm_handle *h, const uint8_t *mask) {
   const long N = h->N, E = h->E;
   const int L = h->L;
-  h->fid.assign(N, -1);
-  h->node_host.clear();
-  for (long n = 0; n < N; n++)
-    if (mask[n] != 1) {
-      h->fid[n] = (int)h->node_host.size();
-      h->node_host.push_back((int)n);
-    }
+  long fluid = 0;
+  for (long n = 0; n < N; n++) fluid += mask[n] != 1;
+  h->fid.resize(N);
+  h->node_host.resize(fluid);
+  int next = 0;
+  for (long n = 0; n < N; n++) {
+    h->fid[n] = mask[n] != 1 ? next : -1;
+    if (mask[n] != 1) h->node_host[next++] = (int)n;
+  }
   const int nf = (int)h->node_host.size();
   h->nf = nf;
   if (nf == 0) return lbm_fail("lattice has no fluid node");

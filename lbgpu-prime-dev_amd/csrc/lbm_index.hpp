@@ -317,13 +317,13 @@ inline void fill_row_words(const int *fid, long rows, int ni, RowWord *rw) {
   for (long r = 0; r < rows; r++)
     for (int w = 0; w < W; w++) {
       RowWord &x = rw[r * W + w];
-      x.bits = 0;
       x.base = (int32_t)count;
-      for (int b = 0; b < 64 && 64 * w + b < ni; b++)
-        if (fid[r * ni + 64 * w + b] >= 0) {
-          x.bits |= 1ull << b;
-          count++;
-        }
+      const int n = ni - 64 * w < 64 ? ni - 64 * w : 64;
+      const int *f = fid + r * ni + 64 * w;
+      uint64_t bits = 0;
+      for (int b = 0; b < n; b++) bits |= (uint64_t)(f[b] >= 0) << b;
+      x.bits = bits;
+      count += popc64(bits);
       const int pc = w > 0 ? 64 * w - 1 : ni - 1;
       const int nc = 64 * (w + 1) < ni ? 64 * (w + 1) : 0;
       const int pid = fid[r * ni + pc], nid = fid[r * ni + nc];
