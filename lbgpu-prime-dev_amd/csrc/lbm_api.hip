@@ -634,14 +634,26 @@ int launch_bcs(lbm_handle *h, int phase, int t) {
         }
       }
     } else {
+      ZfaceArgs Z[2];
+      ZfaceList l[2];
       for (int top = 0; top < 2; top++) {
-        ZfaceArgs Z = zface_args(h, top);
-        if (NS != 2) Z.conc = kCNone;
-        if (Z.flow == kZNone && Z.conc == kCNone) continue;
-        B.list = top ? h->face_hi : h->face_lo;
-        B.n = top ? h->n_hi : h->n_lo;
-        if (!B.n) continue;
-        hipLaunchKernelGGL((k_bc_zface<NS, ST, CT>), dim3(blocks_for(B.n)), dim3(256), 0, h->stream, B, Z);
+        Z[top] = zface_args(h, top);
+        if (NS != 2) Z[top].conc = kCNone;
+        const bool any = Z[top].flow != kZNone || Z[top].conc != kCNone;
+        l[top].list = top ? h->face_hi : h->face_lo;
+        l[top].n = any ? (top ? h->n_hi : h->n_lo) : 0;
+        l[top].blocks = (int)blocks_for(l[top].n);
+      }
+      if (p.nk == 1 && l[0].n && l[1].n) {
+        // the two faces are the same plane: one after the other
+        const ZfaceList none = {nullptr, 0, 0};
+        hipLaunchKernelGGL((k_bc_zface<NS, ST, CT>), dim3(l[0].blocks), dim3(256), 0, h->stream, B, Z[0], Z[1], l[0],
+                           none);
+        hipLaunchKernelGGL((k_bc_zface<NS, ST, CT>), dim3(l[1].blocks), dim3(256), 0, h->stream, B, Z[0], Z[1], none,
+                           l[1]);
+      } else if (l[0].n || l[1].n) {
+        hipLaunchKernelGGL((k_bc_zface<NS, ST, CT>), dim3(l[0].blocks + l[1].blocks), dim3(256), 0, h->stream, B, Z[0],
+                           Z[1], l[0], l[1]);
       }
     }
     HIP_OK(hipGetLastError());
