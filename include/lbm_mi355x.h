@@ -153,14 +153,17 @@ int lbm_set_solids(lbm_handle *h, const uint8_t *mask);
 int lbm_set_ns(lbm_handle *h, const double *ns);
 
 /* f H2D / D2H per subs (src/lbgpu_prime.cu:317-343, :874-900).  Solid
- * nodes are not stored: download returns 0 there. */
+ * nodes are not stored: download returns 0 there.  These calls, the macro
+ * download and the samples move data through pinned host memory (at most
+ * 16 MiB) and up to seven host threads that all handles of the process share:
+ * transfers of several threads take turns; the last lbm_destroy releases
+ * both. */
 int lbm_upload_f(lbm_handle *h, int subs, const double *f1d);
 int lbm_download_f(lbm_handle *h, int subs, double *f1d);
 /* lbm_download_f without any allocation (no counterpart in the reference;
  * for callers that cannot allocate device or host memory during a run, such
  * as serving loops that checkpoint the state): the same [Q][N] values, staged
- * in a static device array of the library instead of a buffer allocated per
- * call.  Q x N may not exceed 8,388,608 (64 MiB of FP64: D3Q19 lattices up to
+ * in a static device array of the library instead of the pinned memory above.  Q x N may not exceed 8,388,608 (64 MiB of FP64: D3Q19 lattices up to
  * 441,505 nodes, D2Q9 up to 932,067); larger lattices are rejected with an
  * error.  Every handle on one GPU shares that GPU's array, and each call
  * rewrites all of the Q x N elements it returns: calls that overlap on one
@@ -184,7 +187,14 @@ int lbm_get_time(const lbm_handle *h, int *time);
  * concentration (pest_output_flag_c, :305-334); other nonzero values act as
  * LBM_MACRO_FRAME. */
 int lbm_step(lbm_handle *h, int write_macro);
-/* nsteps steps, macroscopic write on the last one if write_macro_last */
+/* nsteps steps, macroscopic write on the last one if write_macro_last.  The
+ * results are those of nsteps calls of lbm_step.  With FP64 storage and
+ * collision a D2Q9 lattice runs several steps per launch, for which the first
+ * run of two steps or more allocates a second population array, and a D3Q19
+ * lattice below 65,536 fluid nodes reads its neighbours' locations from a
+ * table that the first run of 128 steps or more allocates; without the
+ * memory the steps run without them.  lbm_set_solids and lbm_destroy release
+ * both. */
 int lbm_run(lbm_handle *h, int nsteps, int write_macro_last);
 
 /* The two half-steps on their own, at an explicit time (a1 / a2):
