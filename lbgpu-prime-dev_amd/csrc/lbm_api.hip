@@ -563,6 +563,13 @@ int launch_half(lbm_handle *h, int odd, int t, int write_mv, bool fuse_bc = fals
         hipLaunchKernelGGL((k_half_step<Q, NS, ST, CT, false, true, true>), grid, block, lds, h->stream, A);
       else
         hipLaunchKernelGGL((k_half_step<Q, NS, ST, CT, false, false, true>), grid, block, lds, h->stream, A);
+    } else if (odd && A.Fo != A.F) {
+      // out of place: objective runs, FP64 flow + solute only
+      if constexpr (Q == 19 && NS == 2 && sizeof(ST) == 8 && sizeof(CT) == 8) {
+        auto *const fn = off32 ? k_half_step<Q, NS, ST, CT, true, true, false, false, true>
+                               : k_half_step<Q, NS, ST, CT, true, false, false, false, true>;
+        hipLaunchKernelGGL(fn, grid, block, lds, h->stream, A);
+      } else return lbm_fail("out-of-place step of this lattice");
     } else if (odd && off32) {
       if constexpr (Q == 19)
         if (A.ltab) {
@@ -2159,8 +2166,9 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
       const dim3 grid = (t & 1) ? odd_grid(h, A, bs) : dim3(8 * A.nblk8), block(bs);
       Prof pr(h, (t & 1) ? 0 : 1);
       if (t & 1) {
-        if (off32) hipLaunchKernelGGL((k_half_step<19, 2, double, double, true, true>), grid, block, lds, h->stream, A);
-        else hipLaunchKernelGGL((k_half_step<19, 2, double, double, true, false>), grid, block, lds, h->stream, A);
+        auto *const fn = off32 ? k_half_step<19, 2, double, double, true, true, false, false, true>
+                               : k_half_step<19, 2, double, double, true, false, false, false, true>;
+        hipLaunchKernelGGL(fn, grid, block, lds, h->stream, A);
       } else {
         if (off32) hipLaunchKernelGGL((k_half_step<19, 2, double, double, false, true>), grid, block, lds, h->stream, A);
         else hipLaunchKernelGGL((k_half_step<19, 2, double, double, false, false>), grid, block, lds, h->stream, A);

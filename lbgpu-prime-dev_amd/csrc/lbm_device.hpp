@@ -720,7 +720,15 @@ __device__ __forceinline__ void walsh_mix(CT (&f)[Q], const CT (&fp)[Q], CT ns, 
   }
 }
 
-template <int Q, int NS, typename ST, typename CT, bool ODD, bool OFF32, bool WALSH = false, bool TAB = false>
+// OUT: the state is stored elsewhere (Fo != F), for the FP64 flow + solute
+// odd step (the adjoint's forward replay, the kept steps of an objective run).
+// It does not write back the lines it reads: streaming loads leave the caches
+// to the lines it writes and the next step reads (128^3 flow + solute, ordinary
+// -> streaming: odd 109.4 -> 103.3, the even step after it 92.3 -> 81.4 us).  A kernel of its own:
+// chosen by a branch on Fo == F, the compiler merges both sides' loads, which
+// then have the same addresses, into ordinary ones.
+template <int Q, int NS, typename ST, typename CT, bool ODD, bool OFF32, bool WALSH = false, bool TAB = false,
+          bool OUT = false>
 __global__ __launch_bounds__(kStepBlock) void k_half_step(StepArgs<ST, CT> A) {
   // node block: from the row-band map when the launch carries one, else the
   // XCD-contiguous remap
@@ -739,17 +747,7 @@ __global__ __launch_bounds__(kStepBlock) void k_half_step(StepArgs<ST, CT> A) {
   }
   if (NS == 2 && A.solute_on) {
     CT g[Q];
-    if constexpr (ODD && NS == 2 && sizeof(ST) == 8 && sizeof(CT) == 8) {
-      // An out-of-place odd step (the adjoint's forward replay, the kept
-      // steps of an objective run) does not write back the lines it reads:
-      // streaming loads leave the L2 to the lines it writes (128^3 flow +
-      // solute: replay 202 -> 188 ms per sweep, objective run with kept
-      // states 188 -> 183 ms; in-place steps unchanged).
-      if (A.Fo != A.F) gather2<Q, ST, CT, ODD, OFF32, true>(A, loc, f, g);
-      else gather2<Q, ST, CT, ODD, OFF32>(A, loc, f, g);
-    } else {
-      gather2<Q, ST, CT, ODD, OFF32>(A, loc, f, g);
-    }
+    gather2<Q, ST, CT, ODD, OFF32, OUT>(A, loc, f, g);
     if constexpr (Q == 19)
       if (zface_node<Q>(A, idx)) zface_fix<ST, CT, true>(A, idx, f, g);
     if constexpr (WALSH) {
