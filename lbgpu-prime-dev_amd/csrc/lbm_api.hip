@@ -500,7 +500,7 @@ int upload_band_map(lbm_handle *h, int bs, long nb, long per, int **dst) {
 // the odd half-step's workgroup size for the handle's kind
 int odd_block(const lbm_handle *h) {
   return dispatch(h, [&]<int Q, int NS, typename ST, typename CT>() -> int {
-    return step_shape<NS, ST, CT>(true, h->nf).block;
+    return step_shape<Q, NS, ST, CT>(true, h->nf).block;
   });
 }
 
@@ -547,7 +547,7 @@ int launch_half(lbm_handle *h, int odd, int t, int write_mv, bool fuse_bc = fals
     A.solute_on = NS == 2 && t >= h->p.sigma_t_on && t <= h->p.sigma_t_off;
     Prof pr(h, odd ? 0 : 1);
     const bool off32 = !h->off64 && (size_t)h->tiles * NS * Q * kTile * sizeof(ST) <= 0xffffffffull;
-    const StepShape shape = step_shape<NS, ST, CT>(odd, h->nf);
+    const StepShape shape = step_shape<Q, NS, ST, CT>(odd, h->nf);
     const int bs = shape.block;
     A.nblk8 = (int)((blocks_for(h->nf, bs) + 7) / 8);
     const dim3 grid = odd ? odd_grid(h, A, bs) : dim3(8 * A.nblk8), block(bs);
@@ -2159,7 +2159,7 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
       if (fz) set_zb(h, A);
       A.Fo = (double *)rp[q];
       A.solute_on = 1;
-      const StepShape shape = step_shape<2, double, double>(t & 1, h->nf);
+      const StepShape shape = step_shape<19, 2, double, double>(t & 1, h->nf);
       const int bs = shape.block;
       const size_t lds = step_lds_pad(shape.per_cu, h->lds_cu);
       A.nblk8 = (int)((blocks_for(h->nf, bs) + 7) / 8);

@@ -48,13 +48,15 @@ constexpr int kBlock = 256;
 //     (512, 256 -> 256, 128 capped at 4)
 //   FP32, FP64 collision  5.9 10.7 49.3 165.4 356.1 -> 5.6 10.3 same (64, 128)
 // FP16 storage keeps 256 threads uncapped: 64 and 128 threads measured within
-// 1 % below 3.2M nodes and 2-4 % slower at 7.0M, caps 3-70 % slower.
+// 1 % below 3.2M nodes and 2-4 % slower at 7.0M, caps 3-70 % slower.  D2Q9 waves
+// carry half the bytes and want more of them: FP32 even steps stay at 256
+// uncapped (flow, 1088 x 1224 15.4 us a step; 128 capped at 4: 16.4).
 constexpr int kFewNodes = 1 << 18;
 constexpr int kStepBlock = 256;  // largest workgroup of a half-step
 struct StepShape {
   int block, per_cu;
 };
-template <int NS, typename ST, typename CT>
+template <int Q, int NS, typename ST, typename CT>
 StepShape step_shape(bool odd, int nf) {
   constexpr bool f64 = sizeof(ST) == 8 && sizeof(CT) == 8, f32_f64 = NS == 2 && sizeof(ST) == 4 && sizeof(CT) == 8;
   if (sizeof(ST) == 2) return {256, 0};
@@ -62,7 +64,7 @@ StepShape step_shape(bool odd, int nf) {
   if (f64 && NS == 2) return odd ? StepShape{64, 6} : StepShape{128, 2};
   if (f64) return odd ? StepShape{256, 3} : StepShape{128, 3};
   if (f32_f64) return odd ? StepShape{64, 0} : StepShape{128, 0};
-  return odd ? StepShape{256, 0} : StepShape{128, 4};
+  return odd || Q == 9 ? StepShape{256, 0} : StepShape{128, 4};
 }
 // LDS a half-step workgroup reserves to cap the workgroups per CU
 inline size_t step_lds_pad(int per_cu, int lds_per_cu) {
