@@ -13,7 +13,7 @@
 // threads wait.
 #pragma once
 
-#include <hip/hip_runtime.h>
+#include <hip/hip_runtime_api.h>
 #include <string.h>
 
 #include <algorithm>
@@ -126,7 +126,9 @@ inline hipError_t stage_hold(Stage &s, size_t bytes) {
   s.bytes = 0;
   // small transfers share one slot, others get all of them
   const size_t want = bytes <= kStageSlot ? kStageSlot : kStageSlot * kStageSlots;
-  const hipError_t e = hipHostMalloc((void **)&s.buf, want, hipHostMallocPortable);
+  // coherent, whatever HIP_HOST_COHERENT says: kernels and host threads read
+  // and write a slot in turn while the process runs on
+  const hipError_t e = hipHostMalloc((void **)&s.buf, want, hipHostMallocPortable | hipHostMallocCoherent);
   if (e != hipSuccess) s.buf = nullptr;
   else s.bytes = want;
   return e;
@@ -177,7 +179,10 @@ hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream,
   std::lock_guard<std::mutex> lock(s.mu);
   if ((e = stage_hold(s, slot * workers)) != hipSuccess) return e;
   for (int w = 0; w < workers; w++)
-    if (!events[w] && (e = hipEventCreateWithFlags(&events[w], hipEventDisableTiming)) != hipSuccess) return e;
+    // the host reads the slot behind the event: its writes are released to the system
+    if (!events[w] &&
+        (e = hipEventCreateWithFlags(&events[w], hipEventDisableTiming | hipEventReleaseToSystem)) != hipSuccess)
+      return e;
   std::atomic<int> next{0}, bad{(int)hipSuccess};
   auto work = [&](int w) {
     hipError_t r = hipSetDevice(dev);
