@@ -157,7 +157,7 @@ int lbm_set_ns(lbm_handle *h, const double *ns);
  * download and the samples move data through pinned host memory (at most
  * 16 MiB) and up to seven host threads that all handles of the process share:
  * transfers of several threads take turns; the last lbm_destroy releases
- * both. */
+ * both.  Where the system pins no memory they go through ordinary copies. */
 int lbm_upload_f(lbm_handle *h, int subs, const double *f1d);
 int lbm_download_f(lbm_handle *h, int subs, double *f1d);
 /* lbm_download_f without any allocation (no counterpart in the reference;

@@ -7,7 +7,9 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -177,6 +179,7 @@ struct lbm_handle {
 namespace {
 
 constexpr int kRedBlocks = 512;
+constexpr int kRedValues = 12 * kRedBlocks;  // doubles of the reduction buffer
 // largest LX: the row words hold the ranks of a row's nodes next to a word
 // as 16-bit offsets from the word's base, which are at most LX
 constexpr int kMaxLX = 32767;
@@ -852,7 +855,7 @@ extern "C" int lbm_create(const lbm_params *p, lbm_handle **out) {
       return lbm_fail("inlet map upload failed");
     }
   }
-  if (hipMalloc(&h->red, sizeof(double) * 12 * kRedBlocks) != hipSuccess ||
+  if (hipMalloc(&h->red, sizeof(double) * kRedValues) != hipSuccess ||
       hipMalloc(&h->flux_dev, sizeof(double) * (2 + 2 * kFluxBlocks)) != hipSuccess) {
     lbm_destroy(h);
     return lbm_fail("hipMalloc failed");
@@ -984,11 +987,14 @@ extern "C" int lbm_set_solids(lbm_handle *h, const uint8_t *mask) {
   return 0;
 }
 
-// Moves the pieces of a transfer through pinned memory (lbm_stage.hpp)
+// Moves the pieces of a transfer through pinned memory (lbm_stage.hpp), or
+// where there is none through the handle's reduction buffer
 template <typename Device, typename Host>
 static int move_pieces(lbm_handle *h, int comps, bool up, Device &&device, Host &&host) {
   try {
-    const hipError_t e = staged(pieces_of(comps, h->N), up, h->stream, h->stage_ev, device, host);
+    bool pinned;
+    hipError_t e = staged(pieces_of(comps, h->N), up, h->stream, h->stage_ev, device, host, pinned);
+    if (!pinned) e = unpinned(pieces_of(comps, h->N, kRedValues), up, h->stream, h->red, kRedValues, device, host);
     if (e != hipSuccess) return lbm_fail("transfer: %s", hipGetErrorString(e));
   } catch (const std::exception &x) {
     return lbm_fail("transfer: %s", x.what());
@@ -1558,16 +1564,28 @@ extern "C" int lbm_sample_macro(lbm_handle *h, int subs, int npts, const long *n
   if (!npts) return sync(h);
   Stage &st = stage();
   std::lock_guard<std::mutex> lock(st.mu);
-  HIP_OK(stage_hold(st, kStageSlot));
-  // a slot holds the values of `most` points, then their compact indices
-  const int most = (int)(kStageSlot / (sizeof(double) * comps + sizeof(int)));
-  double *val = (double *)st.buf;
-  int *at = (int *)(val + (size_t)most * comps);
+  // room for the values of `most` points and then their compact indices, in
+  // pinned memory that the kernel reads and writes, or else on the device
+  const bool pinned = stage_hold(st, kStageSlot);
+  const size_t room = pinned ? kStageSlot : sizeof(double) * kRedValues;
+  const int most = (int)std::min<size_t>(npts, room / (sizeof(double) * comps + sizeof(int)));
+  std::unique_ptr<char[]> copy(pinned ? nullptr : new (std::nothrow) char[room]);
+  if (!pinned && !copy) return lbm_fail("lbm_sample_macro: out of memory");
+  const size_t index_at = sizeof(double) * comps * (size_t)most;
+  char *const dev = pinned ? st.buf : (char *)h->red;
+  char *const host = pinned ? st.buf : copy.get();
+  double *val = (double *)host;
+  int *at = (int *)(host + index_at);
   for (int q0 = 0; q0 < npts; q0 += most) {
     const int n = std::min(most, npts - q0);
     for (int q = 0; q < n; q++) at[q] = h->fid[nodes[q0 + q]];
-    hipLaunchKernelGGL(k_sample_field, dim3(blocks_for(n)), dim3(256), 0, h->stream, mv, nf, comps, at, n, val);
+    if (!pinned)
+      HIP_OK(hipMemcpyAsync(dev + index_at, at, (size_t)n * sizeof(int), hipMemcpyHostToDevice, h->stream));
+    hipLaunchKernelGGL(k_sample_field, dim3(blocks_for(n)), dim3(256), 0, h->stream, mv, nf, comps,
+                       (const int *)(dev + index_at), n, (double *)dev);
     HIP_OK(hipGetLastError());
+    if (!pinned)
+      HIP_OK(hipMemcpyAsync(val, dev, (size_t)n * comps * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     HIP_OK(hipStreamSynchronize(h->stream));
     memcpy(out + (long)q0 * comps, val, (size_t)n * comps * sizeof(double));
   }

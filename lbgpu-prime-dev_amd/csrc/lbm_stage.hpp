@@ -7,6 +7,9 @@
 // that the bus and the copies (for a fresh array mostly the cost of its first
 // touch) run together.
 //
+// Without pinned memory (the system refuses to pin more) transfers go through a
+// small device buffer of the handle and ordinary copies instead.
+//
 // Slots and threads are one set per process, made on first use, at most
 // kStageSlots * kStageSlot bytes and kStageSlots - 1 threads, released with the
 // last handle.  A transfer holds them from start to end; transfers of other
@@ -118,9 +121,10 @@ inline void stage_leave() {
   s.bytes = 0;
 }
 
-// at least `bytes` (up to all slots) of pinned memory; s.mu is held
-inline hipError_t stage_hold(Stage &s, size_t bytes) {
-  if (s.bytes >= bytes) return hipSuccess;
+// at least `bytes` (up to all slots) of pinned memory; false when the system
+// gives none; s.mu is held
+inline bool stage_hold(Stage &s, size_t bytes) {
+  if (s.bytes >= bytes) return true;
   if (s.buf) (void)hipHostFree(s.buf);
   s.buf = nullptr;
   s.bytes = 0;
@@ -129,9 +133,13 @@ inline hipError_t stage_hold(Stage &s, size_t bytes) {
   // coherent, whatever HIP_HOST_COHERENT says: kernels and host threads read
   // and write a slot in turn while the process runs on
   const hipError_t e = hipHostMalloc((void **)&s.buf, want, hipHostMallocPortable | hipHostMallocCoherent);
-  if (e != hipSuccess) s.buf = nullptr;
-  else s.bytes = want;
-  return e;
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    s.buf = nullptr;
+    return false;
+  }
+  s.bytes = want;
+  return true;
 }
 
 // One piece of a transfer: nc components of nn nodes from node n0, at most a
@@ -142,9 +150,8 @@ struct Piece {
   long n0, nn;
 };
 
-// the pieces of comps components of N nodes each
-inline std::vector<Piece> pieces_of(int comps, long N) {
-  constexpr long most = (long)(kStageSlot / sizeof(double));
+// the pieces of comps components of N nodes each, at most `most` values in one
+inline std::vector<Piece> pieces_of(int comps, long N, long most = (long)(kStageSlot / sizeof(double))) {
   std::vector<Piece> v;
   if (N <= most) {
     const int group = (int)std::min<long>(comps, std::max<long>(1, most / N));
@@ -158,10 +165,12 @@ inline std::vector<Piece> pieces_of(int comps, long N) {
 
 // Moves all pieces: device(piece, slot) launches on `stream` and returns a
 // hipError_t, host(piece, slot) copies; up: host memory to the GPU.  events:
-// kStageSlots events of the caller, created here when null.
+// kStageSlots events of the caller, created here when null.  pinned: false
+// when there was no pinned memory and nothing has been moved.
 template <typename Device, typename Host>
 hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream, hipEvent_t *events, Device &&device,
-                  Host &&host) {
+                  Host &&host, bool &pinned) {
+  pinned = true;
   size_t total = 0, largest = 0;
   for (const Piece &p : pieces) {
     const size_t b = (size_t)p.nc * p.nn * sizeof(double);
@@ -177,7 +186,10 @@ hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream,
   if (e != hipSuccess) return e;
   Stage &s = stage();
   std::lock_guard<std::mutex> lock(s.mu);
-  if ((e = stage_hold(s, slot * workers)) != hipSuccess) return e;
+  if (!stage_hold(s, slot * workers)) {
+    pinned = false;
+    return hipSuccess;
+  }
   for (int w = 0; w < workers; w++)
     // the host reads the slot behind the event: its writes are released to the system
     if (!events[w] &&
@@ -209,6 +221,31 @@ hipError_t staged(const std::vector<Piece> &pieces, bool up, hipStream_t stream,
   // the slots are free again once the GPU has read them
   e = hipStreamSynchronize(stream);
   return bad.load() != (int)hipSuccess ? (hipError_t)bad.load() : e;
+}
+
+// The same without pinned memory, one piece after the other: dev is device
+// memory of `values` doubles that holds any of the pieces, and the host's side
+// of a piece is ordinary memory.
+template <typename Device, typename Host>
+hipError_t unpinned(const std::vector<Piece> &pieces, bool up, hipStream_t stream, double *dev, long values,
+                    Device &&device, Host &&host) {
+  std::vector<double> buf((size_t)values);
+  for (const Piece &p : pieces) {
+    const size_t bytes = (size_t)p.nc * p.nn * sizeof(double);
+    hipError_t e;
+    if (up) {
+      host(p, buf.data());
+      if ((e = hipMemcpyAsync(dev, buf.data(), bytes, hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
+      if ((e = device(p, dev)) != hipSuccess) return e;
+      if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
+    } else {
+      if ((e = device(p, dev)) != hipSuccess) return e;
+      if ((e = hipMemcpyAsync(buf.data(), dev, bytes, hipMemcpyDeviceToHost, stream)) != hipSuccess) return e;
+      if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
+      host(p, buf.data());
+    }
+  }
+  return hipSuccess;
 }
 
 }  // namespace lbm

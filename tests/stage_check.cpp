@@ -16,10 +16,12 @@ using namespace lbm;
 
 static std::atomic<unsigned> g_host_flags{0}, g_event_flags{0};
 static std::atomic<int> g_allocs{0}, g_frees{0}, g_events{0};
+static std::atomic<size_t> g_most{SIZE_MAX};  // bytes of the largest pinned allocation granted
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) {
   g_host_flags = flags;
+  if (n > g_most) return hipErrorOutOfMemory;
   g_allocs++;
   *p = malloc(n);
   return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -41,6 +43,10 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned flags) {
 }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t) {
+  memcpy(to, from, n);
+  return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 }
@@ -59,6 +65,7 @@ struct Array {
   int comps;
   std::vector<double> gpu, host;
   hipEvent_t ev[kStageSlots] = {};
+  bool pinned = true;
   Array(long N_, int comps_) : N(N_), comps(comps_), gpu((size_t)N_ * comps_), host((size_t)N_ * comps_) {}
   template <typename Wait>
   hipError_t move(bool up, Wait &&wait) {
@@ -78,7 +85,11 @@ struct Array {
         else memcpy(h, s, (size_t)p.nn * sizeof(double));
       }
     };
-    return staged(pieces_of(comps, N), up, nullptr, ev, device, copy);
+    const hipError_t e = staged(pieces_of(comps, N), up, nullptr, ev, device, copy, pinned);
+    if (pinned) return e;
+    constexpr long room = 777;  // values of the handle's buffer
+    double dev[room];
+    return unpinned(pieces_of(comps, N, room), up, nullptr, dev, room, device, copy);
   }
   hipError_t move(bool up) {
     return move(up, [] {});
@@ -105,9 +116,29 @@ static void coherent() {
   CHECK(g_allocs == g_frees);
 }
 
+// a system that pins no more memory, or none of the size wanted: the transfer
+// goes without, and with again once there is some
+static void refused() {
+  stage_join();
+  for (long N : {1L, 500L, 777L, 778L, 300000L}) {
+    Array a(N, 4), b(N, 19);
+    g_most = 0;
+    CHECK(a.round_trip(1.0) && !a.pinned);
+    CHECK(b.round_trip(2.0) && !b.pinned);
+    g_most = SIZE_MAX;
+    CHECK(a.round_trip(3.0) && a.pinned);
+    CHECK(b.round_trip(4.0) && b.pinned);
+    stage_leave();  // gives everything back
+    stage_join();
+  }
+  stage_leave();
+  CHECK(g_allocs == g_frees);
+}
+
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "coherent")) coherent();
+  else if (!strcmp(what, "refused")) refused();
   else return 2;
   printf("ok\n");
   return 0;
