@@ -155,8 +155,8 @@ int lbm_set_ns(lbm_handle *h, const double *ns);
 /* f H2D / D2H per subs (src/lbgpu_prime.cu:317-343, :874-900).  Solid
  * nodes are not stored: download returns 0 there.  These calls, the macro
  * download and the samples move data through pinned host memory (at most
- * 16 MiB) and up to seven host threads that all handles of the process share:
- * transfers of several threads take turns; the last lbm_destroy releases
+ * 16 MiB) and up to seven host threads that all handles of the process share,
+ * also transfers of several threads at once; the last lbm_destroy releases
  * both.  Where the system pins no memory they go through ordinary copies. */
 int lbm_upload_f(lbm_handle *h, int subs, const double *f1d);
 int lbm_download_f(lbm_handle *h, int subs, double *f1d);

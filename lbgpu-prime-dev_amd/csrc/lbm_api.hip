@@ -7,9 +7,7 @@
 #include <string.h>
 
 #include <algorithm>
-#include <memory>
 #include <mutex>
-#include <new>
 #include <string>
 #include <vector>
 
@@ -1563,31 +1561,36 @@ extern "C" int lbm_sample_macro(lbm_handle *h, int subs, int npts, const long *n
     if (nodes[q] < 0 || nodes[q] >= h->N) return lbm_fail("sample node %ld outside the lattice", nodes[q]);
   if (!npts) return sync(h);
   Stage &st = stage();
-  std::lock_guard<std::mutex> lock(st.mu);
-  // room for the values of `most` points and then their compact indices, in
-  // pinned memory that the kernel reads and writes, or else on the device
-  const bool pinned = stage_hold(st, kStageSlot);
-  const size_t room = pinned ? kStageSlot : sizeof(double) * kRedValues;
-  const int most = (int)std::min<size_t>(npts, room / (sizeof(double) * comps + sizeof(int)));
-  std::unique_ptr<char[]> copy(pinned ? nullptr : new (std::nothrow) char[room]);
-  if (!pinned && !copy) return lbm_fail("lbm_sample_macro: out of memory");
-  const size_t index_at = sizeof(double) * comps * (size_t)most;
-  char *const dev = pinned ? st.buf : (char *)h->red;
-  char *const host = pinned ? st.buf : copy.get();
-  double *val = (double *)host;
-  int *at = (int *)(host + index_at);
-  for (int q0 = 0; q0 < npts; q0 += most) {
-    const int n = std::min(most, npts - q0);
-    for (int q = 0; q < n; q++) at[q] = h->fid[nodes[q0 + q]];
-    if (!pinned)
-      HIP_OK(hipMemcpyAsync(dev + index_at, at, (size_t)n * sizeof(int), hipMemcpyHostToDevice, h->stream));
-    hipLaunchKernelGGL(k_sample_field, dim3(blocks_for(n)), dim3(256), 0, h->stream, mv, nf, comps,
-                       (const int *)(dev + index_at), n, (double *)dev);
-    HIP_OK(hipGetLastError());
-    if (!pinned)
-      HIP_OK(hipMemcpyAsync(val, dev, (size_t)n * comps * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIP_OK(hipStreamSynchronize(h->stream));
-    memcpy(out + (long)q0 * comps, val, (size_t)n * comps * sizeof(double));
+  Stage::Job job;
+  try {
+    StageLease lease(st, job);
+    // room for the values of `most` points and then their compact indices, in
+    // pinned memory that the kernel reads and writes, or else on the device
+    char *const slot = st.memory(lease.slot);
+    const bool pinned = slot;
+    const size_t room = pinned ? kStageSlot : sizeof(double) * kRedValues;
+    const int most = (int)std::min<size_t>(npts, room / (sizeof(double) * comps + sizeof(int)));
+    std::vector<char> copy(pinned ? 0 : room);
+    const size_t index_at = sizeof(double) * comps * (size_t)most;
+    char *const dev = pinned ? slot : (char *)h->red;
+    char *const host = pinned ? slot : copy.data();
+    double *val = (double *)host;
+    int *at = (int *)(host + index_at);
+    for (int q0 = 0; q0 < npts; q0 += most) {
+      const int n = std::min(most, npts - q0);
+      for (int q = 0; q < n; q++) at[q] = h->fid[nodes[q0 + q]];
+      if (!pinned)
+        HIP_OK(hipMemcpyAsync(dev + index_at, at, (size_t)n * sizeof(int), hipMemcpyHostToDevice, h->stream));
+      hipLaunchKernelGGL(k_sample_field, dim3(blocks_for(n)), dim3(256), 0, h->stream, mv, nf, comps,
+                         (const int *)(dev + index_at), n, (double *)dev);
+      HIP_OK(hipGetLastError());
+      if (!pinned)
+        HIP_OK(hipMemcpyAsync(val, dev, (size_t)n * comps * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+      HIP_OK(hipStreamSynchronize(h->stream));
+      memcpy(out + (long)q0 * comps, val, (size_t)n * comps * sizeof(double));
+    }
+  } catch (const std::exception &x) {
+    return lbm_fail("lbm_sample_macro: %s", x.what());
   }
   return 0;
 }

@@ -6,6 +6,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <thread>
@@ -135,10 +136,57 @@ static void refused() {
   CHECK(g_allocs == g_frees);
 }
 
+// a transfer that begins while another one runs does not wait for its end: it
+// gets slots when the other is between two pieces, and memory that no one
+// else uses meanwhile
+static void beside() {
+  stage_join();
+  constexpr long N = kStageSlot / sizeof(double);
+  Array large(N, 100), small(1000, 3);
+  std::atomic<int> pieces{0}, done{0};
+  std::thread t([&] {
+    const hipError_t e = large.move(false, [&] {
+      pieces++;
+      std::this_thread::sleep_for(std::chrono::milliseconds(10));
+    });
+    CHECK(e == hipSuccess);
+    done++;
+  });
+  while (pieces < 20) std::this_thread::yield();
+  CHECK(small.round_trip(1.0));
+  CHECK(done == 0 && pieces < 90);
+  t.join();
+  CHECK(pieces == 100);
+  stage_leave();
+  CHECK(g_allocs == g_frees);
+}
+
+// many transfers at once, more than there are slots, some refused memory;
+// handles come and go beside them
+static void crowd() {
+  std::atomic<int> rounds{0};
+  std::vector<std::thread> t;
+  for (int q = 0; q < 12; q++)
+    t.emplace_back([&, q] {
+      for (int r = 0; r < 6; r++) {
+        stage_join();
+        Array a(q % 3 ? 1000 + 131 * q : 400000 + 7777 * q, 1 + (q + r) % 7);
+        CHECK(a.round_trip(1000.0 * q + r));
+        if (q == 0) g_most = r & 1 ? SIZE_MAX : kStageSlot - 1;
+        stage_leave();
+        rounds++;
+      }
+    });
+  for (auto &x : t) x.join();
+  CHECK(rounds == 72 && g_allocs == g_frees);
+}
+
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!strcmp(what, "coherent")) coherent();
   else if (!strcmp(what, "refused")) refused();
+  else if (!strcmp(what, "beside")) beside();
+  else if (!strcmp(what, "crowd")) crowd();
   else return 2;
   printf("ok\n");
   return 0;

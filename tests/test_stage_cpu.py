@@ -20,7 +20,7 @@ def stage_check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["coherent", "refused"])
+@pytest.mark.parametrize("check", ["coherent", "refused", "beside", "crowd"])
 def test_host_transfers(stage_check, check):
     out = subprocess.run([stage_check, check], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
