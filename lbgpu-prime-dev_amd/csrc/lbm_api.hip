@@ -1531,24 +1531,33 @@ extern "C" int lbm_download_macro(lbm_handle *h, int subs, double *rho, double *
   const int nf = h->nf, D = h->D;
   const double *src = h->mv + (long)subs * (1 + D) * nf;
   const Geo G = make_args<double, double>(h).G;
-  double *dst[4] = {rho, ux, uy, uz};
-  // components beyond the lattice's velocity are 0; null ones are skipped
+  // the wanted components, in order; those beyond the lattice's velocity are 0
+  double *const all[4] = {rho, ux, uy, uz};
+  double *dst[4];
+  int comps = 0, stored = 0;
+  uint32_t comp = 0;  // component of the c-th wanted one, 8 bits each
+  for (int c = 0; c < 4; c++) {
+    if (!all[c]) continue;
+    comp |= (uint32_t)c << (8 * comps);
+    dst[comps++] = all[c];
+    if (c <= D) stored = comps;
+  }
+  if (!comps) return sync(h);
   auto device = [&](const Piece &p, double *slot) {
-    const int nc = std::min(p.nc, 1 + D - p.c0);
+    const int nc = std::min(p.nc, stored - p.c0);
     if (nc > 0)
-      hipLaunchKernelGGL(k_dense_field, dim3(blocks_for(p.nn), nc), dim3(256), 0, h->stream, G, src, nf, p.c0, p.n0,
-                         p.nn, slot);
+      hipLaunchKernelGGL(k_dense_field, dim3(blocks_for(p.nn), nc), dim3(256), 0, h->stream, G, src, nf,
+                         comp >> (8 * p.c0), p.n0, p.nn, slot);
     return hipGetLastError();
   };
   auto host = [&](const Piece &p, double *slot) {
     for (int c = 0; c < p.nc; c++) {
       double *d = dst[p.c0 + c];
-      if (!d) continue;
-      if (p.c0 + c > D) memset(d + p.n0, 0, (size_t)p.nn * sizeof(double));
+      if (p.c0 + c >= stored) memset(d + p.n0, 0, (size_t)p.nn * sizeof(double));
       else memcpy(d + p.n0, slot + (size_t)c * p.nn, (size_t)p.nn * sizeof(double));
     }
   };
-  return move_pieces(h, 4, false, device, host);
+  return move_pieces(h, comps, false, device, host);
 }
 
 extern "C" int lbm_sample_macro(lbm_handle *h, int subs, int npts, const long *nodes, double *out) {

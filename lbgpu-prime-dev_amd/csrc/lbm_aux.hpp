@@ -23,12 +23,14 @@ __device__ __forceinline__ bool dense_node(const Geo &G, long n0, long nn, long 
   return true;
 }
 
-// fields: host[c][n] = src[c][compact node], 0 at a solid node
-__global__ void k_dense_field(Geo G, const double *src, int nf, int c0, long n0, long nn, double *host) {
+// fields: host[c][n] = src[component c][compact node], 0 at a solid node;
+// comps holds the components, 8 bits each
+__global__ void k_dense_field(Geo G, const double *src, int nf, uint32_t comps, long n0, long nn, double *host) {
   long t;
   int idx;
   if (!dense_node(G, n0, nn, t, idx)) return;
-  host[(long)blockIdx.y * nn + t] = idx < 0 ? 0.0 : src[(long)(c0 + blockIdx.y) * nf + idx];
+  const int c = (int)(comps >> (8 * blockIdx.y) & 0xffu);
+  host[(long)blockIdx.y * nn + t] = idx < 0 ? 0.0 : src[(long)c * nf + idx];
 }
 
 // fields at single nodes: out[q][c] = src[c][at[q]], 0 where at[q] < 0 (solid);
