@@ -111,17 +111,12 @@ struct lbm_handle {
   double *ns = nullptr;  // [nf] Walsh partial bounce-back fraction, or null
   // 2-D runs of several steps per launch (k_tile2d): the plan, its tables and
   // the population array its launches write (swapped with F after each)
-  struct {
+  struct Tiles : Plan2d {
     int state = 0;  // 0 not planned, 1 ready, -1 not for this lattice
-    TileGeo T{};
-    int steps = 0, shrink = 0, threads = 0;
-    bool keep = false;  // one tile per CU, one node per thread
     int lds_set = 0;  // kernels whose LDS limit has been raised
-    size_t lds = 0;
     int *gidx = nullptr, *cnt = nullptr;
     uint32_t *list = nullptr;
-    int2 *tab = nullptr;  // k_sweep2d: strips instead of tiles
-    SweepGeo S{};
+    int2 *tab = nullptr;  // k_sweep2d
     void *F2 = nullptr;
   } tile;
   bool off64 = false;    // 64-bit element offsets at every size (LBM_OFFSET64=1)
@@ -1251,46 +1246,6 @@ int tile_launch(lbm_handle *h, const TileArgs &B) {
   return t.keep ? tiles(k_tile2d<NS, SOL, WALSH, true>) : tiles(k_tile2d<NS, SOL, WALSH, false>);
 }
 
-// Steps per launch and core of k_tile2d for the handle's lattice.
-// A lattice that one tile per CU covers takes the smallest square core that
-// does: its time is launch (2 us) and per-step latency (1 us), so it takes
-// as many steps a launch as the halo's work allows, 8 (flow with cores up to
-// 10: 10; two components with cores above 12: 6).  Measured when the kernel was first
-// tuned, us per step, flow | flow + solute with row conditions: 128^2 8 x 8
-// cores 1.54 | 1.94 (4 steps 1.74 | 2.06), 200 x 170 12 x 12 cores 1.64 | 2.07
-// (4 steps 1.9 | 2.19), 300 x 310 20 x 20 cores 1.97 with 8 steps | 2.71 with 6
-// (4 steps: 2.3 | 2.86).
-// Larger lattices run several tiles per CU and are bound by the loads of the
-// halo and the FP64 units together: 4 steps, flow in 32 x 16 cores of which a
-// CU holds two (1000^2 10.8, 2100 x 1900 44.9 us; 30 x 30 cores with 8 steps
-// 11.3, 43.7), flow + solute in the largest square core that LDS holds, 25 x
-// 25 (19.7, 85.3 us; 32 x 16 20.4, 91.4; 20 x 20 with 6 steps 22.2, 94.9).
-// Now, with entries in registers: 1.26 (10 steps; 8: 1.31) | 1.77, 1.38 | 1.91,
-// 1.82 | 2.61 us; 413 x 307 flow, 23 x 23 cores with 8 steps, 2.05 (32 x 16
-// cores with 4: 3.02); 1000^2 9.8 | 18.2, 2100 x 1900 41.0 us.
-void tile_shape(const lbm_handle *h, int shrink, int &steps, int &cx, int &cy) {
-  const int ns = h->p.nsubs;
-  const double per_cu = (double)h->N / h->cus;
-  int s = 8;
-  while ((double)s * s < per_cu && s < 64) s++;
-  // most one-tile cores: what LDS holds with 8 (flow) and 6 steps
-  const int one = ns == 1 ? 29 : 20;
-  steps = s <= 10 && ns == 1 ? 10 : (s <= 12 ? 8 : (s <= one ? (ns == 1 ? 8 : 6) : 4));
-  auto most = [&](int k) {  // largest square core of k steps
-    int c = 0;
-    const int halo = shrink * k / 2;
-    auto fits = [&](int r) { return r * r <= kTileRegion && (size_t)r * r * 72 * ns <= (size_t)h->lds_cu; };
-    while (fits(c + 1 + 2 * halo)) c++;
-    return c;
-  };
-  if (most(steps) < s) steps = 4;
-  cx = cy = std::min(s, most(steps));
-  if (s > one && ns == 1) {
-    cx = 32;
-    cy = 16;
-  }
-}
-
 // Plans the tiles of the handle's lattice on first use; h->tile.state tells
 // whether lbm_run may use them.
 int plan_tiles(lbm_handle *h) {
@@ -1318,7 +1273,9 @@ int plan_tiles(lbm_handle *h) {
       for (int d = -1; d <= 1; d++) handed |= h->fid[src * ni + (i + d + ni) % ni] < 0;
     }
   }
-  t.shrink = handed ? 3 : 2;
+  Plan2d P;
+  if (!plan2d(ni, nj, p.nsubs, handed, h->lds_cu, h->cus, P)) return 0;
+  static_cast<Plan2d &>(t) = P;
   const size_t sb = (size_t)h->tiles * p.nsubs * h->Q * kTile * h->st_bytes;
   const StepArgs<double, double> A = make_args<double, double>(h);
   auto off = [&]() {  // no memory: the steps are launched one by one
@@ -1327,56 +1284,15 @@ int plan_tiles(lbm_handle *h) {
     h->tile.state = -1;
     return 0;
   };
-  t.T.ni = ni;
-  t.T.nj = nj;
-  // Strips (k_sweep2d) for flow + solute lattices of many tiles per CU, us per
-  // step, tiles -> strips: 1000^2 18.2 -> 19.6, 1088 x 1224 28 -> 23.8,
-  // 2100 x 1900 80 -> 62, below that tiles are faster (600 x 500 6.7
-  // against 9.2: short strips repeat their pipeline's start too often).  Flow
-  // alone keeps tiles (1088 x 1224 12.4 against 17.2, 2100 x 1900 41.0 against
-  // 41.9).  Rows that hand values to a neighbour need the tiles' barrier.
-  if (two && !handed && h->N >= 4500L * h->cus) {
-    SweepGeo &S = t.S;
-    const size_t col = (size_t)kSweepRows * (72 * p.nsubs + 8) + 8 * kSweepEntries;
-    const int most = (int)std::min<size_t>(kSweepCols, h->lds_cu / col) - 2 * kSweepHalo;
-    if (most < kSweepHalo) return 0;
-    S.strips = (ni + most - 1) / most;
-    S.cw = (ni + S.strips - 1) / S.strips;
-    S.strips = (ni + S.cw - 1) / S.cw;
-    S.rw = S.cw + 2 * kSweepHalo;
-    S.pieces = std::max(1, h->cus / S.strips);
-    S.ch = (nj + S.pieces - 1) / S.pieces;
-    S.pieces = (nj + S.ch - 1) / S.ch;
-    S.blocks8 = (S.strips * S.pieces + 7) / 8;
-    t.lds = col * S.rw;
-    t.steps = kSweepSteps;
-    t.threads = kSweepBlock;
-    const long n = (long)S.strips * nj * S.rw;
+  if (P.sweep) {
+    const long n = (long)P.S.strips * nj * P.S.rw;
     if (hipMalloc(&t.tab, (size_t)n * sizeof(int2)) != hipSuccess || hipMalloc(&t.F2, sb) != hipSuccess) return off();
-    hipLaunchKernelGGL(k_sweep_build, dim3(blocks_for(n)), dim3(256), 0, h->stream, A.G, S, t.tab);
+    hipLaunchKernelGGL(k_sweep_build, dim3(blocks_for(n)), dim3(256), 0, h->stream, A.G, P.S, t.tab);
     HIP_OK(hipGetLastError());
     t.state = 1;
     return 0;
   }
-  tile_shape(h, t.shrink, t.steps, t.T.cx, t.T.cy);
-  const int cx = t.T.cx, cy = t.T.cy;
-  TileGeo &T = t.T;
-  T.halo = t.shrink * t.steps / 2;
-  T.tx = (ni + cx - 1) / cx;
-  T.ty = (nj + cy - 1) / cy;
-  T.cx = (ni + T.tx - 1) / T.tx;
-  T.cy = (nj + T.ty - 1) / T.ty;
-  T.tx = (ni + T.cx - 1) / T.cx;
-  T.ty = (nj + T.cy - 1) / T.cy;
-  T.rx = T.cx + 2 * T.halo;
-  T.rn = T.rx * (T.cy + 2 * T.halo);
-  T.tiles8 = (T.tx * T.ty + 7) / 8;
-  t.lds = (size_t)T.rn * 72 * p.nsubs;
-  t.threads = std::min(kTileThreads, (T.rn + 63) / 64 * 64);
-  t.keep = T.rn <= kTileThreads && T.tx * T.ty <= h->cus;
-  // two workgroups of a CU fit its registers with 512 threads each
-  if (!t.keep && 2 * t.lds <= (size_t)h->lds_cu) t.threads = std::max(512, (T.rn / 2 + 63) / 64 * 64);
-  if (T.rn > kTileRegion || t.lds > (size_t)h->lds_cu) return 0;
+  const TileGeo &T = P.T;
   const long n = (long)T.tx * T.ty;
   if (hipMalloc(&t.gidx, (size_t)n * T.rn * sizeof(int)) != hipSuccess ||
       hipMalloc(&t.list, (size_t)n * T.rn * sizeof(uint32_t)) != hipSuccess ||

@@ -33,27 +33,15 @@
 #pragma once
 
 #include "lbm_device.hpp"
+#include "lbm_plan2d.hpp"
 
 namespace lbm {
-
-constexpr int kTileSteps = 16;   // most steps of one launch
-constexpr int kTileRegion = 2048;  // most region nodes (below 4096: 12-bit region index)
 
 // list entry of a fluid region node: region index, bit 12 + a - 1 set when
 // x - c_a is fluid, the boundary rows, and from bit 22 its distance from the
 // region's edge (at most the halo)
 constexpr uint32_t kTileNorth = 1u << 20, kTileSouth = 1u << 21;
 constexpr int kTileDist = 22;
-constexpr int kTileThreads = 1024;  // most threads of k_tile2d, which take at most two nodes each
-
-struct TileGeo {
-  int ni, nj;
-  int cx, cy;      // core size
-  int tx, ty;      // tiles
-  int halo;        // H
-  int rx, rn;      // region row length cx + 2 H and node count
-  int tiles8;      // launched tiles / 8 (XCD mapping)
-};
 
 // core origin, core size and region size of tile t
 LBM_HD void tile_span(const TileGeo &T, int t, int &x0, int &y0, int &cw, int &ch) {
@@ -382,16 +370,6 @@ __global__ __launch_bounds__(kTileThreads) void k_tile2d(TileArgs B) {
 // takes 1.7 us: 0.9 us without the collision (LDS traffic and latency of two
 // waves per SIMD, which is all that 160 KB of rows feed), 0.1 us of it waiting
 // for the global loads; solid columns leave 30 % of the lanes idle.
-constexpr int kSweepSteps = 4, kSweepHalo = 4, kSweepRows = 9;
-constexpr int kSweepEntries = 16;  // rows whose table entries are in LDS (i - 6 .. i + 4)
-
-struct SweepGeo {
-  int cw, strips;   // core columns of a strip
-  int rw;           // table row length cw + 2 kSweepHalo
-  int ch, pieces;   // rows of a piece, pieces of a strip
-  int blocks8;      // launched workgroups / 8
-};
-
 // tab[strip][row][column] = {compact index (-1 solid or past the strip),
 // entry bits of the node}
 __global__ __launch_bounds__(256) void k_sweep_build(Geo G, SweepGeo S, int2 *tab) {
@@ -421,9 +399,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-
-// one thread per column and stage
-constexpr int kSweepCols = 128, kSweepBlock = 4 * kSweepCols;
 
 template <bool SOL, bool WALSH>
 __global__ __launch_bounds__(kSweepBlock) void k_sweep2d(TileArgs B, SweepGeo S, const int2 *tab) {
