@@ -313,7 +313,7 @@ int lbm_objective_observations(lbm_handle *h, int n, const long *node, const int
  * segment between saved states out of place and sweeping it backwards:
  * grad[0..4] = dJ/d(g_x, g_y, g_z, tau, tau_s) of the flow's body force
  * and relaxation times; grad_cmap (optional, [LY][LX]) = dJ/dc_bot_map.
- * Device memory: nsteps/every saved states (objective run) and every + 2
+ * Device memory: nsteps/every saved states (objective run) and every + 1
  * states (adjoint run), each the size of the population array; both stay
  * allocated for the next run and are released by lbm_set_solids and
  * lbm_destroy.  An objective run may be swept more than once, except when
@@ -326,7 +326,7 @@ int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap);
  * of its last whole segments of `every` steps, as many as max_bytes holds
  * (one state is the size of the population array) while the checkpoints of
  * the other segments, the adjoint state, the states of one replayed segment
- * (every + 1; the first kept buffers serve when there are that many) and
+ * (every; the first kept buffers serve when every + 1 are kept) and
  * 1 GiB of device memory stay free, and the adjoint sweep uses them instead
  * of replaying those segments from checkpoints.  The gradient is the same
  * bit for bit.  The kept states stay allocated like the checkpoints. */

@@ -147,7 +147,7 @@ struct lbm_handle {
     size_t keep_bytes = 0;     // lbm_objective_keep_states
     std::vector<void *> kept;  // states (after the BCs) before the last kept steps of the run
     int kept_from = 0;         // the run's first kept step index (0-based; nsteps: none)
-    int kept_replay = 0;       // the sweep replays into kept[0..every] (no segment buffers
+    int kept_replay = 0;       // the sweep replays into the first kept buffers (no segment buffers
                                // of its own), which then no longer hold the run's states
     double *jacc = nullptr;
     double J = 0.0;
@@ -1840,10 +1840,10 @@ extern "C" int lbm_objective_run(lbm_handle *h, int nsteps, int window, int ever
     const long cap = (long)(h->obj.keep_bytes / sb);
     // The most steps (nsteps - m * every, m = 0, 1, ...) the budget holds
     // whose states fit in device memory together with the checkpoints of the
-    // m replayed segments, the adjoint state and, when m > 0, the states of
-    // one replayed segment (every + 1, the first kept buffers when there are
-    // that many), and 1 GiB besides; memory these buffers already hold
-    // counts as available.
+    // m replayed segments, the adjoint state and, when m > 0, the states
+    // before the steps of one replayed segment (in kept buffers when there
+    // are every + 1 or more), and 1 GiB besides; memory these buffers already
+    // hold counts as available.
     size_t free_b = 0, total_b = 0;
     HIP_OK(hipMemGetInfo(&free_b, &total_b));
     const double held = (double)(h->obj.kept.size() + h->obj.ckpt.size() + h->obj.seg.size()) * (double)sb;
@@ -1851,7 +1851,7 @@ extern "C" int lbm_objective_run(lbm_handle *h, int nsteps, int window, int ever
     const long needL = h->obj.L ? 0 : 1;
     for (long m = 0; m * every < nsteps; m++) {
       const long p = nsteps - m * every;
-      const long segbuf = m > 0 && p < every + 1 ? every + 1 : 0;
+      const long segbuf = m > 0 && p < every + 1 ? std::min(every, nsteps) : 0;
       if (p <= cap && (double)(p + m + segbuf + needL) * (double)sb <= avail) {
         P = p;
         break;
@@ -1863,7 +1863,8 @@ extern "C" int lbm_objective_run(lbm_handle *h, int nsteps, int window, int ever
   // With every + 1 kept states or more and segments to replay, the sweep
   // replays them into the first kept buffers (it sweeps the kept segments
   // first) instead of segment buffers of its own; the run then supports one
-  // sweep.
+  // sweep.  (It needs `every` of them; with exactly that many kept, as with
+  // fewer, a run goes on supporting any number of sweeps.)
   const bool kept_replay = nck > 0 && P >= every + 1;
   // release what this run and its sweep will not use before allocating:
   // the sizing above counted it as available
@@ -2032,12 +2033,12 @@ extern "C" int lbm_adjoint_run(lbm_handle *h, double *grad, double *grad_cmap) {
     return rc;
   };
   hipError_t e;
-  // workspace: K + 1 segment states (or the first K + 1 kept buffers, free
-  // once the kept segments are swept), the adjoint state and the gradient
-  // accumulators, kept for the next call
+  // workspace: the states before the steps of one replayed segment (or the
+  // first kept buffers, free once the kept segments are swept), the adjoint
+  // state and the gradient accumulators, kept for the next call
   std::vector<void *> &seg = h->obj.seg;
   const bool kept_replay = h->obj.kept_replay && nrep > 0 && h->obj.kept.size() >= (size_t)K + 1;
-  const size_t nsegbuf = nrep > 0 && !kept_replay ? (size_t)K + 1 : 0;
+  const size_t nsegbuf = nrep > 0 && !kept_replay ? (size_t)std::min(K, T) : 0;
   while (seg.size() > nsegbuf) {
     (void)hipFree(seg.back());
     seg.pop_back();
