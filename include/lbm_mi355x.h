@@ -190,11 +190,11 @@ int lbm_step(lbm_handle *h, int write_macro);
 /* nsteps steps, macroscopic write on the last one if write_macro_last.  The
  * results are those of nsteps calls of lbm_step.  With FP64 storage and
  * collision a D2Q9 lattice runs several steps per launch, for which the first
- * run of two steps or more allocates a second population array, and a D3Q19
- * lattice below 65,536 fluid nodes reads its neighbours' locations from a
- * table that the first run of 128 steps or more allocates; without the
- * memory the steps run without them.  lbm_set_solids and lbm_destroy release
- * both. */
+ * run that does so allocates a second population array and tables, if they
+ * take no more than an eighth of the free device memory; and a D3Q19 lattice
+ * below 65,536 fluid nodes reads its neighbours' locations from a table that
+ * the first run of 128 steps or more allocates.  Without the memory the steps
+ * run without them.  lbm_set_solids and lbm_destroy release both. */
 int lbm_run(lbm_handle *h, int nsteps, int write_macro_last);
 
 /* The two half-steps on their own, at an explicit time (a1 / a2):

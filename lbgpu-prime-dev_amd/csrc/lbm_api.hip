@@ -112,7 +112,7 @@ struct lbm_handle {
   // 2-D runs of several steps per launch (k_tile2d): the plan, its tables and
   // the population array its launches write (swapped with F after each)
   struct Tiles : Plan2d {
-    int state = 0;  // 0 not planned, 1 ready, -1 not for this lattice
+    int state = 0;  // 0 not planned, 1 planned, 2 ready, -1 not for this lattice
     int lds_set = 0;  // kernels whose LDS limit has been raised
     int *gidx = nullptr, *cnt = nullptr;
     uint32_t *list = nullptr;
@@ -1248,20 +1248,20 @@ int tile_launch(lbm_handle *h, const TileArgs &B) {
 
 // Plans the tiles of the handle's lattice on first use; h->tile.state tells
 // whether lbm_run may use them.
-int plan_tiles(lbm_handle *h) {
+void plan_tiles(lbm_handle *h) {
   auto &t = h->tile;
-  if (t.state) return 0;
+  if (t.state) return;
   t.state = -1;
   const lbm_params &p = h->p;
-  if (h->D != 2 || p.storage != LBM_STORE_F64 || p.compute != LBM_COMPUTE_F64 || p.halo_mode || h->off64) return 0;
+  if (h->D != 2 || p.storage != LBM_STORE_F64 || p.compute != LBM_COMPUTE_F64 || p.halo_mode || h->off64) return;
   int kind[2], which;
-  if (!row_condition(p, 0, kind[0], which) || !row_condition(p, 1, kind[1], which)) return 0;
+  if (!row_condition(p, 0, kind[0], which) || !row_condition(p, 1, kind[1], which)) return;
   const bool two = p.nsubs == 2;
-  if (two && (p.pressure_n_in[1] || p.pressure_n_out[1] || p.pressure_s_in[1] || p.pressure_s_out[1])) return 0;
+  if (two && (p.pressure_n_in[1] || p.pressure_n_out[1] || p.pressure_s_in[1] || p.pressure_s_out[1])) return;
   const int grad[2] = {two && p.zeroconcgrad_n, two && p.zeroconcgrad_s};
   const bool rows = kind[0] || kind[1] || grad[0] || grad[1];
   const int ni = p.ni, nj = p.nj;
-  if (rows && nj < 3) return 0;
+  if (rows && nj < 3) return;
   // whether a density or zero-gradient row hands a value to a neighbour: a
   // row node whose source across the wrapped edge is solid
   bool handed = false;
@@ -1274,34 +1274,48 @@ int plan_tiles(lbm_handle *h) {
     }
   }
   Plan2d P;
-  if (!plan2d(ni, nj, p.nsubs, handed, h->lds_cu, h->cus, P)) return 0;
+  if (!plan2d(ni, nj, p.nsubs, handed, h->lds_cu, h->cus, P)) return;
   static_cast<Plan2d &>(t) = P;
-  const size_t sb = (size_t)h->tiles * p.nsubs * h->Q * kTile * h->st_bytes;
-  const StepArgs<double, double> A = make_args<double, double>(h);
-  auto off = [&]() {  // no memory: the steps are launched one by one
+  t.state = 1;
+}
+
+// Makes what the planned launches need, before the first of them: the tables
+// and the second population array.  They are taken from memory that the
+// caller may have other uses for, so only where they need no more than an
+// eighth of what is free; without them (state -1) the steps are launched one
+// by one.
+constexpr size_t kTileShare = 8;
+
+int make_tiles(lbm_handle *h) {
+  auto &t = h->tile;
+  if (t.state != 1) return 0;
+  auto off = [&]() {
     (void)hipGetLastError();
     free_tiles(h);
     h->tile.state = -1;
     return 0;
   };
-  if (P.sweep) {
-    const long n = (long)P.S.strips * nj * P.S.rw;
-    if (hipMalloc(&t.tab, (size_t)n * sizeof(int2)) != hipSuccess || hipMalloc(&t.F2, sb) != hipSuccess) return off();
-    hipLaunchKernelGGL(k_sweep_build, dim3(blocks_for(n)), dim3(256), 0, h->stream, A.G, P.S, t.tab);
-    HIP_OK(hipGetLastError());
-    t.state = 1;
-    return 0;
+  const size_t sb = (size_t)h->tiles * h->p.nsubs * h->Q * kTile * h->st_bytes;
+  const TileGeo &T = t.T;
+  const long n = t.sweep ? (long)t.S.strips * T.nj * t.S.rw : (long)T.tx * T.ty;
+  const size_t tables = t.sweep ? (size_t)n * sizeof(int2)
+                                : (size_t)n * (T.rn * (sizeof(int) + sizeof(uint32_t)) + sizeof(int));
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || sb + tables > free_b / kTileShare) return off();
+  const Geo G = make_args<double, double>(h).G;
+  if (hipMalloc(&t.F2, sb) != hipSuccess) return off();
+  if (t.sweep) {
+    if (hipMalloc(&t.tab, (size_t)n * sizeof(int2)) != hipSuccess) return off();
+    hipLaunchKernelGGL(k_sweep_build, dim3(blocks_for(n)), dim3(256), 0, h->stream, G, t.S, t.tab);
+  } else {
+    if (hipMalloc(&t.gidx, (size_t)n * T.rn * sizeof(int)) != hipSuccess ||
+        hipMalloc(&t.list, (size_t)n * T.rn * sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&t.cnt, (size_t)n * sizeof(int)) != hipSuccess)
+      return off();
+    hipLaunchKernelGGL(k_tile_build, dim3((unsigned)n), dim3(256), 0, h->stream, G, T, t.gidx, t.list, t.cnt);
   }
-  const TileGeo &T = P.T;
-  const long n = (long)T.tx * T.ty;
-  if (hipMalloc(&t.gidx, (size_t)n * T.rn * sizeof(int)) != hipSuccess ||
-      hipMalloc(&t.list, (size_t)n * T.rn * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&t.cnt, (size_t)n * sizeof(int)) != hipSuccess ||
-      hipMalloc(&t.F2, sb) != hipSuccess)
-    return off();
-  hipLaunchKernelGGL(k_tile_build, dim3((unsigned)n), dim3(256), 0, h->stream, A.G, T, t.gidx, t.list, t.cnt);
   HIP_OK(hipGetLastError());
-  t.state = 1;
+  t.state = 2;
   return 0;
 }
 
@@ -1367,21 +1381,22 @@ extern "C" int lbm_run(lbm_handle *h, int nsteps, int write_macro_last) {
   if (need_lattice(h)) return 1;
   int q = 0;
   if (nsteps >= kTableSteps && build_table(h)) return 1;
-  if (nsteps >= 2 && !h->profile && plan_tiles(h)) return 1;
-  if (nsteps >= 2 && !h->profile && h->tile.state == 1) {
+  if (nsteps >= 2 && !h->profile) {
+    plan_tiles(h);
     // a step that records the plane flux reads the state before it
     const int keep = h->n_flux && write_macro_last ? 1 : 0;
-    while (q < nsteps) {
+    while (q < nsteps && h->tile.state > 0) {
       const int len = tile_steps(h, nsteps - q - keep);
+      if (len && make_tiles(h)) return 1;
+      if (h->tile.state < 0) break;
       if (len ? run_tile(h, len, q + len == nsteps ? write_macro_last : 0)
               : do_step(h, q == nsteps - 1 ? write_macro_last : 0))
         return 1;
       q += len ? len : 1;
     }
-    return sync(h);
   }
   // the steps before the last in captured chunks where their launches repeat
-  if (nsteps - 1 >= kChunk && chunkable(h, h->time + 1, h->time + nsteps - 1)) {
+  if (nsteps - 1 - q >= kChunk && chunkable(h, h->time + 1, h->time + nsteps - 1 - q)) {
     while (nsteps - 1 - q >= kChunk) {
       hipGraphExec_t g = chunk_for(h);
       if (!g) break;
