@@ -113,6 +113,7 @@ struct lbm_handle {
   // the population array its launches write (swapped with F after each)
   struct Tiles : Plan2d {
     int state = 0;  // 0 not planned, 1 planned, 2 ready, -1 not for this lattice
+    bool rows = false;  // some row carries a condition
     int lds_set = 0;  // kernels whose LDS limit has been raised
     int *gidx = nullptr, *cnt = nullptr;
     uint32_t *list = nullptr;
@@ -324,6 +325,11 @@ int dispatch(const lbm_handle *h, Fn &&fn) {
   if (h->Q == 19 && h->p.nsubs == 2) { LBM_DISPATCH_T(19, 2) }
 #undef LBM_DISPATCH_T
   return lbm_fail("unsupported storage/compute combination");
+}
+
+// bytes of the population array
+size_t state_bytes(const lbm_handle *h) {
+  return (size_t)h->tiles * h->p.nsubs * h->Q * kTile * h->st_bytes;
 }
 
 inline unsigned blocks_for(long n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
@@ -1276,6 +1282,7 @@ void plan_tiles(lbm_handle *h) {
   Plan2d P;
   if (!plan2d(ni, nj, p.nsubs, handed, h->lds_cu, h->cus, P)) return;
   static_cast<Plan2d &>(t) = P;
+  t.rows = rows;
   t.state = 1;
 }
 
@@ -1295,7 +1302,7 @@ int make_tiles(lbm_handle *h) {
     h->tile.state = -1;
     return 0;
   };
-  const size_t sb = (size_t)h->tiles * h->p.nsubs * h->Q * kTile * h->st_bytes;
+  const size_t sb = state_bytes(h);
   const TileGeo &T = t.T;
   const long n = t.sweep ? (long)t.S.strips * T.nj * t.S.rw : (long)T.tx * T.ty;
   const size_t tables = t.sweep ? (size_t)n * sizeof(int2)
@@ -1337,7 +1344,8 @@ int tile_steps(const lbm_handle *h, int n) {
     if (same) break;
     len -= 2;
   }
-  return len;
+  const bool resting = h->p.nsubs == 2 && !solute_on(h, t1);
+  return len < least_steps(h->tile, h->p.nsubs, h->tile.rows, resting, state_bytes(h), h->cus) ? 0 : len;
 }
 
 int run_tile(lbm_handle *h, int steps, int write_macro) {
@@ -1759,10 +1767,6 @@ static int adjoint_supported(const lbm_handle *h) {
         (h->zconc[0] == kCNone && h->zconc[1] == kCNone)))
     return lbm_fail("the adjoint needs a Dirichlet solute inlet at z = 0 with a zero-gradient outlet, or none");
   return 0;
-}
-
-static size_t state_bytes(const lbm_handle *h) {
-  return (size_t)h->tiles * h->p.nsubs * h->Q * kTile * h->st_bytes;
 }
 
 extern "C" int lbm_objective_observations(lbm_handle *h, int n, const long *node, const int *step,

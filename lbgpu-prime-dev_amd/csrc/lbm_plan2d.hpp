@@ -138,4 +138,29 @@ inline bool plan2d(int ni, int nj, int ns, bool handed, int lds_cu, int cus, Pla
   return T.rn <= kTileRegion && P.lds <= (size_t)lds_cu;
 }
 
+// The fewest steps a launch has to take to beat as many half-steps launched
+// one by one.  With row conditions, two: a step by itself costs two to four
+// launches more (run(2) of 102 x 11500 flow + solute 57.6 us a step one by one,
+// 56.8 in a launch; 420 x 300 31 and 12).  Without them a launch of two steps
+// pays only where it loads little more than the half-steps do; us a step in
+// runs of two, one by one and in a launch:
+//   flow in one round of tiles (128^2 8.9 8.2, 413 x 307 10.0 10.0), and in
+//   many tiles while both arrays stay in the 256 MB memory-side cache (512^2
+//   12.6 10.6, 1000^2 25.9 20.6, 1300^2 36.8 29.9; beyond it 2100 x 1900 74.6
+//   78.0, with partial bounce-back 78 and 88);
+//   a resting solute, whose half-steps touch its lines all the same (1000^2
+//   47.8 34.3, 2100 x 1900 170 104);
+//   not flow + solute (200 x 170 9.4 9.7, with partial bounce-back 9.6 10.8; in
+//   strips of 51 columns, 102 x 11500, 45.1 57.1);
+//   nor where some CUs run a second tile (420 x 300 flow 10.0 12.1, 480 x 340
+//   10.7 13.1), where cores beyond 20 x 20 do not pay in four steps either
+//   (480 x 340 8.0 7.9, with partial bounce-back 8.1 8.4; in six 7.3 6.5).
+inline int least_steps(const Plan2d &P, int ns, bool rows, bool resting, size_t state_bytes, int cus) {
+  if (rows) return 2;
+  const long tiles = P.sweep ? 0 : (long)P.T.tx * P.T.ty;
+  if (tiles > cus && tiles < 2L * cus) return std::min(P.steps, P.T.cx * P.T.cy > 400 ? 6 : 4);
+  if (resting || (ns == 1 && (tiles <= cus || 2 * state_bytes <= 200000000))) return 2;
+  return std::min(P.steps, 4);
+}
+
 }  // namespace lbm

@@ -50,3 +50,21 @@ def test_second_array_leaves_the_callers_memory():
     for x, y in zip(scarce, (a.mv(0), a.mv(1))):
         assert all(np.array_equal(p, q) for p, q in zip(x, y))
     a.close()
+
+def test_short_runs_take_no_memory():
+    """two steps without row conditions are launched one by one: a program
+    that runs no more at a time pays for no second array"""
+    L = _pkg.load()
+    ni, nj = 1201, 1103
+    state = ni * nj * 9 * 2 * 8
+    a = L.Lattice(mask=np.zeros((nj, ni), np.uint8), dims=2, ni=ni, nj=nj, nsubs=2, tau=(0.8, 0.75))
+    a.init_rest()
+    a.step()
+    a.step()
+    before = free()
+    for _ in range(3):
+        a.run(2)
+    assert before - free() < state // 2
+    a.run(4)
+    assert before - free() > state // 2
+    a.close()
