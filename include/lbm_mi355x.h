@@ -191,7 +191,7 @@ int lbm_step(lbm_handle *h, int write_macro);
  * results are those of nsteps calls of lbm_step.  With FP64 storage and
  * collision a D2Q9 lattice runs several steps per launch, for which the first
  * run that does so allocates a second population array and tables, if they
- * take no more than an eighth of the free device memory; and a D3Q19 lattice
+ * take no more than 32 MiB or an eighth of the free device memory; and a D3Q19 lattice
  * below 65,536 fluid nodes reads its neighbours' locations from a table that
  * the first run of 128 steps or more allocates.  Without the memory the steps
  * run without them.  lbm_set_solids and lbm_destroy release both. */

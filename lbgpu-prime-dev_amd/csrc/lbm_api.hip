@@ -1289,9 +1289,10 @@ void plan_tiles(lbm_handle *h) {
 // Makes what the planned launches need, before the first of them: the tables
 // and the second population array.  They are taken from memory that the
 // caller may have other uses for, so only where they need no more than an
-// eighth of what is free; without them (state -1) the steps are launched one
-// by one.
-constexpr size_t kTileShare = 8;
+// eighth of what is free, or next to nothing (asking costs the first run of a
+// small lattice 14 us of 60); without them (state -1) the steps are launched
+// one by one.
+constexpr size_t kTileShare = 8, kTileSmall = 32u << 20;
 
 int make_tiles(lbm_handle *h) {
   auto &t = h->tile;
@@ -1307,8 +1308,10 @@ int make_tiles(lbm_handle *h) {
   const long n = t.sweep ? (long)t.S.strips * T.nj * t.S.rw : (long)T.tx * T.ty;
   const size_t tables = t.sweep ? (size_t)n * sizeof(int2)
                                 : (size_t)n * (T.rn * (sizeof(int) + sizeof(uint32_t)) + sizeof(int));
-  size_t free_b = 0, total_b = 0;
-  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || sb + tables > free_b / kTileShare) return off();
+  if (sb + tables > kTileSmall) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || sb + tables > free_b / kTileShare) return off();
+  }
   const Geo G = make_args<double, double>(h).G;
   if (hipMalloc(&t.F2, sb) != hipSuccess) return off();
   if (t.sweep) {
