@@ -47,10 +47,16 @@ constexpr int kBlock = 256;
 //   FP32             6.2 12.0 49.4 165.3 353.6 -> 5.4 10.0 48.7 163.5 352.5
 //     (512, 256 -> 256, 128 capped at 4)
 //   FP32, FP64 collision  5.9 10.7 49.3 165.4 356.1 -> 5.6 10.3 same (64, 128)
-// FP16 storage keeps 256 threads uncapped: 64 and 128 threads measured within
-// 1 % below 3.2M nodes and 2-4 % slower at 7.0M, caps 3-70 % slower.  D2Q9 waves
-// carry half the bytes and want more of them: FP32 even steps stay at 256
-// uncapped (flow, 1088 x 1224 15.4 us a step; 128 capped at 4: 16.4).
+// (FP32: flow + solute.)  FP16 storage keeps 256 threads uncapped: 64 and 128
+// threads measured within 1 % below 3.2M nodes and 2-4 % slower at 7.0M, caps
+// 3-70 % slower.  Waves that carry half the bytes want more of them.  D2Q9 FP32
+// even steps run 256 uncapped (flow, 1088 x 1224 15.4 us a step; 128 capped at
+// 4: 16.4).  D3Q19 flow alone in FP32 runs 256 capped at 4 (us per step at 386k,
+// 470k, 499k, 1.1M, 2.8M and 6.9M fluid nodes: 128 capped at 4 12.2 15.5 17.0
+// 33.3 76.7 198.4; 256 capped at 4 11.7 14.5 15.7 32.5 76.7 189.2; uncapped,
+// whose last round of waves is nearly empty at some sizes, 11.9 16.3 17.5 32.1
+// 77.3 192.7; with the FP64 collision 13.1 16.5 18.0 34.4 80.3 206.4 and 12.1
+// 15.2 16.6 33.2 79.8 194.8).
 constexpr int kFewNodes = 1 << 18;
 constexpr int kStepBlock = 256;  // largest workgroup of a half-step
 struct StepShape {
@@ -64,7 +70,8 @@ StepShape step_shape(bool odd, int nf) {
   if (f64 && NS == 2) return odd ? StepShape{64, 6} : StepShape{128, 2};
   if (f64) return odd ? StepShape{256, 3} : StepShape{128, 3};
   if (f32_f64) return odd ? StepShape{64, 0} : StepShape{128, 0};
-  return odd || Q == 9 ? StepShape{256, 0} : StepShape{128, 4};
+  if (odd || Q == 9) return {256, 0};
+  return NS == 1 && sizeof(ST) == 4 ? StepShape{256, 4} : StepShape{128, 4};
 }
 // LDS a half-step workgroup reserves to cap the workgroups per CU
 inline size_t step_lds_pad(int per_cu, int lds_per_cu) {
