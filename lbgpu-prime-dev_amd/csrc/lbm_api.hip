@@ -1191,22 +1191,27 @@ hipGraphExec_t chunk_for(lbm_handle *h) {
 // compute the same locations.
 constexpr int kTableSteps = 128;
 
-int build_table(lbm_handle *h) {
-  if (h->ltab || h->D != 3 || h->nf >= kTableNodes || h->off64) return 0;
-  if (hipMalloc(&h->ltab, (size_t)(h->Q - 1) * h->nf * sizeof(uint32_t)) != hipSuccess) {
+void build_table(lbm_handle *h) {
+  if (h->ltab || h->D != 3 || h->nf >= kTableNodes || h->off64) return;
+  uint32_t *tab = nullptr;
+  if (hipMalloc(&tab, (size_t)(h->Q - 1) * h->nf * sizeof(uint32_t)) != hipSuccess) {
     (void)hipGetLastError();
-    h->ltab = nullptr;
-    return 0;
+    return;
   }
-  drop_chunks(h);  // captured without it
   const Geo G = make_args<double, double>(h).G;
-  return dispatch(h, [&]<int Q, int NS, typename ST, typename CT>() -> int {
+  const int rc = dispatch(h, [&]<int Q, int NS, typename ST, typename CT>() -> int {
     if constexpr (Q == 19)
       hipLaunchKernelGGL((k_loc_table<Q, loc_unit<NS, ST, true>()>), dim3(blocks_for(h->nf)), dim3(256), 0, h->stream,
-                         G, h->nf, h->ltab);
+                         G, h->nf, tab);
     HIP_OK(hipGetLastError());
     return 0;
   });
+  if (rc) {  // not written: the steps must not read it
+    (void)hipFree(tab);
+    return;
+  }
+  drop_chunks(h);  // captured without it
+  h->ltab = tab;
 }
 
 // ---- several 2-D steps per launch -----------------------------------------
@@ -1294,14 +1299,13 @@ void plan_tiles(lbm_handle *h) {
 // one by one.
 constexpr size_t kTileShare = 8, kTileSmall = 32u << 20;
 
-int make_tiles(lbm_handle *h) {
+void make_tiles(lbm_handle *h) {
   auto &t = h->tile;
-  if (t.state != 1) return 0;
+  if (t.state != 1) return;
   auto off = [&]() {
     (void)hipGetLastError();
     free_tiles(h);
     h->tile.state = -1;
-    return 0;
   };
   const size_t sb = state_bytes(h);
   const TileGeo &T = t.T;
@@ -1324,9 +1328,8 @@ int make_tiles(lbm_handle *h) {
       return off();
     hipLaunchKernelGGL(k_tile_build, dim3((unsigned)n), dim3(256), 0, h->stream, G, T, t.gidx, t.list, t.cnt);
   }
-  HIP_OK(hipGetLastError());
+  if (hipGetLastError() != hipSuccess) return off();
   t.state = 2;
-  return 0;
 }
 
 bool solute_on(const lbm_handle *h, int t) {
@@ -1391,14 +1394,14 @@ int run_tile(lbm_handle *h, int steps, int write_macro) {
 extern "C" int lbm_run(lbm_handle *h, int nsteps, int write_macro_last) {
   if (need_lattice(h)) return 1;
   int q = 0;
-  if (nsteps >= kTableSteps && build_table(h)) return 1;
+  if (nsteps >= kTableSteps) build_table(h);
   if (nsteps >= 2 && !h->profile) {
     plan_tiles(h);
     // a step that records the plane flux reads the state before it
     const int keep = h->n_flux && write_macro_last ? 1 : 0;
     while (q < nsteps && h->tile.state > 0) {
       const int len = tile_steps(h, nsteps - q - keep);
-      if (len && make_tiles(h)) return 1;
+      if (len) make_tiles(h);
       if (h->tile.state < 0) break;
       if (len ? run_tile(h, len, q + len == nsteps ? write_macro_last : 0)
               : do_step(h, q == nsteps - 1 ? write_macro_last : 0))
