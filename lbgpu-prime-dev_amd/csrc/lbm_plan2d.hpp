@@ -43,22 +43,29 @@ struct Plan2d {
 };
 
 // Steps per launch and core of k_tile2d.
-// A lattice that one tile per CU covers takes the smallest square core that
-// does: its time is launch (2 us) and per-step latency (1 us), so it takes
-// as many steps a launch as the halo's work allows, 8 (flow with cores up to
-// 10: 10; two components with cores above 12: 6).  Measured when the kernel was first
-// tuned, us per step, flow | flow + solute with row conditions: 128^2 8 x 8
-// cores 1.54 | 1.94 (4 steps 1.74 | 2.06), 200 x 170 12 x 12 cores 1.64 | 2.07
-// (4 steps 1.9 | 2.19), 300 x 310 20 x 20 cores 1.97 with 8 steps | 2.71 with 6
-// (4 steps: 2.3 | 2.86).
+//
+// Up to 29 x 29 (flow) or 25 x 25 nodes per CU (two components, by what LDS
+// holds) the core is the smallest square of at least a CU's share of the nodes,
+// so that about as many tiles as CUs run, each on its own.  Time is then launch
+// (2 us) and per-step latency (1 us), and a launch takes as many steps as the
+// halo's work allows: 8 (flow with cores up to 10: 10; two components with cores
+// above 12: 6, above 20: 4).  us per step, flow | flow + solute with rows: 128^2
+// 1.10 | 1.68, 200 x 170 1.27 | 1.87, 300 x 310 1.77 | 2.55, 413 x 307 2.00 | 3.29
+// (fewer steps, measured with an earlier form of the kernel: 128^2 1.74 with 4
+// against 1.54 with 8, 300 x 310 2.3 against 1.97 | 2.86 against 2.71 with 6; 413
+// x 307 flow in 32 x 16 cores with 4 steps 3.02).
+// The share is one of area: where neither side is near a multiple of the core,
+// the rounded tile counts exceed the CUs and some run a second tile (420 x 300
+// 266 tiles, 3.27 | 4.81 us; 130 x 126 272, 1.51 | 2.83; 480 x 340 266, 3.48 |
+// 5.30).  Handed-on rows keep these step counts with halos half as wide again (a
+// 128^2 flow then has regions of 38 x 38, two nodes a thread: 1.68 us).
+//
 // Larger lattices run several tiles per CU and are bound by the loads of the
 // halo and the FP64 units together: 4 steps, flow in 32 x 16 cores of which a
-// CU holds two (1000^2 10.8, 2100 x 1900 44.9 us; 30 x 30 cores with 8 steps
-// 11.3, 43.7), flow + solute in the largest square core that LDS holds, 25 x
-// 25 (19.7, 85.3 us; 32 x 16 20.4, 91.4; 20 x 20 with 6 steps 22.2, 94.9).
-// Now, with entries in registers: 1.26 (10 steps; 8: 1.31) | 1.77, 1.38 | 1.91,
-// 1.82 | 2.61 us; 413 x 307 flow, 23 x 23 cores with 8 steps, 2.05 (32 x 16
-// cores with 4: 3.02); 1000^2 9.8 | 18.2, 2100 x 1900 41.0 us.
+// CU holds two (1000^2 9.9, 2100 x 1900 40.1 us; 30 x 30 cores with 8 steps,
+// measured when the former took 10.8 and 44.9: 11.3, 43.7), flow + solute in the
+// largest square core that LDS holds, 25 x 25 (600 x 500 6.5, 1000^2 18.5 us; when
+// 1000^2 took 19.7, 32 x 16 cores 20.4 and 20 x 20 with 6 steps 22.2).
 inline void tile_shape(int ni, int nj, int ns, int shrink, int lds_cu, int cus, int &steps, int &cx, int &cy) {
   const double per_cu = (double)ni * nj / cus;
   int s = 8;
@@ -92,11 +99,14 @@ inline bool plan2d(int ni, int nj, int ns, bool handed, int lds_cu, int cus, Pla
   P.T.ni = ni;
   P.T.nj = nj;
   // Strips (k_sweep2d) for flow + solute lattices of many tiles per CU, us per
-  // step, tiles -> strips: 1000^2 18.2 -> 19.6, 1088 x 1224 28 -> 23.8,
-  // 2100 x 1900 80 -> 62, below that tiles are faster (600 x 500 6.7
-  // against 9.2: short strips repeat their pipeline's start too often).  Flow
-  // alone keeps tiles (1088 x 1224 12.4 against 17.2, 2100 x 1900 41.0 against
-  // 41.9).  Rows that hand values to a neighbour need the tiles' barrier.
+  // step, tiles -> strips: 1000^2 18.2 -> 19.6, 1088 x 1224 28 -> 23.7,
+  // 2100 x 1900 80 -> 61.0, below that tiles are faster (600 x 500 6.5
+  // against 9.2: short strips repeat their pipeline's start too often).  The
+  // node count decides alone; narrow lattices, whose strips fill half of their
+  // lanes, take strips too (102 x 11500 28.7 us, half-steps 50.5; tiles were not
+  // tried there).  Flow alone keeps tiles (1088 x 1224 12.2 against 17.2, 2100 x
+  // 1900 40.1 against 41.9).  Rows that hand values to a neighbour need the
+  // tiles' barrier.
   if (ns == 2 && !handed && (long)ni * nj >= 4500L * cus) {
     SweepGeo &S = P.S;
     const size_t col = (size_t)kSweepRows * (72 * ns + 8) + 8 * kSweepEntries;

@@ -22,14 +22,14 @@
 // The arithmetic is collide() of the half-step kernel on the same values, so
 // results equal the step-by-step launches bit for bit.
 //
-// Measured per step, against half-steps and row launches one by one: 128^2
-// flow between walls 3.3 -> 1.1 us; 1088 x 1224 flow + solute with series rows
-// 58 -> 28 us (strips, below: 23.8); 600 x 500 with partial bounce-back 24 ->
-// 7.5 us; 413 x 307 with rows 18.5 -> 3.3 us.  Small lattices are bound by the latency of a
-// step inside the workgroup (about 1 us: LDS gathers, the collision's serial
-// sums, the barrier), large ones by the loads of core and halo (1.7 times the
-// core at 25 x 25 with 4 steps) followed by the FP64 units, which one
-// workgroup per CU does not overlap.
+// Measured per step in runs of 240 to 1200, against half-steps and row launches
+// one by one: 128^2 flow 3.3 -> 1.1 us; flow + solute with rows: 413 x 307 18.5
+// -> 3.3, 600 x 500 with partial bounce-back 24 -> 7.3, 1088 x 1224 58 -> 23.7
+// (strips, below; tiles 28).  Small lattices are bound by the latency of a step
+// inside the workgroup (about 1 us: LDS gathers, the collision's serial sums,
+// the barrier), large ones by the loads of core and halo (1.7 times the core at
+// 25 x 25 with 4 steps) followed by the FP64 units, which one workgroup per CU
+// does not overlap.
 #pragma once
 
 #include "lbm_device.hpp"
@@ -366,10 +366,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile2d(TileArgs B) {
 // either side and, once per strip piece, rows at either end.
 //
 // Measured (flow + solute, porosity 0.7, row conditions), us per step, tiles
-// -> strips: 1088 x 1224 30.0 -> 24.2, 2100 x 1900 84.6 -> 63.4.  An iteration
+// -> strips: 1088 x 1224 28 -> 23.7, 2100 x 1900 80 -> 61.0.  An iteration
 // takes 1.7 us: 0.9 us without the collision (LDS traffic and latency of two
 // waves per SIMD, which is all that 160 KB of rows feed), 0.1 us of it waiting
 // for the global loads; solid columns leave 30 % of the lanes idle.
+
 // tab[strip][row][column] = {compact index (-1 solid or past the strip),
 // entry bits of the node}
 __global__ __launch_bounds__(256) void k_sweep_build(Geo G, SweepGeo S, int2 *tab) {
